@@ -517,13 +517,64 @@ void Chain::eigensolve_mixed() {
     large_blocks_begin(*this, {});
     wide_begin(big);
   }
+  // Batches whose blocks all have up to SM_MAX rows: one launch for their whole solve, a workgroup each.
+  // Measured at K = 64 (blocks of up to 25 rows, ~50 launches per step before): 0.80 -> 0.36 ms per step;
+  // 40 blocks of 2 .. 64 rows: 1.34 -> 0.79 ms.  Beside wider blocks, whose rounds take the narrow ones
+  // along at no cost, that launch would come on top (0.33 ms at 64 rows: 60.7 -> 66.2 ms for 25 steps at
+  // K = 500).
+  int small_max = 0;
+  for (int n : cur_n)
+    if (n <= mixed_max) small_max = std::max(small_max, n);
+  small_max = small_max <= SM_MAX ? small_max : 0;
+  std::vector<EigBlock> small;
+  std::vector<int> small_sec;
+  int nmax_s = 0;
+  for (int s = 0; s < S; s++) {
+    const int n = cur_n[s];
+    if (n == 0 || n > small_max) continue;
+    EigBlock b{};
+    b.off = cur_off[s];
+    b.n = n;
+    b.e_off = cur_eoff[s];
+    small.push_back(b);
+    small_sec.push_back(s);
+    nmax_s = std::max(nmax_s, n);
+  }
+  int* d_small = nullptr;  // status per block, then the largest sweep count
+  const int* h_small = nullptr;
+  std::vector<int> redo;  // sectors whose block the batched solve left unconverged
+  if (!small.empty()) {
+    Staging::Region rg = stg.open(Staging::span<EigBlock>(small.size()) + Staging::span<int>(small.size() + 1));
+    const EigBlock* db = stg.place(rg, small);
+    d_small = stg.place_zero<int>(rg, small.size() + 1);
+    stg.commit(rg, st);
+    prof_begin("eig_small");
+    launch_eig_small(db, (int)small.size(), nmax_s, dH.as<double>(), dU.as<double>(), dlam_raw.as<double>(), d_small,
+                     d_small + small.size(), st);
+    prof_end("eig_small", 1, 0.0, 0.0);
+    h_small = stg.get(d_small, small.size() + 1, st);
+  }
+  auto small_done = [&] {  // after a synchronisation
+    if (small.empty()) return;
+    for (size_t i = 0; i < small.size(); i++)
+      if (h_small[i]) redo.push_back(small_sec[i]);
+    sweeps = h_small[small.size()];
+  };
+  // A block the batched solve left short of its stopping point is solved again in FP64 by the direct
+  // solver (the next Hamiltonian is built from these vectors, so they must meet the same bar as every
+  // other block's); nrgk_chain_refine_stats reports how many were.  The stand-alone nrgk_eigh_batched
+  // fails with NRGK_ERR_NOCONV instead (solve_blocks).
+  auto resolve_unconverged = [&] {
+    oa_unconverged = (int)redo.size();
+    if (!redo.empty() && !fail_on_unconverged) solve_dense_fp64(*this, redo);
+  };
   std::vector<EigBlock> blks;
   std::vector<int> row_block, row_local;
   std::vector<int2> tasks;
   int nbc_max = 2, n_bc = 0;
   for (int s = 0; s < S; s++) {
     const int n = cur_n[s];
-    if (n == 0 || n > mixed_max) continue;
+    if (n <= small_max || n > mixed_max) continue;
     EigBlock b{};
     b.off = cur_off[s];
     b.n = n;
@@ -549,12 +600,14 @@ void Chain::eigensolve_mixed() {
     large_blocks_join(*this);
     wide_join();
     sync();
+    sweeps = maxcluster = unresolved = oa_steps = 0;
+    small_done();
     large_blocks_check(*this);
-    sweeps = maxcluster = unresolved = oa_steps = oa_unconverged = 0;
     if (need_full_u || fail_on_unconverged) {
       wide_vectors(true);
       sync();
     }
+    resolve_unconverged();
     return;
   }
   const int nrows = (int)row_block.size();
@@ -667,6 +720,7 @@ void Chain::eigensolve_mixed() {
     prof_end("jacobi_round", nbc_act - 1, fl, by);
     const int* hf = stg.get(dflags, 2 * nb, st);
     sync();
+    if (sw == 0) small_done();
     sweeps = sw + 1;
     // a block goes on while it rotated and some pair was still far from orthogonal
     bool any = false;
@@ -841,7 +895,6 @@ void Chain::eigensolve_mixed() {
       launch_copy_converged(m_blk, na, m_conv, e_tol, d_tol, e_pred, d_pred, dX.as<double>(), dX2.as<double>(), st);
     act.swap(next);
   }
-  oa_unconverged = (int)act.size();
   launch_final_sort(dblk, nb, d_tiles_blk, (int)n_tiles_blk, dX.as<double>(), dlam_tmp.as<double>(),
                     dU.as<double>(), dlam_raw.as<double>(), d_sidx.as<int>(), final_sort_lds(nmax_m), st);
   const int* hs = stg.get(d_stats.as<int>(), 4, st);
@@ -855,20 +908,13 @@ void Chain::eigensolve_mixed() {
     wide_vectors(true);
     sync();
   }
-  // A block the refinement left short of its stopping point is solved again in FP64 by the direct
-  // solver (the next Hamiltonian is built from these vectors, so they must meet the same bar as every
-  // other block's); nrgk_chain_refine_stats reports how many were.  The stand-alone nrgk_eigh_batched
-  // fails with NRGK_ERR_NOCONV instead (solve_blocks).
-  if (oa_unconverged && !fail_on_unconverged) {
-    std::vector<int> secs;
-    for (auto& a : act)
-      for (int s = 0; s < S; s++)
-        if (cur_off[s] == a.off && cur_n[s] == a.n) {
-          secs.push_back(s);
-          break;
-        }
-    solve_dense_fp64(*this, secs);
-  }
+  for (auto& a : act)
+    for (int s = 0; s < S; s++)
+      if (cur_off[s] == a.off && cur_n[s] == a.n) {
+        redo.push_back(s);
+        break;
+      }
+  resolve_unconverged();
 }
 
 // The eigensolver of the current blocks in the chain's mode.  Whatever way it leaves (a status

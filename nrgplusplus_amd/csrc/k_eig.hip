@@ -1416,6 +1416,7 @@ void launch_final_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_
 }
 void set_kernel_lds_limits(int bytes) {
   set_trunc_lds_limit();
+  set_small_lds_limit();
   NRGK_HIP(hipFuncSetAttribute((const void*)k_jacobi_round, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 JAC_W * JAC_CS * sizeof(float)));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_normalize_sort, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));

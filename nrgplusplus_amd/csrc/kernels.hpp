@@ -27,6 +27,11 @@ void launch_final_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_
 size_t normalize_sort_lds(int nmax);
 size_t final_sort_lds(int nmax);
 void set_kernel_lds_limits(int bytes);
+// k_small.hip: blocks of up to SM_MAX rows, solved whole by one workgroup each
+constexpr int SM_MAX = 64;
+void launch_eig_small(const EigBlock* blocks, int nb, int nmax, const double* H, double* U, double* lam, int* status,
+                      int* sweeps, hipStream_t s);
+void set_small_lds_limit();
 // k_gemm.hip
 int prepare_gemm(std::vector<GemmProb>& probs);
 void launch_gemm(const GemmProb* d_probs, int n_probs, int tiles, hipStream_t s);
