@@ -111,7 +111,7 @@ def kernel_table(kstats, K):
 
 # compute families (flops counted) and HBM families (bytes counted) of the library's timers
 HBM_FAMILIES = ("oa_update", "assemble", "fdm_bin", "ht_symv", "tridiagonalise", "tridiag_vectors")
-F32_FAMILIES = ("jacobi_round",)
+F32_FAMILIES = ("mid_reduce", "mid_back")
 
 
 def measured_traffic(kernel):
@@ -127,7 +127,7 @@ def measured_traffic(kernel):
     return None, None
 
 
-FAMILY_KERNEL = {"jacobi_round": "k_jacobi_round", "gemm_f64": "k_gemm64", "ht_symv": "k_ht_symv",
+FAMILY_KERNEL = {"mid_reduce": "k_mid_reduce", "gemm_f64": "k_gemm64", "ht_symv": "k_ht_symv",
                  "assemble": "k_assemble", "fdm_bin": "k_fdm_bin"}
 
 
@@ -553,7 +553,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "fp64 (eigensolve: fp32 jacobi + fp64 refinement below the crossover, fp64 householder above)",
+        "dtype": "fp64 (eigensolve: fp32 householder + fp64 refinement below the crossover, fp64 householder above)",
         "data": "synthetic (model Hamiltonian; no dataset)",
         "config": {"workload": "two-channel SIAM RG flow: U=0.4 eps=-0.2 Gamma1=Gamma2=0.01 Lambda=3 K=4096, "
                                "50 iterations, all_eigenvalue read each iteration",

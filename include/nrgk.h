@@ -32,7 +32,7 @@ extern "C" {
 #define NRGK_ERR_UNSUPPORTED (-6)
 
 /* eigensolver / rotation precision modes */
-#define NRGK_MODE_MIXED 0   /* FP32 block Jacobi + FP64 Ogita-Aishima refinement, batched  */
+#define NRGK_MODE_MIXED 0   /* FP32 Householder + FP64 Ogita-Aishima refinement, batched  */
 #define NRGK_MODE_PLAIN64 1 /* one launch per block: rocSOLVER dsyevd + rocBLAS dgemm, FP64 */
 
 typedef struct nrgk_ctx nrgk_ctx;
@@ -121,11 +121,11 @@ int nrgk_ctx_set_capacity(nrgk_ctx* ctx, size_t bytes);
 int nrgk_ctx_used_bytes(nrgk_ctx* ctx, size_t* used, size_t* capacity);
 
 /* Autotuner (no reference counterpart): measures, on batches of random symmetric blocks of widths
- * 192..768, the batched Jacobi path (all eigenvectors) against the Householder path (eigenvalues and
+ * 192..768, the batched path (all eigenvectors) against the wide blocks' path (eigenvalues and
  * the first quarter of the eigenvectors) and sets the context's crossover to the widest width at which
- * the Jacobi path is not slower.  The result and the measured times go to a cache file (cache_path, or
+ * the batched path is not slower.  The result and the measured times go to a cache file (cache_path, or
  * NULL: $NRGK_TUNE_CACHE, else $HOME/.cache/nrgk/tune-<arch>-<CUs>cu.txt) that every context created
- * later on the same GPU model reads.  table[n_rows][4]: width, blocks, Jacobi ms, Householder ms (may
+ * later on the same GPU model reads.  table[n_rows][4]: width, blocks, batched ms, wide-path ms (may
  * be NULL).  NRGK_MIXED_MAX, when set, overrides the crossover per call. */
 int nrgk_tune(nrgk_ctx* ctx, const char* cache_path, int* crossover, double* table, int cap_rows, int* n_rows);
 /* the context's crossover and whether it came from the autotuner (its cache or nrgk_tune) */
@@ -157,7 +157,7 @@ int nrgk_chain_step(nrgk_chain* chain, const double* t_hopping, int n_hopping, d
  * packed one after another in H (sum dims[b]^2 doubles, only the blocks' full storage is read).
  * Ascending eigenvalues go to w (sum dims[b]), the eigenvectors as the columns of each block to U
  * (packed like H).  Host arrays; mode NRGK_MODE_MIXED or NRGK_MODE_PLAIN64.  Allocates its
- * device buffers per call.  NRGK_ERR_NOCONV when a block does not converge (the FP32 Jacobi, the
+ * device buffers per call.  NRGK_ERR_NOCONV when a block does not converge (the small blocks' Jacobi, the
  * FP64 refinement within its step limit, or dsyevd); the reference only prints dsyevd's info. */
 int nrgk_eigh_batched(nrgk_ctx* ctx, int n_blocks, const int* dims, const double* H, double* w, double* U,
                       int mode);
@@ -214,7 +214,8 @@ int nrgk_chain_fdag_blocks(nrgk_chain* chain, int op, int* n_blocks, int* bi, in
  * their kept energies and the kept x kept f-dagger blocks.  Layout as nrgk_site_desc with
  * dims = kept counts. */
 int nrgk_chain_set_state(nrgk_chain* chain, const nrgk_site_desc* state, int cnt);
-/* per-step device timings (ms): assemble, eigensolve, truncate, rotate; and eigensolver stats */
+/* per-step device timings (ms): assemble, eigensolve, truncate, rotate; and eigensolver stats (the most sweeps of
+ * a small block's Jacobi, the widest cluster) */
 int nrgk_chain_step_stats(nrgk_chain* chain, double* ms4, int* jacobi_sweeps, int* max_cluster);
 /* the last truncation: E_cut = sorted[K] (discard_higher_energies, nrgcore.hpp:285) and the number of
  * eigenvalues within 2e-10 of E_cut + 1e-8 (either side), whose keep/discard decision an eigenvalue
@@ -231,7 +232,8 @@ int nrgk_chain_refine_stats(nrgk_chain* chain, int* oa_steps, int* unconverged);
  * (nrgcore/include/utils/timer.hpp:22-79) at kernel granularity.  While enabled (enabling clears the
  * totals), each run of consecutive launches of one family is bracketed by HIP events on the chain's
  * stream, and its device time is accumulated with the launch count and the algorithmic flops and
- * bytes of those launches.  Families: "jacobi_round", "oa_update", "gemm_f64". */
+ * bytes of those launches.  Families: "mid_reduce", "mid_tridiag",
+ * "mid_back", "oa_update", "gemm_f64", "eig_small", ... */
 typedef struct {
   char family[32];
   double ms;

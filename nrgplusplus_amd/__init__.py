@@ -381,8 +381,8 @@ class Context:
         _check(lib().nrgk_ctx_set_capacity(self._h, nbytes))
 
     def tune(self, cache_path=None):
-        """autotune the eigensolver crossover (nrgk_tune): (crossover, rows of (width, blocks, jacobi ms,
-        householder ms))"""
+        """autotune the eigensolver crossover (nrgk_tune): (crossover, rows of (width, blocks, batched ms,
+        wide-path ms))"""
         cross, nr = C.c_int(), C.c_int()
         tab = np.zeros(4 * 32)
         _check(lib().nrgk_tune(self._h, os.fsencode(cache_path) if cache_path else None, C.byref(cross), _dp(tab),

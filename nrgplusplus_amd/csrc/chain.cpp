@@ -97,11 +97,10 @@ Chain::Chain(Ctx* c, int mode_) : ctx(c), mode(mode_) { init_device(); }
 
 void Chain::init_device() {
   NRGK_REQUIRE(mode == NRGK_MODE_MIXED || mode == NRGK_MODE_PLAIN64, NRGK_ERR_INVALID, "nrgk: unknown mode");
-  for (DevBuf* b : {&eprev_own, &fbuf[0], &fbuf[1], &d_bathE, &d_bathF, &dH, &dW, &dX, &dX2, &dP, &dS, &dR, &dE, &dU,
-                    &dY, &dC, &dlam_tmp, &dlam_raw, &dlam_prev, &dlam_shift[0], &dlam_shift[1], &d_asm, &d_eig, &d_misc, &d_rot,
-                    &d_gemm, &d_flags, &d_sigma_bits, &d_sigma, &d_stats, &d_kept, &d_trunc, &d_conv, &d_eig_act,
-                    &dQ, &d_rrv, &d_cid, &d_sidx, &d_offmax, &d_dgram, &d_dgv, &d_ht, &d_wide_ws, &d_wide_s, &d_wide_q,
-                    &d_wide_A, &d_wide_V})
+  for (DevBuf* b : {&eprev_own, &fbuf[0], &fbuf[1], &d_bathE, &d_bathF, &dH, &dX, &dX2, &d_oa, &dU,
+                    &dY, &dC, &dlam_tmp, &dlam_raw, &dlam_prev, &dlam_shift[0], &dlam_shift[1], &d_eig, &d_stats, &d_kept,
+                    &d_trunc, &d_eig_act, &d_rrv, &d_cid, &d_sidx, &d_mid_A, &d_mid_tau, &d_mid_ws, &d_mid_q, &d_ht,
+                    &d_wide_ws, &d_wide_s, &d_wide_q, &d_wide_A, &d_wide_V})
     b->ctx = ctx;
   stg.ctx = ctx;
   NRGK_HIP(hipSetDevice(ctx->device));
@@ -484,11 +483,7 @@ static double knob(const char* name, double dflt) {
   return v ? std::atof(v) : dflt;
 }
 
-// block-column width of the Jacobi tournament: 16 (a task's Gram matrix is 32 x 32), or half the
-// block for blocks of at most 32
-static int choose_bw(int n) { return n <= 32 ? std::max(1, (n + 1) / 2) : 16; }
-
-// K2 + K6: FP32 block Jacobi, then two Ogita-Aishima refinement steps in FP64.
+// K2 + K6: start vectors by an FP32 Householder solve, then Ogita-Aishima refinement in FP64.
 void Chain::eigensolve_mixed() {
   const int S = (int)cur_qn.size();
   // blocks wider than the crossover (the context's, tuned or 768; NRGK_MIXED_MAX overrides it) go to
@@ -569,30 +564,13 @@ void Chain::eigensolve_mixed() {
     if (!redo.empty() && !fail_on_unconverged) solve_dense_fp64(*this, redo);
   };
   std::vector<EigBlock> blks;
-  std::vector<int> row_block, row_local;
-  std::vector<int2> tasks;
-  int nbc_max = 2, n_bc = 0;
   for (int s = 0; s < S; s++) {
     const int n = cur_n[s];
     if (n <= small_max || n > mixed_max) continue;
     EigBlock b{};
     b.off = cur_off[s];
     b.n = n;
-    b.bw = choose_bw(n);
-    int nbc = (n + b.bw - 1) / b.bw;
-    if (nbc < 2) nbc = 2;
-    if (nbc & 1) nbc++;
-    b.nbc = nbc;
     b.e_off = cur_eoff[s];
-    b.bc_off = n_bc;
-    n_bc += nbc;
-    const int bi = (int)blks.size();
-    for (int j = 0; j < nbc / 2; j++) tasks.push_back(make_int2(bi, j));
-    for (int r = 0; r < n; r++) {
-      row_block.push_back(bi);
-      row_local.push_back(r);
-    }
-    nbc_max = std::max(nbc_max, nbc);
     blks.push_back(b);
   }
   const int nb = (int)blks.size();
@@ -610,149 +588,80 @@ void Chain::eigensolve_mixed() {
     resolve_unconverged();
     return;
   }
-  const int nrows = (int)row_block.size();
   int nmax_m = 1;  // widest block of the batched solve (LDS sizes)
   for (auto& b : blks) nmax_m = std::max(nmax_m, b.n);
-  upload_to(d_eig, blks.data(), nb);
-  const size_t o_rb = 0, o_rl = ((nrows * 4 + 255) / 256) * 256;
-  d_misc.ensure(o_rl + std::max(1, nrows) * sizeof(int));
-  upload_to(d_misc, row_block.data(), nrows, o_rb);
-  upload_to(d_misc, row_local.data(), nrows, o_rl);
-  char* mb = d_misc.as<char>();
-  const EigBlock* dblk = d_eig.as<EigBlock>();
-
+  const EigBlock* dblk = upload_to(d_eig, blks.data(), nb);
+  // ---- FP32 stage (k_mid.hip): every block's start vectors in a dozen launches, widest blocks first
+  // (each is one workgroup's work in the reduction)
   const size_t bytes64 = std::max<long long>(1, tot_elems) * sizeof(double);
-  dW.ensure(std::max<long long>(1, tot_elems) * sizeof(float));
-  d_sigma_bits.ensure(std::max(1, nb) * 2 * sizeof(unsigned));
-  d_sigma.ensure(std::max(1, nb) * sizeof(float));
-  NRGK_HIP(hipMemsetAsync(d_sigma_bits.p, 0, std::max(1, nb) * 2 * sizeof(unsigned), st));
-  launch_shift_convert(dblk, (const int*)(mb + o_rb), (const int*)(mb + o_rl), nrows, dH.as<double>(),
-                       d_sigma_bits.as<unsigned>(), d_sigma.as<float>(), dW.as<float>(), st);
-  // Jacobi sweeps.  The tasks of the blocks still rotating are listed per sweep (a block that a sweep
-  // leaves unrotated has converged), blocks with the longest tournaments first, so that round r
-  // launches the prefix of tasks whose block has a round r.
-  const int max_sweeps = 20;
-  // Gram blocks of the block columns, carried between rounds (invalid until first formed)
-  d_dgram.ensure(std::max(1, n_bc) * 256 * sizeof(double));
-  d_dgv.ensure(std::max(1, n_bc) * sizeof(int));
-  NRGK_HIP(hipMemsetAsync(d_dgv.p, 0, std::max(1, n_bc) * sizeof(int), st));
-  // rotate a column pair while cos > jac_tol and the rotation angle tan > jac_ang: the angle test
-  // stops pairs of very different norms at the FP32 floor, the cosine test degenerate pairs
-  const float jac_tol = knob("NRGK_JAC_TOL", 5e-7);
-  const float jac_ang = knob("NRGK_JAC_ANGLE", 1e-7);
-  const int jac_inner = (int)knob("NRGK_JAC_INNER", 1);  // Jacobi sweeps over a task's Gram matrix
-  // stop a block after a sweep whose pairs all started near orthogonal (0: only after a sweep
-  // without rotations)
-  const bool jac_quad = knob("NRGK_JAC_QUAD", 1) != 0;
-  const double jac_far = knob("NRGK_JAC_FAR", 1e-4);
-  const bool dbg_jac = knob("NRGK_DEBUG_JAC", 0) != 0;
-  // Workgroup g of a launch runs on XCD g mod 8 (round-robin dispatch).  Every block is kept on one
-  // XCD for the whole solve, so that its columns stay in that XCD's L2 from round to round: blocks,
-  // longest tournaments first, go to the XCD with the fewest tasks so far, and slot k of XCD x's
-  // task list sits at grid index 8 k + x (unused slots hold an empty task, which returns at once).
-  constexpr int NXCD = 8;
   std::vector<int> order(nb);
   std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blks[x].nbc > blks[y].nbc; });
-  // The balance counts the tasks that do work: after round 0 the pair holding the empty block column
-  // that pads an odd count returns at once.  Blocks with rounds after the first are balanced on their
-  // tasks per later round (32 CUs per XCD: more than 32 tasks on one XCD need a second wave), the
-  // one-round blocks on their round-0 tasks.
-  std::vector<int> xcd_of(std::max(1, nb), 0);
-  {
-    int load[NXCD] = {0}, load0[NXCD] = {0};
-    for (int bi : order) {
-      const EigBlock& e = blks[bi];
-      const int w = e.nbc > 2 ? e.nbc / 2 - ((e.nbc - 1) * e.bw >= e.n ? 1 : 0) : 0;
-      int x = 0;
-      for (int y = 1; y < NXCD; y++) {
-        const bool better = w > 0 ? (load[y] < load[x] || (load[y] == load[x] && load0[y] < load0[x]))
-                                  : (load0[y] < load0[x] || (load0[y] == load0[x] && load[y] < load[x]));
-        if (better) x = y;
-      }
-      xcd_of[bi] = x;
-      load[x] += w;
-      load0[x] += e.nbc / 2;
-    }
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blks[x].n > blks[y].n; });
+  std::vector<MidBlock> mid;
+  std::vector<HtBlock> mht;
+  long long po = 0, vo = 0, wo = 0, so = 0, no = 0;
+  for (int i : order) {
+    const EigBlock& e = blks[i];
+    HtBlock t{};
+    t.n = t.m = e.n;
+    t.T = (e.n + HT_TB - 1) / HT_TB;
+    t.a_off = e.off;
+    t.w_off = wo;
+    t.s_off = so;
+    t.e_off = e.e_off;
+    t.mpad = ht_stein_slots(e.n);
+    mht.push_back(t);
+    mid.push_back(MidBlock{e.off, po, vo, wo, e.n, t.T, e.e_off});
+    const long long ldv = md_ldv(e.n);
+    po += md_matrix_floats(e.n);
+    vo += ldv * ldv;
+    wo += (ht_ws_size(e.n, t.T) + 31) / 32 * 32;
+    so += 3LL * e.n * t.mpad;
+    no += e.n;
   }
-  std::vector<int> hflags(std::max(1, nb), 1);
-  std::vector<JacTask> xtasks[NXCD], grid_tasks;
-  sweeps = 0;
-  bool converged = false;
-  for (int sw = 0; sw < max_sweeps && nb > 0; sw++) {
-    for (auto& v : xtasks) v.clear();
-    int nbc_act = 2;
-    double fl = 0, by = 0;
-    for (int bi : order) {
-      if (!hflags[bi]) continue;
-      const EigBlock& e = blks[bi];
-      nbc_act = std::max(nbc_act, e.nbc);
-      for (int jj = 0; jj < e.nbc / 2; jj++)
-        xtasks[xcd_of[bi]].push_back(JacTask{e.off, e.n, e.nbc, e.bw, e.bc_off, bi, jj});
-      if (prof_on) {  // per task and round: the cross Gram block (2 n (w/2)^2) and P V (2 n w^2)
-        const double n = e.n, w = std::min(e.n, 2 * e.bw);
-        const double rounds = e.nbc - 1, pairs = std::ceil(n / w);
-        fl += rounds * pairs * 2.5 * n * w * w;
-        by += rounds * pairs * (n <= 768 ? 2.0 : 3.0) * n * w * 4.0;  // FP32 panel read once, written once
-      }
-    }
-    size_t maxlen = 0;
-    for (auto& v : xtasks) maxlen = std::max(maxlen, v.size());
-    grid_tasks.assign(NXCD * maxlen, JacTask{0, 0, 0, 1, 0, 0, 0});
-    for (int x = 0; x < NXCD; x++)
-      for (size_t k = 0; k < xtasks[x].size(); k++) grid_tasks[NXCD * k + x] = xtasks[x][k];
-    Staging::Region rg = stg.open(Staging::span<JacTask>(grid_tasks.size()) + Staging::span<int>(2 * nb));
-    const JacTask* dt = stg.place(rg, grid_tasks);
-    int* dflags = stg.place_zero<int>(rg, 2 * nb);
-    stg.commit(rg, st);
-    prof_begin("jacobi_round");
-    size_t cnt[NXCD];
-    for (int x = 0; x < NXCD; x++) cnt[x] = xtasks[x].size();
-    for (int r = 0; r < nbc_act - 1; r++) {
-      size_t len = 0;
-      for (int x = 0; x < NXCD; x++) {  // tasks of blocks whose tournament has ended drop off the end
-        while (cnt[x] > 0 && xtasks[x][cnt[x] - 1].nbc - 1 <= r) cnt[x]--;
-        len = std::max(len, cnt[x]);
-      }
-      launch_jacobi_round(dt, (int)(NXCD * len), dW.as<float>(), r, dflags, d_dgram.as<double>(), d_dgv.as<int>(),
-                          jac_tol, jac_ang, jac_inner, jac_far, st);
-    }
-    prof_end("jacobi_round", nbc_act - 1, fl, by);
-    const int* hf = stg.get(dflags, 2 * nb, st);
-    sync();
-    if (sw == 0) small_done();
-    sweeps = sw + 1;
-    // a block goes on while it rotated and some pair was still far from orthogonal
-    bool any = false;
-    for (int bi = 0; bi < nb; bi++) {
-      hflags[bi] = hflags[bi] && hf[2 * bi] && (jac_quad ? hf[2 * bi + 1] : 1);
-      any |= hflags[bi] != 0;
-    }
-    if (dbg_jac) {  // NRGK_DEBUG_JAC=1: blocks still rotating (and their largest width) after each sweep
-      int act = 0, wmax = 0;
-      for (int bi = 0; bi < nb; bi++)
-        if (hflags[bi]) act++, wmax = std::max(wmax, blks[bi].n);
-      std::fprintf(stderr, "nrgk jacobi sweep %d: %d of %d blocks go on (widest %d)\n", sw, act, nb, wmax);
-    }
-    if (!any) {
-      converged = true;
-      break;
-    }
-  }
-  NRGK_REQUIRE(converged || nb == 0, NRGK_ERR_NOCONV, "nrgk: FP32 Jacobi did not converge in 20 sweeps");
   dX.ensure(bytes64);
   dX2.ensure(bytes64);
-  dP.ensure(bytes64);
-  dS.ensure(bytes64);
-  dR.ensure(bytes64);
-  dE.ensure(bytes64);
   dU.ensure(bytes64);
-  dQ.ensure(bytes64);
+  // five n x n arenas for the refinement: P = H X, S, R, E and the Rayleigh-Ritz scratch Q; before it, the
+  // same memory holds the Householder vectors, V T, and the inverse iteration's factors
+  const long long na = std::max<long long>(1, tot_elems);
+  d_oa.ensure((size_t)std::max(5 * na, vo + so) * sizeof(double));
+  double* dP = d_oa.as<double>();
+  double *dS = dP + na, *dR = dS + na, *dE = dR + na, *dQ = dE + na;
   d_rrv.ensure(std::max<long long>(1, N_tot) * 3 * sizeof(double));
   dlam_tmp.ensure(std::max<long long>(1, N_tot) * sizeof(double));
   dlam_raw.ensure(std::max<long long>(1, N_tot) * sizeof(double));
-  // 32 x 32 tiles of every block, for the gathers into X and U, then the 32-column groups for the
-  // column norms
+  d_cid.ensure(std::max<long long>(1, N_tot) * sizeof(int));
+  d_sidx.ensure(std::max<long long>(1, N_tot) * sizeof(int));
+  d_mid_A.ensure((size_t)po * sizeof(float));
+  d_mid_tau.ensure(std::max<long long>(1, N_tot) * sizeof(float));
+  d_mid_ws.ensure((size_t)wo * sizeof(double));
+  d_mid_q.ensure((size_t)(64 + 3 * no) * sizeof(int));
+  {
+    Staging::Region rg = stg.open(Staging::span<MidBlock>(mid.size()) + Staging::span<HtBlock>(mht.size()));
+    const MidBlock* dm = stg.place(rg, mid);
+    const HtBlock* dht = stg.place(rg, mht);
+    stg.commit(rg, st);
+    float* V = d_oa.as<float>();        // vo floats, then V T
+    double* scr = d_oa.as<double>() + vo;
+    double* W = d_mid_ws.as<double>();
+    double fl = 0;
+    if (prof_on)
+      for (auto& e : blks) fl += 4.0 / 3.0 * std::pow((double)e.n, 3);
+    prof_begin("mid_reduce");
+    launch_mid_reduce(dm, mid, dH.as<double>(), d_mid_A.as<float>(), V, d_mid_tau.as<float>(), W, st);
+    prof_end("mid_reduce", 1, fl, 0.0);
+    // eigenpairs of T: eigenvalues far closer than FP32 resolves them, then inverse iteration
+    prof_begin("mid_tridiag");
+    launch_ht_sturm(dht, mht, W, dlam_tmp.as<double>(), 1e-11, st);
+    launch_ht_stein(dht, mht, W, dlam_tmp.as<double>(), dX.as<double>(), scr, 1e-6,
+                    d_mid_q.as<int>() + 64, d_mid_q.as<int>(), st);
+    prof_end("mid_tridiag", 7, 0.0, 0.0);
+    prof_begin("mid_back");
+    launch_mid_back(dm, mid, V, d_mid_tau.as<float>(), V + vo, dX.as<double>(), st);
+    prof_end("mid_back", 2, 1.5 * fl, 0.0);
+  }
+  // 32 x 32 tiles of every block, for the gather into U
   std::vector<int4> tiles_blk;
   for (int bi = 0; bi < nb; bi++) {
     const int T = (blks[bi].n + 31) / 32;
@@ -760,44 +669,27 @@ void Chain::eigensolve_mixed() {
       for (int tj = 0; tj < T; tj++) tiles_blk.push_back(int4{bi, ti, tj, 0});
   }
   const size_t n_tiles_blk = tiles_blk.size();
-  for (int bi = 0; bi < nb; bi++)
-    for (int c0 = 0; c0 < blks[bi].n; c0 += 32) tiles_blk.push_back(int4{bi, 0, c0, 0});
   const int4* d_tiles_blk = upload_to(d_eig_act, tiles_blk.data(), tiles_blk.size());
-  const int4* d_colg = d_tiles_blk + n_tiles_blk;
-  const int n_colg = (int)(tiles_blk.size() - n_tiles_blk);
-  d_cid.ensure(std::max<long long>(1, N_tot) * sizeof(int));
-  d_sidx.ensure(std::max<long long>(1, N_tot) * sizeof(int));
-  launch_normalize_sort(dblk, nb, d_tiles_blk, (int)n_tiles_blk, d_colg, n_colg, dW.as<float>(), d_sigma.as<float>(),
-                        dX.as<double>(), dlam_tmp.as<double>(), d_cid.as<int>(), d_rrv.as<double>(),
-                        d_rrv.as<double>() + std::max<long long>(1, N_tot), normalize_sort_lds(nmax_m), st);
   // NRGK_DEBUG_FINITE=1: the first stage and block that produces a non-finite value fail the call
   // with NRGK_ERR_NOCONV (the stage and block are in the message)
   const bool dbg = knob("NRGK_DEBUG_FINITE", 0) != 0;
-  auto check = [&](const char* stage, const DevBuf& buf, bool is_float, bool per_block_vec) {
+  auto check = [&](const char* stage, const double* buf, bool per_block_vec) {
     if (!dbg) return;
     NRGK_HIP(stream_sync(st));
     for (auto& b : blks) {
       const size_t cnt = per_block_vec ? (size_t)b.n : (size_t)b.n * b.n;
       const size_t off = per_block_vec ? (size_t)b.e_off : (size_t)b.off;
       std::vector<double> v(cnt);
-      if (is_float) {
-        std::vector<float> f(cnt);
-        d2h(f.data(), buf.as<float>() + off, cnt, st);
-        NRGK_HIP(stream_sync(st));
-        for (size_t i = 0; i < cnt; i++) v[i] = f[i];
-      } else {
-        d2h(v.data(), buf.as<double>() + off, cnt, st);
-        NRGK_HIP(stream_sync(st));
-      }
+      d2h(v.data(), buf + off, cnt, st);
+      NRGK_HIP(stream_sync(st));
       for (double x : v)
         if (!std::isfinite(x))
           throw Error(NRGK_ERR_NOCONV, std::string("nrgk: non-finite value after ") + stage + " in block n=" +
                                            std::to_string(b.n) + " off=" + std::to_string(b.off));
     }
   };
-  check("shift_convert+jacobi (W)", dW, true, false);
-  check("normalize_sort (X)", dX, false, false);
-  check("normalize_sort (lam)", dlam_tmp, false, true);
+  check("start vectors (X)", dX.as<double>(), false);
+  check("start vectors (lam)", dlam_tmp.as<double>(), true);
   d_stats.ensure(4 * sizeof(int));
   NRGK_HIP(hipMemsetAsync(d_stats.p, 0, 4 * sizeof(int), st));
   // Ogita-Aishima steps, per block until the out-of-cluster rotation residuals |rho_ij| are at the
@@ -839,10 +731,10 @@ void Chain::eigensolve_mixed() {
       const int n = b.n;
       double* H = dH.as<double>() + b.off;
       double* X = dX.as<double>() + b.off;
-      double* P = dP.as<double>() + b.off;
-      double* Sm = dS.as<double>() + b.off;
-      double* R = dR.as<double>() + b.off;
-      double* E = dE.as<double>() + b.off;
+      double* P = dP + b.off;
+      double* Sm = dS + b.off;
+      double* R = dR + b.off;
+      double* E = dE + b.off;
       double* X2 = dX2.as<double>() + b.off;
       g1.push_back(GemmProb{H, X, nullptr, P, n, n, n, n, n, n, n, 0, 0, 1.0, 0.0, 0, 0});
       g1.push_back(GemmProb{X, X, nullptr, R, n, n, n, n, n, n, n, 1, 0, 1.0, 0.0, 0, 0, 1});
@@ -851,28 +743,29 @@ void Chain::eigensolve_mixed() {
     }
     run_gemms(g1);
     run_gemms(g2);
-    check("P=HX", dP, false, false);
-    check("S=X^T P", dS, false, false);
-    check("R=X^T X", dR, false, false);
+    check("P=HX", dP, false);
+    check("S=X^T P", dS, false);
+    check("R=X^T X", dR, false);
     // clusters wider than the LDS Rayleigh-Ritz work in P (free after S = X^T P), X2 (written only
     // by the X + X E product that follows) and Q
     double oa_bytes = 0;  // symmetrise S, Rp (read and write both), E from S and Rp, masking pass
     if (prof_on)
       for (auto& b : act) oa_bytes += 8.0 * 9.0 * (double)b.n * b.n;
     prof_begin("oa_update");
-    launch_oa(m_blk, na, m_sym, (int)tiles_sym.size(), m_all, (int)tiles_all.size(), dS.as<double>(), dR.as<double>(),
-              dE.as<double>(), dlam_tmp.as<double>(), d_cid.as<int>(), d_sidx.as<int>(), m_offmax,
-              d_stats.as<int>(), m_conv, dP.as<double>(), dX2.as<double>(), dQ.as<double>(),
+    launch_oa(m_blk, na, m_sym, (int)tiles_sym.size(), m_all, (int)tiles_all.size(), dS, dR,
+              dE, dlam_tmp.as<double>(), d_cid.as<int>(), d_sidx.as<int>(), m_offmax,
+              d_stats.as<int>(), m_conv, dP, dX2.as<double>(), dQ,
               d_rrv.as<double>(), nmax_m, e_tol, d_tol, st);
     prof_end("oa_update", 5, 0.0, oa_bytes);
-    check("oa_update (E)", dE, false, false);
-    check("oa_update (lam)", dlam_tmp, false, true);
+    check("oa_update (E)", dE, false);
+    check("oa_update (lam)", dlam_tmp.as<double>(), true);
     const double* h_conv = stg.get(m_conv, 4 * na, st);
     run_gemms(g3);
     sync();
+    if (it == 0) small_done();
     const std::vector<double> conv(h_conv, h_conv + 4 * na);
     std::swap(dX, dX2);
-    check("X+XE", dX, false, false);
+    check("X+XE", dX.as<double>(), false);
     oa_steps = it + 1;
     std::vector<EigBlock> next;
     for (int a = 0; a < na; a++) {

@@ -125,11 +125,12 @@ struct Chain {
   int nmax = 0;
   std::vector<int> kept;  // after update_internal_state
 
-  DevBuf dH, dW, dX, dX2, dP, dS, dR, dE, dU, dY, dC, dQ, d_rrv;
+  DevBuf dH, dX, dX2, d_oa, dU, dY, dC, d_rrv;
   DevBuf dlam_tmp, dlam_raw, dlam_shift[2];
   int lcur = 0;
-  DevBuf d_asm, d_eig, d_misc, d_rot, d_gemm;
-  DevBuf d_flags, d_sigma_bits, d_sigma, d_stats, d_kept, d_trunc, d_conv, d_eig_act, d_cid, d_sidx, d_offmax, d_dgram, d_dgv;
+  DevBuf d_eig, d_stats, d_kept, d_trunc, d_eig_act, d_cid, d_sidx;
+  // FP32 stage (k_mid.hip): working matrices, tau, T's workspaces, cluster list
+  DevBuf d_mid_A, d_mid_tau, d_mid_ws, d_mid_q;
   int oa_steps = 0, oa_unconverged = 0;
   bool fail_on_unconverged = false;  // nrgk_eigh_batched: an unconverged block is an error
 
@@ -175,7 +176,7 @@ struct Chain {
 
   // plain-mode handles (rocSOLVER / rocBLAS), created on first use
   void* rocblas = nullptr;
-  // blocks wider than the batched solver's LDS panel: rocSOLVER on side streams (plain.cpp)
+  // blocks wider than the batched solver takes: rocSOLVER on side streams (plain.cpp)
   static constexpr int N_SIDE = 4;
   hipStream_t st_big[N_SIDE] = {};
   void* rocblas_big[N_SIDE] = {};

@@ -99,8 +99,8 @@ struct Ctx {
   int lds_max = 65536;  // bytes of LDS one workgroup may allocate
   int n_cu = 0;
   std::string arch;     // gcnArchName of the device
-  // the eigensolver crossover: blocks wider than this leave the batched Jacobi for the Householder
-  // path (768, the widest LDS-resident Jacobi panel, unless the autotuner's cache says otherwise)
+  // the eigensolver crossover: blocks wider than this leave the batched solve for the wide-block
+  // path (768, MD_MAX, unless the autotuner's cache says otherwise)
   int mixed_max = 768;
   bool tuned = false;
   void charge(size_t bytes) {
@@ -291,18 +291,7 @@ struct AsmSector {
 struct EigBlock {
   long long off;   // element offset of the n x n block (same in every per-block arena)
   int n;
-  int nbc;         // number of block columns in the Jacobi tournament (even)
-  int bw;          // block-column width
   int e_off;       // offset of the block's eigenvalues (prefix of n)
-  int bc_off;      // offset of the block's block columns (prefix of nbc)
-};
-
-// One Jacobi task (a pair slot j of block b's tournament) with the block's fields, so that a
-// workgroup reads everything it needs to start in one record.
-struct JacTask {
-  long long off;
-  int n, nbc, bw, bc_off;
-  int b, j;
 };
 
 // Batched GEMM problem: C = alpha * op(A) * op(B) + beta * C0, all row-major.
@@ -370,6 +359,17 @@ struct DiagItem {     // diagonal of block (i, i) of one system operator
   long long src;      // element offset of the n x n block, -1 if the operator has no such block
   long long dst;      // op * N_tot + first state of sector i
   int n;
+};
+
+// A block of the batched solver's FP32 tridiagonalisation (k_mid.hip): the FP32 working matrix (lower
+// triangle in strips of tiles) at p_off, the Householder vectors (row k holds v_k) and V T products at
+// v_off with a row stride of n rounded up to 32, and T in the workspace of the HtBlock of the same index.
+struct MidBlock {
+  long long h_off;  // element offset of the block's n x n FP64 arenas (H, X)
+  long long p_off, v_off;
+  long long w_off;  // workspace (ht_ws)
+  int n, T;
+  int e_off;        // offset of the block's tau (prefix of n)
 };
 
 // Wide-block eigensolver (k_tridiag.hip): blocked Householder tridiagonalisation in FP64, bisection

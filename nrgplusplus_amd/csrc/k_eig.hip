@@ -1,12 +1,8 @@
 // K2/K6: batched symmetric eigensolver replacing per-block LAPACKE_dsyevd
 // (nrgcore/include/utils/qmatrix.hpp:375-404; called serially per sector at nrgcore.hpp:85-89).
 //
-// Stage 1 (FP32): block one-sided (Hestenes) Jacobi on W = H + sigma I (positive definite, so
-//   W converges to V diag(lambda + sigma) and no separate V is kept).  Block columns of width bw
-//   are paired by a round-robin tournament; one workgroup owns one pair: it stages the n x 2bw
-//   panel in LDS, runs inner Jacobi sweeps over the panel's columns (16 waves = 16 column pairs in
-//   flight, dot products accumulated in FP64) and writes the panel back.  All blocks of an
-//   iteration advance one tournament round per launch.
+// Stage 1 (FP32, k_mid.hip): start vectors by Householder tridiagonalisation.  (Batches of small blocks
+//   are solved whole by k_small.hip instead.)
 // Stage 2 (FP64): Ogita-Aishima refinement X <- X + X E from S = X^T H X and R = X^T X, with
 //   clusters of close eigenvalues resolved by a Rayleigh-Ritz step in FP64 (one-sided Jacobi on the
 //   cluster's k x k matrix), then eigenvalues sorted ascending with their columns, as dsyevd
@@ -16,31 +12,16 @@
 
 namespace nrgk {
 
-constexpr int JAC_THREADS = 1024;
-typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
-// tournament_pair without integer division: j < N/2 and round < N-1 keep both sums below 2(N-1)
-__device__ __forceinline__ void tournament_pair_fast(int N, int round, int j, int& p, int& q) {
-  const int m = N - 1;
-  if (j == 0) {
-    p = 0;
-    q = 1 + round;
-  } else {
-    int x = j + round;
-    x -= x >= m ? m : 0;
-    int y = m - j + round;
-    y -= y >= m ? m : 0;
-    p = 1 + x;
-    q = 1 + y;
-  }
-}
+// The bitonic sorts' filling entries stay behind every key: a NaN (of a block with a non-finite entry)
+// or an infinity compares with nothing or equal and would leave them among the block's own
+constexpr double SORT_PAD = 1e300;
+__device__ __forceinline__ double sort_key(double v) { return v < 0.9 * SORT_PAD ? v : 0.9 * SORT_PAD; }
 
 __device__ __forceinline__ void tournament_pair(int N, int round, int j, int& p, int& q) {
   // N players (even); round in [0, N-1); pair j in [0, N/2)
@@ -50,504 +31,6 @@ __device__ __forceinline__ void tournament_pair(int N, int round, int j, int& p,
   } else {
     p = 1 + (j + round) % (N - 1);
     q = 1 + (N - 1 - j + round) % (N - 1);
-  }
-}
-
-// One tournament round for the tasks of the blocks still rotating.  flags[2b] is set when block b
-// rotates during the sweep, flags[2b + 1] when some pair of it starts a round more than JAC_FAR from
-// orthogonal (cosine of the angle between the columns; far2 = JAC_FAR^2).  The host drops a block after
-// a sweep that leaves it unrotated, or whose pairs all started within JAC_FAR: Jacobi converges
-// quadratically, so that sweep has taken them to about JAC_FAR^2, below the rotation tolerance, and
-// a further sweep would only find that out.
-//
-// A task owns the pair (p, q) of block columns of W (column-major, length n).  Its local columns
-// are p's at 0..wp-1 and q's at bw..bw+wq-1 (bw <= 16; the columns between exist only beside the
-// last, partial block column and are zero).  Instead of rotating the columns pair by pair, it forms
-// their Gram matrix G = P^T P in FP64 on the matrix cores (P read once, staged through LDS in row
-// chunks), runs the cyclic Jacobi rotations on G (two-sided, the same rotations a one-sided sweep of
-// P would make) while accumulating V, and finally writes P <- P V in one pass, also on the matrix
-// cores.  The rounding of P to FP32 then happens once per round, not per rotation.
-constexpr int JAC_BW = 16;
-constexpr int JAC_W = 2 * JAC_BW;
-constexpr int JAC_CHUNK = 768;         // rows per LDS chunk of the Gram pass
-constexpr int JAC_CS = JAC_CHUNK + 4;  // column stride of the chunk: 16 columns x 4 rows fall in distinct banks
-// G and V carry a zero row and column JAC_DUMMY, read in place of a missing member of a rotation
-// pair, and a row and column JAC_SINK that take its writes, so that a rotation step has no branches
-constexpr int JAC_DUMMY = JAC_W, JAC_SINK = JAC_W + 1;
-constexpr int GP = JAC_W + 3;          // row stride of G and V (rows and columns 0..JAC_SINK)
-constexpr int GSZ = (JAC_W + 2) * GP;
-
-// sum of the four partial 16 x 16 blocks at P, P + 256, P + 512, P + 768
-__device__ __forceinline__ double sum4(const double* P, int t) { return (P[t] + P[256 + t]) + (P[512 + t] + P[768 + t]); }
-
-__global__ void __launch_bounds__(JAC_THREADS) k_jacobi_round(const JacTask* __restrict__ tasks, float* __restrict__ W,
-                                                              int round, int* __restrict__ flags,
-                                                              double* __restrict__ dgram, int* __restrict__ dgv,
-                                                              float tol, float ang_tol, int max_inner, double far2) {
-  extern __shared__ float4 chunk4[];  // [JAC_W * JAC_CS] floats, column-major, 16-byte aligned
-  float* chunk = reinterpret_cast<float*>(chunk4);
-  __shared__ double G[GSZ], G2[GSZ], Vd[GSZ];
-  __shared__ double Gpart[3 * 1024];  // partial Gram blocks of the matrix-core waves
-  __shared__ int s_slots[32 * 16];
-  __shared__ float Vf[JAC_W * GP];
-  __shared__ int s_any;
-  const JacTask task = tasks[blockIdx.x];
-  const int b = task.b, j = task.j;
-  const int N = task.nbc;
-  if (round >= N - 1) return;
-  int p, q;
-  tournament_pair(N, round, j, p, q);
-  const int n = task.n, bw = task.bw;
-  const int tid = threadIdx.x;
-  const int c0p = p * bw, c0q = q * bw;
-  const int wp = c0p < n ? min(bw, n - c0p) : 0;
-  const int wq = c0q < n ? min(bw, n - c0q) : 0;
-  if (wp + wq == 0) return;
-  // beside the empty block column that pads the tournament to an even count there is nothing to
-  // pair after round 0 (which rotates the pairs inside each block column)
-  if (round > 0 && (wp == 0 || wq == 0)) return;
-  const int wl = bw + wq;  // local columns in use: [0, wp) and [bw, wl)
-  float* Wb = W + task.off;
-  auto valid = [&](int i) { return i < wp || (i >= bw && i < wl); };
-  auto gcol = [&](int i) { return i < bw ? c0p + i : c0q + (i - bw); };
-  const bool resident = n <= JAC_CHUNK;
-  // Gram blocks of the two block columns (16 x 16 slots, FP64), kept from their last round: when both
-  // are valid, only the cross block is formed from P.  They are the Gram blocks of the exact rotated
-  // columns, which the FP32 panel holds to rounding.  A block column keeps its block current in every
-  // round that touches it, so a stored block is never stale.  Their validity and the blocks are read
-  // together (both slots exist whatever their state).
-  double* dgp = dgram + ((long long)task.bc_off + p) * 256;
-  double* dgq = dgram + ((long long)task.bc_off + q) * 256;
-  const int vp = dgv[task.bc_off + p], vq = dgv[task.bc_off + q];
-  double pre_p = 0.0, pre_q = 0.0;
-  if (tid < 256) {
-    pre_p = dgp[tid];
-    pre_q = dgq[tid];
-  }
-  const bool keepP = wp > 0, keepQ = wq > 0;
-  const bool fast = resident && keepP && keepQ && vp && vq;
-  // ---- step schedule of the Jacobi rotations.  A step rotates up to 16 disjoint column pairs
-  // ("slots").  Each pair of columns is rotated once per outer sweep: the pairs inside p and inside q
-  // in round 0 (a circle tournament of bwp = bw rounded up to even players on each block at once,
-  // bwp - 1 steps, slots 0..bwp/2-1 on p and bwp/2..bwp-1 on q), the bw x bw cross pairs in every
-  // round (step k, slot i: p-column i with q-column (i + k) mod bw).  A column without a partner in
-  // a step sits in a slot with -1.
-  const int bwp = bw + (bw & 1);
-  const int n_intra = round == 0 ? bwp - 1 : 0;
-  const int steps_per = n_intra + bw;
-  const int nsteps = max_inner * steps_per;
-  auto slot = [&](int st, int sl, int& u, int& v) {
-    if (st >= n_intra) {  // cross step (uniform branch)
-      int jj = sl + st - n_intra;
-      jj -= jj >= bw ? bw : 0;
-      u = sl < wp ? sl : -1;
-      v = sl < bw && jj < wq ? bw + jj : -1;
-      return;
-    }
-    u = v = -1;
-    const int half = bwp >> 1, M = bwp - 1;
-    const bool sq = sl >= half;
-    const int m = sq ? sl - half : sl;
-    if (m >= half) return;
-    int a = 0, c = 1 + st;
-    if (m > 0) {
-      int x = st + m;
-      x -= x >= M ? M : 0;
-      int y = st - m;
-      y += y < 0 ? M : 0;
-      a = 1 + x;
-      c = 1 + y;
-    }
-    if (a > c) {
-      const int t = a;
-      a = c;
-      c = t;
-    }
-    const int wb = sq ? wq : wp, base = sq ? bw : 0;
-    u = a < wb ? base + a : -1;
-    v = c < wb ? base + c : -1;
-  };
-  // set-up that needs no data, done while the panel loads are in flight: the slot table (one period,
-  // steps_per x 16: read and write indices of the pair packed ru | rv << 8 | wu << 16 | wv << 24, a
-  // missing member reading JAC_DUMMY and writing JAC_SINK), V = I, and the dummy row and column of
-  // both G buffers set to zero
-  auto setup = [&]() {
-    if (tid == 0) s_any = 0;
-    for (int e = tid; e < steps_per * 16; e += JAC_THREADS) {
-      int u, v;
-      slot(e >> 4, e & 15, u, v);
-      const int ru = u >= 0 ? u : JAC_DUMMY, rv = v >= 0 ? v : JAC_DUMMY;
-      const int wu = u >= 0 ? u : JAC_SINK, wv2 = v >= 0 ? v : JAC_SINK;
-      s_slots[e] = ru | (rv << 8) | (wu << 16) | (wv2 << 24);
-    }
-    for (int e = tid; e < (JAC_W + 2) * (JAC_W + 2); e += JAC_THREADS) {
-      const int x = e / (JAC_W + 2), y = e - x * (JAC_W + 2);
-      Vd[x * GP + y] = x == y && x < JAC_W ? 1.0 : 0.0;
-      if (x == JAC_DUMMY || y == JAC_DUMMY) {
-        G[x * GP + y] = 0.0;
-        G2[x * GP + y] = 0.0;
-      }
-    }
-  };
-  // ---- Gram matrix on the FP64 matrix cores (16 x 16 x 4 steps).  Job of wave v: the p x q block
-  // (fast: waves 0-11, each taking every twelfth group of 4 rows), or the p x p, p x q and q x q
-  // blocks (waves 0-3, 4-7, 8-11, every fourth group); two accumulators in flight.  Lane l supplies column
-  // l%16 of its left block as A and of its right block as B, at row 4 kb + l/16; entry (i, j) of the
-  // product lands in lane 16 (i%4) + j, register i/4.  The partial blocks meet in Gpart.
-  const int wv = tid >> 6, lane = tid & 63, lx = lane & 15;
-  const int job = wv < 12 ? (fast ? 1 : wv >> 2) : -1;
-  const int kq = fast ? wv : wv & 3, kstride = fast ? 12 : 4;
-  const float* ca = chunk + (job == 2 ? bw + lx : lx) * JAC_CS + (lane >> 4);
-  const float* cb = chunk + (job == 0 ? lx : bw + lx) * JAC_CS + (lane >> 4);
-  // a 16-wide tile of p reaches into q when bw < 16: those lanes supply zeros
-  const bool am = job == 2 || lx < bw, bm = job != 0 || lx < bw;
-  dbl4 m0 = {0.0, 0.0, 0.0, 0.0}, m1 = {0.0, 0.0, 0.0, 0.0};
-  for (int r0 = 0; r0 < n; r0 += JAC_CHUNK) {
-    const int rows = min(JAC_CHUNK, n - r0);
-    const int rows4 = (rows + 3) & ~3;
-    // thread = (column tid/32, rows tid%32 + 32k): one column pointer per thread, 128-byte runs, all
-    // of a chunk's loads in flight before their LDS stores; rows are filled up to a multiple of 4
-    {
-      const int i = tid >> 5, l = tid & 31;
-      const bool ok = valid(i);
-      const float* src = Wb + (long long)gcol(ok ? i : 0) * n + r0 + l;
-      float* dst = chunk + i * JAC_CS + l;
-      const int lim = ok ? rows - l : 0, lim4 = rows4 - l;
-      float t[JAC_CHUNK / 32];
-#pragma unroll
-      for (int k = 0; k < JAC_CHUNK / 32; k++) t[k] = 32 * k < lim ? src[32 * k] : 0.0f;
-#pragma unroll
-      for (int k = 0; k < JAC_CHUNK / 32; k++)
-        if (32 * k < lim4) dst[32 * k] = t[k];
-    }
-    if (r0 == 0) setup();
-    if (fast && tid < 256) {  // (resident: this is the only chunk); entries outside a partial block
-      const int a = tid >> 4, c = tid & 15;  // column's width are zero
-      if (a < bw && c < bw) {
-        G[a * GP + c] = a < wp && c < wp ? pre_p : 0.0;
-        G[(bw + a) * GP + bw + c] = a < wq && c < wq ? pre_q : 0.0;
-      }
-    }
-    __syncthreads();
-    if (job >= 0) {
-      const int nkb = rows4 >> 2;
-      int kb = kq;
-      // four groups per iteration: all eight operands are read before the products
-      for (; kb + 3 * kstride < nkb; kb += 4 * kstride) {
-        double xa[4], xb[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          xa[u] = am ? (double)ca[4 * (kb + u * kstride)] : 0.0;
-          xb[u] = bm ? (double)cb[4 * (kb + u * kstride)] : 0.0;
-        }
-        m0 = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[0], xb[0], m0, 0, 0, 0);
-        m1 = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[1], xb[1], m1, 0, 0, 0);
-        m0 = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[2], xb[2], m0, 0, 0, 0);
-        m1 = __builtin_amdgcn_mfma_f64_16x16x4f64(xa[3], xb[3], m1, 0, 0, 0);
-      }
-      for (; kb < nkb; kb += kstride)
-        m0 = __builtin_amdgcn_mfma_f64_16x16x4f64(am ? (double)ca[4 * kb] : 0.0, bm ? (double)cb[4 * kb] : 0.0, m0,
-                                                  0, 0, 0);
-    }
-    if (!resident) __syncthreads();  // the next chunk overwrites this one
-  }
-  if (job >= 0) {
-    double* part = Gpart + (fast ? 0 : job * 1024) + kq * 256 + (lane >> 4) * 16 + lx;
-#pragma unroll
-    for (int r = 0; r < 4; r++) part[64 * r] = m0[r] + m1[r];
-  }
-  __syncthreads();
-  if (tid < 256) {
-    const int a = tid >> 4, c = tid & 15;
-    if (a < bw && c < bw) {
-      const double gx =
-          fast ? (sum4(Gpart, tid) + sum4(Gpart + 1024, tid)) + sum4(Gpart + 2048, tid) : sum4(Gpart + 1024, tid);
-      G[a * GP + bw + c] = gx;
-      G[(bw + c) * GP + a] = gx;
-      if (!fast) {
-        G[a * GP + c] = sum4(Gpart, tid);
-        G[(bw + a) * GP + bw + c] = sum4(Gpart + 2048, tid);
-      }
-    }
-  }
-  __syncthreads();
-  if (!fast) {  // keep the freshly formed diagonal blocks
-    if (tid < 256) {
-      const int a = tid >> 4, c = tid & 15;
-      if (a < bw && c < bw) {
-        if (keepP) dgp[tid] = G[a * GP + c];
-        if (keepQ) dgq[tid] = G[(bw + a) * GP + bw + c];
-      }
-    }
-    if (tid == 0) {
-      if (keepP) dgv[task.bc_off + p] = 1;
-      if (keepQ) dgv[task.bc_off + q] = 1;
-    }
-  }
-  {
-    // a task whose columns are already orthogonal to the tolerance has nothing to rotate (the zero
-    // columns between p and q have zero entries)
-    const int x = tid >> 5, y = tid & 31;
-    bool need = false, far = false;
-    if (x < y && y < wl) {
-      const double ga = G[x * GP + y], ab = G[x * GP + x] * G[y * GP + y];
-      need = ga * ga > ((double)tol * (double)tol) * ab;
-      far = ga * ga > far2 * ab;
-    }
-    // one barrier for both tests; flags[2b + 1]: some pair of the block was at least JAC_FAR from
-    // orthogonal during the sweep
-    const unsigned long long bneed = __ballot(need), bfar = __ballot(far);
-    if ((tid & 63) == 0 && (bneed | bfar)) atomicOr(&s_any, (bneed ? 1 : 0) | (bfar ? 2 : 0));
-    __syncthreads();
-    const int any = s_any;
-    if ((any & 2) && tid == 0) flags[2 * b + 1] = 1;
-    if (!(any & 1)) return;
-  }
-  // ---- cyclic Jacobi on G.  Column x of slot (u, v), u < v, moves as P'(:,u) = c P(:,u) - s P(:,v),
-  // P'(:,v) = s P(:,u) + c P(:,v), so G' = J^T G J and V' = V J.  Every thread that needs a slot's
-  // rotation computes it from the same three entries of the current G (so all copies agree exactly).
-  // One barrier per step.
-  const double tol2 = (double)tol * (double)tol;
-  // rotation of slot (u, v) (read indices) from the current G: identity for a lone column (its
-  // partner is the zero dummy, ga = 0) or a pair below tolerance.  Branch-free: a zero or tiny ga
-  // gives inf/NaN on the discarded side of the final selection only.
-  auto rot = [&](const double* Gc, int u, int v, double& cs, double& sn) {
-    const double al = Gc[u * GP + u], be = Gc[v * GP + v], ga = Gc[u * GP + v];
-    // the angle to FP32 accuracy; cos and sin then normalised in FP64 (cs^2 + sn^2 = 1 to rounding,
-    // one Newton step on the FP32 reciprocal square root), so the accumulated V stays orthogonal
-    const float zeta = (float)(be - al) * __builtin_amdgcn_rcpf((float)(2.0 * ga));
-    const float tf = __builtin_copysignf(1.0f, zeta) *
-                     __builtin_amdgcn_rcpf(fabsf(zeta) + __builtin_amdgcn_sqrtf(1.0f + zeta * zeta));
-    const double t = (double)tf, xx = 1.0 + t * t;
-    double z = (double)__builtin_amdgcn_rsqf((float)xx);
-    z = z * (1.5 - 0.5 * xx * z * z);
-    // a rotation below the angle tolerance changes the vectors by less than FP32 can hold
-    const bool go = (ga != 0.0) & (ga * ga > tol2 * (al * be)) & (fabsf(tf) > ang_tol);
-    cs = go ? z : 1.0;
-    sn = go ? z * t : 0.0;
-  };
-  // thread (a, c) < 256 rotates the entries (rows of slot a) x (columns of slot c) of G into the
-  // other buffer, and the same entries of V in place (V' = V J needs only slot c's rotation); the
-  // slots partition the columns, so every entry is written once.  Lane l computes the rotation of
-  // slot l%16, so slot a's comes from lane a of the same wave.  Threads 256 and up only keep the
-  // barrier.
-  double* Gc = G;
-  double* Gn = G2;
-  const int sa_i = tid >> 4, sc_i = tid & 15;
-  bool rotated = false;
-  int ea = 0, ec = 0;
-  if (tid < 256) {
-    ea = s_slots[sa_i];
-    ec = s_slots[sc_i];
-  }
-  for (int st = 0, row = 0; st < nsteps; st++) {
-    row = row + 1 == steps_per ? 0 : row + 1;  // the next step's row of the table
-    if (tid < 256) {
-      const int rua = ea & 0xff, rva = (ea >> 8) & 0xff, wua = (ea >> 16) & 0xff, wva = ea >> 24;
-      const int ruc = ec & 0xff, rvc = (ec >> 8) & 0xff, wuc = (ec >> 16) & 0xff, wvc = ec >> 24;
-      ea = s_slots[row * 16 + sa_i];
-      ec = s_slots[row * 16 + sc_i];
-      double cc, sc;
-      rot(Gc, ruc, rvc, cc, sc);
-      const double g00 = Gc[rua * GP + ruc], g01 = Gc[rua * GP + rvc], g10 = Gc[rva * GP + ruc], g11 = Gc[rva * GP + rvc];
-      const double v00 = Vd[rua * GP + ruc], v01 = Vd[rua * GP + rvc], v10 = Vd[rva * GP + ruc], v11 = Vd[rva * GP + rvc];
-      const double ca = __shfl(cc, sa_i, 64), sa = __shfl(sc, sa_i, 64);
-      rotated |= sc != 0.0;
-      // columns, then rows
-      const double r00 = cc * g00 - sc * g01, r01 = sc * g00 + cc * g01;
-      const double r10 = cc * g10 - sc * g11, r11 = sc * g10 + cc * g11;
-      Gn[wua * GP + wuc] = ca * r00 - sa * r10;
-      Gn[wua * GP + wvc] = ca * r01 - sa * r11;
-      Gn[wva * GP + wuc] = sa * r00 + ca * r10;
-      Gn[wva * GP + wvc] = sa * r01 + ca * r11;
-      Vd[wua * GP + wuc] = cc * v00 - sc * v01;
-      Vd[wua * GP + wvc] = sc * v00 + cc * v01;
-      Vd[wva * GP + wuc] = cc * v10 - sc * v11;
-      Vd[wva * GP + wvc] = sc * v10 + cc * v11;
-    }
-    __syncthreads();
-    double* t = Gc;
-    Gc = Gn;
-    Gn = t;
-  }
-  const bool any_rot = __syncthreads_or(rotated);
-  if (!any_rot) return;  // P unchanged: nothing to write
-  const int ex = tid >> 5, ey = tid & 31;
-  Vf[ex * GP + ey] = (float)Vd[ex * GP + ey];
-  {  // the diagonal blocks of G' = V^T G V for the next round
-    const double gv = Gc[ex * GP + ey];
-    if (keepP && ex < wp && ey < wp) dgp[ex * JAC_BW + ey] = gv;
-    if (keepQ && ex >= bw && ey >= bw && ex < wl && ey < wl) dgq[(ex - bw) * JAC_BW + (ey - bw)] = gv;
-  }
-  __syncthreads();
-  // ---- P <- P V in FP32
-  if (resident) {
-    // (P V)^T = V^T P^T on the FP32 matrix cores in 16-row tiles: per tile and half h of the new
-    // columns, 8 steps of 16 x 16 x 4 over the 32 old columns.  Lane l keeps V(4 ks + l/16, 16 h + l%16)
-    // (A) in registers and reads P(row0 + l%16, 4 ks + l/16) (B); entry (i, j) = (P V)(row0 + j,
-    // 16 h + i) lands in lane 16 (i/4) + j, register i%4 and goes straight to W (16 consecutive rows
-    // of 4 columns per store).  Tile rows past n read the column's padding and are not stored.
-    const int li = lane & 15, lk = lane >> 4;
-    float va[2][8];
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int ks = 0; ks < 8; ks++) va[h][ks] = Vf[(4 * ks + lk) * GP + 16 * h + li];
-    // the eight columns this lane stores: 16 h + 4 (l/16) + r (absent ones flagged)
-    float* colp[2][4];
-    bool colv[2][4];
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int col = 16 * h + 4 * lk + r;
-        colv[h][r] = valid(col);
-        colp[h][r] = Wb + (long long)gcol(colv[h][r] ? col : 0) * n;
-      }
-    auto store = [&](const flt4& m, int row, int h) {
-      if (row < n)
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (colv[h][r]) colp[h][r][row] = m[r];
-    };
-    // two tiles per pass (waves take tiles v, v + 16, v + 32, ...): four independent accumulator
-    // chains keep the matrix pipeline busy
-    const int ntile = (n + 15) >> 4, nw = JAC_THREADS / 64;
-    for (int t0 = wv; t0 < ntile; t0 += 2 * nw) {
-      const int t1 = t0 + nw;
-      const int row0 = 16 * t0 + li, row1 = 16 * t1 + li;
-      const bool two = t1 < ntile;
-      float pb0[8], pb1[8];
-#pragma unroll
-      for (int ks = 0; ks < 8; ks++) {
-        pb0[ks] = chunk[(4 * ks + lk) * JAC_CS + row0];
-        pb1[ks] = two ? chunk[(4 * ks + lk) * JAC_CS + row1] : 0.0f;
-      }
-      flt4 m00 = {0.0f, 0.0f, 0.0f, 0.0f}, m01 = m00, m10 = m00, m11 = m00;
-#pragma unroll
-      for (int ks = 0; ks < 8; ks++) {
-        m00 = __builtin_amdgcn_mfma_f32_16x16x4f32(va[0][ks], pb0[ks], m00, 0, 0, 0);
-        m01 = __builtin_amdgcn_mfma_f32_16x16x4f32(va[1][ks], pb0[ks], m01, 0, 0, 0);
-        m10 = __builtin_amdgcn_mfma_f32_16x16x4f32(va[0][ks], pb1[ks], m10, 0, 0, 0);
-        m11 = __builtin_amdgcn_mfma_f32_16x16x4f32(va[1][ks], pb1[ks], m11, 0, 0, 0);
-      }
-      store(m00, row0, 0);
-      store(m01, row0, 1);
-      if (two) {
-        store(m10, row1, 0);
-        store(m11, row1, 1);
-      }
-    }
-    if (tid == 0) flags[2 * b] = 1;
-    return;
-  }
-  // larger panels: one row per thread from global memory (every value of the row is read before it
-  // is overwritten)
-  for (int r = tid; r < n; r += JAC_THREADS) {
-    float x[JAC_W];
-#pragma unroll
-    for (int i = 0; i < JAC_W; i++) x[i] = valid(i) ? Wb[(long long)gcol(i) * n + r] : 0.0f;
-    for (int c = 0; c < JAC_W; c++) {
-      if (!valid(c)) continue;
-      float s = 0.0f;
-#pragma unroll
-      for (int i = 0; i < JAC_W; i++) s = fmaf(x[i], Vf[i * GP + c], s);
-      Wb[(long long)gcol(c) * n + r] = s;
-    }
-  }
-  if (tid == 0) flags[2 * b] = 1;
-}
-
-// Column norms of the converged W give lambda + sigma; columns are normalised, sorted by lambda
-// and written as FP64 X (row-major, eigenvectors in columns).
-// Column norms of W, 32 columns of one block per workgroup (one wave per column at a time)
-__global__ void __launch_bounds__(256) k_col_norms(const EigBlock* __restrict__ blocks, const int4* __restrict__ groups,
-                                                   const float* __restrict__ W, double* __restrict__ nrm_g) {
-  const int4 g = groups[blockIdx.x];
-  const EigBlock blk = blocks[g.x];
-  const int n = blk.n, c1 = min(g.z + 32, n);
-  const float* Wb = W + blk.off;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int c = g.z + wave; c < c1; c += 4) {
-    double s = 0.0;
-    for (int r = lane; r < n; r += 64) {
-      const double v = Wb[(long long)c * n + r];
-      s += v * v;
-    }
-    s = wave_sum(s);
-    if (lane == 0) nrm_g[blk.e_off + c] = sqrt(s);
-  }
-}
-
-__global__ void __launch_bounds__(1024) k_normalize_sort(const EigBlock* __restrict__ blocks, const double* __restrict__ nrm_g,
-                                                         const float* __restrict__ sigma, double* __restrict__ lam,
-                                                         int* __restrict__ perm, double* __restrict__ nrm_s) {
-  extern __shared__ double sh[];
-  const EigBlock blk = blocks[blockIdx.x];
-  const int n = blk.n;
-  if (n == 0) return;
-  int np2 = 1;
-  while (np2 < n) np2 <<= 1;
-  double* key = sh;                 // [np2]
-  int* idx = (int*)(sh + np2);      // [np2]
-  double* nrm = sh + np2 + (np2 + 1) / 2 + 1;  // [n]
-  for (int c = threadIdx.x; c < n; c += blockDim.x) nrm[c] = nrm_g[blk.e_off + c];
-  __syncthreads();
-  const double sg = sigma[blockIdx.x];
-  for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-    key[i] = i < n ? nrm[i] - sg : 1e300;
-    idx[i] = i;
-  }
-  __syncthreads();
-  // bitonic sort ascending
-  for (int k = 2; k <= np2; k <<= 1) {
-    for (int jj = k >> 1; jj > 0; jj >>= 1) {
-      for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-        const int l = i ^ jj;
-        if (l > i) {
-          const bool up = ((i & k) == 0);
-          const double a = key[i], bb = key[l];
-          if ((a > bb) == up) {
-            key[i] = bb;
-            key[l] = a;
-            const int t = idx[i];
-            idx[i] = idx[l];
-            idx[l] = t;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
-  for (int c = threadIdx.x; c < n; c += blockDim.x) {
-    lam[blk.e_off + c] = key[c];
-    perm[blk.e_off + c] = idx[c];
-    nrm_s[blk.e_off + c] = nrm[idx[c]];
-  }
-}
-
-// X(r, c) = W(:, perm c)(r) / |W(:, perm c)| in FP64 (row-major X, eigenvectors in columns), one
-// 32 x 32 tile of one block per workgroup: columns are read along W's contiguous direction into LDS
-// and the tile is written along X's rows.
-__global__ void __launch_bounds__(256) k_gather_x(const EigBlock* __restrict__ blocks, const int4* __restrict__ tiles,
-                                                  const float* __restrict__ W, const int* __restrict__ perm,
-                                                  const double* __restrict__ nrm_s, double* __restrict__ X) {
-  __shared__ float T[32][33];
-  const int4 t = tiles[blockIdx.x];
-  const EigBlock blk = blocks[t.x];
-  const int n = blk.n, r0 = 32 * t.y, c0 = 32 * t.z;
-  const float* Wb = W + blk.off;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int e = threadIdx.x + 256 * k, c = e >> 5, rr = e & 31;
-    if (c0 + c < n && r0 + rr < n) T[c][rr] = Wb[(long long)perm[blk.e_off + c0 + c] * n + r0 + rr];
-  }
-  __syncthreads();
-  double* Xb = X + blk.off;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int e = threadIdx.x + 256 * k, rr = e >> 5, c = e & 31;
-    if (c0 + c < n && r0 + rr < n) Xb[(long long)(r0 + rr) * n + c0 + c] = (double)T[c][rr] / nrm_s[blk.e_off + c0 + c];
   }
 }
 
@@ -1000,13 +483,13 @@ __global__ void __launch_bounds__(1024) k_oa_prep(const EigBlock* __restrict__ b
   const double* Rb = Rp + blk.off;
   double ml = 0.0;
   for (int i = tid; i < np2; i += blockDim.x) {
-    double v = 1e300;
+    double v = SORT_PAD;
     if (i < n) {
       v = Sb[(long long)i * n + i] / Rb[(long long)i * n + i];
       lam[blk.e_off + i] = v;
       ml = fmax(ml, fabs(v));
     }
-    key[i] = v;
+    key[i] = sort_key(v);
     idx[i] = i;
   }
   const double bq = block_max(ml, red);
@@ -1301,7 +784,7 @@ __global__ void __launch_bounds__(1024) k_final_sort(const EigBlock* __restrict_
   double* key = sh;
   int* idx = (int*)(sh + np2);
   for (int i = threadIdx.x; i < np2; i += blockDim.x) {
-    key[i] = i < n ? lam_in[blk.e_off + i] : 1e300;
+    key[i] = i < n ? sort_key(lam_in[blk.e_off + i]) : SORT_PAD;
     idx[i] = i;
   }
   __syncthreads();
@@ -1324,7 +807,7 @@ __global__ void __launch_bounds__(1024) k_final_sort(const EigBlock* __restrict_
       __syncthreads();
     }
   for (int c = threadIdx.x; c < n; c += blockDim.x) {
-    lam_out[blk.e_off + c] = key[c];
+    lam_out[blk.e_off + c] = lam_in[blk.e_off + idx[c]];
     perm[blk.e_off + c] = idx[c];
   }
 }
@@ -1348,11 +831,6 @@ __global__ void __launch_bounds__(256) k_gather_u(const EigBlock* __restrict__ b
   }
 }
 
-size_t normalize_sort_lds(int nmax) {
-  int np2 = 1;
-  while (np2 < nmax) np2 <<= 1;
-  return (size_t)(np2 + (np2 + 1) / 2 + 1 + nmax) * sizeof(double) + 64;
-}
 size_t oa_prep_lds(int nmax) {
   int np2 = 1;
   while (np2 < nmax) np2 <<= 1;
@@ -1368,25 +846,6 @@ size_t final_sort_lds(int nmax) {
   return (size_t)np2 * 12 + 64;
 }
 
-void launch_jacobi_round(const JacTask* tasks, int n_tasks, float* W, int round, int* flags, double* dgram, int* dgv,
-                         float tol, float ang_tol, int max_inner, double jac_far, hipStream_t s) {
-  if (n_tasks <= 0) return;
-  NRGK_LAUNCH(k_jacobi_round, dim3(n_tasks), dim3(JAC_THREADS), JAC_W * JAC_CS * sizeof(float), s, tasks, W,
-                     round, flags, dgram, dgv, tol, ang_tol, max_inner, jac_far * jac_far);
-  NRGK_HIP(hipGetLastError());
-}
-void launch_normalize_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_tiles, const int4* groups,
-                           int n_groups, const float* W, const float* sigma, double* X, double* lam, int* perm,
-                           double* nrm_s, double* nrm_g, size_t lds, hipStream_t s) {
-  if (nb <= 0) return;
-  NRGK_LAUNCH(k_col_norms, dim3(n_groups), dim3(256), 0, s, blocks, groups, W, nrm_g);
-  NRGK_HIP(hipGetLastError());
-  NRGK_LAUNCH(k_normalize_sort, dim3(nb), dim3(1024), lds, s, blocks, nrm_g, sigma, lam, perm, nrm_s);
-  NRGK_HIP(hipGetLastError());
-  if (n_tiles <= 0) return;
-  NRGK_LAUNCH(k_gather_x, dim3(n_tiles), dim3(256), 0, s, blocks, tiles, W, perm, nrm_s, X);
-  NRGK_HIP(hipGetLastError());
-}
 void launch_oa(const EigBlock* blocks, int nb, const int4* sym_tiles, int n_sym, const int4* all_tiles, int n_all,
                double* S, double* Rp, double* E, double* lam, int* cid, int* sidx, double* offmax, int* stats,
                double* conv, double* scrW, double* scrG, double* scrT, double* rrv, int nmax, double e_tol,
@@ -1417,9 +876,7 @@ void launch_final_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_
 void set_kernel_lds_limits(int bytes) {
   set_trunc_lds_limit();
   set_small_lds_limit();
-  NRGK_HIP(hipFuncSetAttribute((const void*)k_jacobi_round, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                JAC_W * JAC_CS * sizeof(float)));
-  NRGK_HIP(hipFuncSetAttribute((const void*)k_normalize_sort, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+  set_mid_lds_limits(bytes);
   NRGK_HIP(hipFuncSetAttribute((const void*)k_oa_prep, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_oa_rr, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_final_sort, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));

@@ -1,0 +1,931 @@
+// The FP32 stage of the batched eigensolver (blocks wider than SM_MAX rows up to MD_MAX), replacing
+// per-block LAPACKE_dsyevd (nrgcore/include/utils/qmatrix.hpp:375-404) together with the FP64 refinement
+// that follows it (k_eig.hip): start vectors X with H X = X diag(lambda) to FP32 rounding, ascending.
+//
+//   k_mid_reduce  Householder tridiagonalisation of every block in one launch, a workgroup per block
+//   k_ht_sturm    eigenvalues of T (FP64, multisection)
+//   k_ht_stein_*  eigenvectors of T (FP64 inverse iteration, clusters orthonormalised; k_tridiag.hip)
+//   k_mid_larft   the WY factors V_p T_p, a workgroup per panel
+//   k_mid_back    X = Q Z, a workgroup per 64 columns, every panel in one launch
+//
+// The whole sequence takes a dozen launches whatever the block widths; the one-sided block Jacobi it
+// replaces took n/16 dependent launches per sweep and nine sweeps for the widest blocks (n = 330, a SIAM step
+// at K = 1024: 2.7 -> 1.7 ms; n = 190, K = 500: 1.3 -> 0.75 ms; n = 619, K = 2048: 6.8 -> 5.0 ms).
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace nrgk {
+
+typedef float flt4 __attribute__((ext_vector_type(4)));
+
+constexpr int MD_THREADS = 512;
+constexpr int MD_WAVES = MD_THREADS / 64;
+constexpr int MD_RB = (MD_MAX + MD_THREADS - 1) / MD_THREADS;  // rows per thread
+
+// The working matrix holds the lower triangle in strips of 16 rows (an even number of them), each strip as
+// tiles of 64 columns (the last one reaching past the diagonal), a tile's 16 x 64 entries row-major.  Strips
+// 2p and 2p + 1 have equally many tiles.  Entries right of the diagonal are zero and the diagonal is held
+// halved, so that the row sums of a strip (A v) and its column sums (A^T v) add up to the symmetric product
+// without a mask.  The trailing matrix from a row that is a multiple of 64 on has the same form.
+__host__ __device__ __forceinline__ int md_strip(int s) {  // tiles of strips 0 .. s-1
+  const int q = s >> 2, r = s & 3;
+  return (q + 1) * (2 * q + r);
+}
+__host__ __device__ __forceinline__ int md_strips(int n) { return ((n + 31) >> 5) * 2; }
+int md_ldv(int n) { return 16 * md_strips(n); }
+long long md_matrix_floats(int n) { return 1024LL * md_strip(md_strips(n)); }
+__host__ __device__ __forceinline__ int md_np(int n) { return (n + 63) & ~63; }
+// row stride of the staged panel columns: the four 16-lane groups of a matrix-core operand 16 banks apart
+__host__ __device__ __forceinline__ int md_ld(int n) { return md_np(n) + 16; }
+// the widest trailing matrix held in registers: 20 strips of up to 5 tiles, three strips to a wave
+constexpr int MD_REG = 320;
+
+template <int CTRL>
+__device__ __forceinline__ float md_dpp(float v) {
+  return __builtin_amdgcn_update_dpp(0.0f, v, CTRL, 0xF, 0xF, false);
+}
+// the two halves (16-lane rows) of a and b exchanged crosswise and added: lanes of the lower half (even
+// rows) get a's total over both, the others b's
+__device__ __forceinline__ float md_add32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float md_add16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+// sum over the 16 lanes of a DPP row; over the wavefront
+__device__ __forceinline__ float md_sum16(float v) {
+  v += md_dpp<0xB1>(v);
+  v += md_dpp<0x4E>(v);
+  v += md_dpp<0x141>(v);
+  v += md_dpp<0x140>(v);
+  return v;
+}
+__device__ __forceinline__ float md_sum64(float v) {
+  v = md_sum16(v);
+  v = md_add16(v, v);
+  return md_add32(v, v);
+}
+
+// four row sums of a 16-lane row, summed over its lanes and scattered: lane p ends with row md_row(p)
+__device__ __forceinline__ int md_row(int li) { return 2 * (li & 1) + ((li >> 1) & 1); }
+__device__ __forceinline__ float md_rows(const flt4& ra, int li) {
+  const bool h0 = li & 1, h1 = li & 2;
+  float r0 = h0 ? ra[2] : ra[0], r1 = h0 ? ra[3] : ra[1];
+  r0 += md_dpp<0xB1>(h0 ? ra[0] : ra[2]);
+  r1 += md_dpp<0xB1>(h0 ? ra[1] : ra[3]);
+  float rs = h1 ? r1 : r0;
+  rs += md_dpp<0x4E>(h1 ? r0 : r1);
+  rs += md_dpp<0x124>(rs);  // the other quads: rotations by 4 and 8 lanes
+  rs += md_dpp<0x128>(rs);
+  return rs;
+}
+
+// LDS of a workgroup working on n trailing rows
+struct MdLds {
+  float2* VW;   // [MD_NB][ld] the panel's V and W, zero beyond column k
+  float* part;  // [MD_WAVES][np] column sums of a wave's strips
+  float* us;    // [np] u, zero up to row k
+  float* ysum;  // [np] row sums
+};
+__device__ __forceinline__ MdLds md_lds(float* base, int n) {
+  MdLds m;
+  m.VW = reinterpret_cast<float2*>(base);
+  m.part = base + 2 * MD_NB * md_ld(n);
+  m.us = m.part + MD_WAVES * md_np(n);
+  m.ysum = m.us + md_np(n);
+  return m;
+}
+
+// The symmetric product's share of R adjacent strips from st on (they have nt tiles from tile t0 on): their
+// row sums into ysum, their column sums added to (first: put into) the wave's pw.  Lane (lk, li) holds rows
+// 4 lk .. + 3 and columns 4 li .. + 3 of a strip's tile; the next tile is asked for before the current one
+// is used.  s is u's first row (its entry is u0, not us[s]).  Returns this lane's share of u^T A u.
+template <int R>
+__device__ __forceinline__ float md_strip_product(const float* A, const MdLds& m, int st, int t0, int s, float u0,
+                                                  float* pw, bool first, int li, int lk) {
+  const int nt = (st >> 2) - t0 + 1;
+  const flt4* tp[R];
+  flt4 a[R][4], ra[R], ur[R];
+#pragma unroll
+  for (int x = 0; x < R; x++) {
+    tp[x] = reinterpret_cast<const flt4*>(A + 1024 * (md_strip(st + x) + t0) + 256 * lk + 4 * li);
+#pragma unroll
+    for (int i = 0; i < 4; i++) a[x][i] = tp[x][16 * i];
+    const int r4 = 16 * (st + x) + 4 * lk;
+    ur[x] = *reinterpret_cast<const flt4*>(m.us + r4);
+    if (16 * st <= s)
+#pragma unroll
+      for (int i = 0; i < 4; i++) ur[x][i] = r4 + i == s ? u0 : ur[x][i];
+    ra[x] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  for (int t = 0; t < nt; t++) {
+    const int c4 = 64 * (t0 + t) + 4 * li;
+    flt4 an[R][4];
+    if (t + 1 < nt) {
+#pragma unroll
+      for (int x = 0; x < R; x++) {
+        tp[x] += 256;
+#pragma unroll
+        for (int i = 0; i < 4; i++) an[x][i] = tp[x][16 * i];
+      }
+    }
+    flt4 uc = *reinterpret_cast<const flt4*>(m.us + c4);
+    if (t == 0)
+#pragma unroll
+      for (int i = 0; i < 4; i++) uc[i] = c4 + i == s ? u0 : uc[i];
+    float ca[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int x = 0; x < R; x++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          ca[c] += a[x][i][c] * ur[x][i];
+          ra[x][i] += a[x][i][c] * uc[c];
+        }
+    // the four row groups' column sums: lane (lk, li) ends with column 4 li + lk
+    const float cs = md_add16(md_add32(ca[0], ca[2]), md_add32(ca[1], ca[3]));
+    float* pc = pw + 64 * (t0 + t);
+    *pc = first ? cs : *pc + cs;
+    if (t + 1 < nt)
+#pragma unroll
+      for (int x = 0; x < R; x++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) a[x][i] = an[x][i];
+  }
+  float asum = 0.0f;
+#pragma unroll
+  for (int x = 0; x < R; x++) {
+    const float rs = md_rows(ra[x], li);
+    const int row = 16 * (st + x) + 4 * lk + md_row(li);
+    if (li < 4) {
+      m.ysum[row] = rs;
+      asum += rs * (row == s ? u0 : m.us[row]);
+    }
+  }
+  return asum;
+}
+
+// Blocked Householder tridiagonalisation (lower form, panels of MD_NB columns) of the first ncol columns of
+// the n x n matrix A: H_k = I - tau_k v_k v_k^T annihilates column k below its subdiagonal; d, e, tau and v
+// (row stride ldv) go to the pointers given.  Thread t owns rows t and t + MD_THREADS; the panel's V and W
+// are held in LDS by columns.  Three barriers per column:
+//   1  the column (with the panel's corrections) and its norm
+//   2  the symmetric product with the panel-start matrix (waves take strips of rows, longest first, to
+//      and fro; each entry is read once and used for its row and its column), V^T v, W^T v, v^T A v
+//   3  w
+// v enters the products unscaled (u, with u[k+1] = alpha - beta in the place of 1): v = u / (alpha - beta).
+// One CU works on a block, so instructions count: waves whose rows are done or absent skip the per-row
+// phases, and a strip's sums cross lanes by three register swaps per tile and eleven operations per strip.
+__device__ __forceinline__ void md_columns(float* A, const MdLds& m, int n, int ncol, int ex, float* V, int ldv,
+                                           float* tau_g, double* dg, double* eg) {
+  __shared__ float nrm[16], ap[16];  // (entries MD_WAVES .. 15 stay zero)
+  __shared__ float2 dots[MD_NB];     // V^T v and W^T v
+  __shared__ float s_alpha;
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, lk = l >> 4;
+  const int S = md_strips(n), np = md_np(n), ld = md_ld(n);
+  if (tid < 16) nrm[tid] = ap[tid] = 0.0f;
+  for (int r = tid; r < np; r += MD_THREADS) m.us[r] = 0.0f;
+  for (int j0 = 0; j0 < ncol; j0 += MD_NB) {
+    // this thread's rows of the panel-start matrix: entry (r, k) is asked for one column ahead
+    const float* arow[MD_RB];
+    float an[MD_RB];
+    for (int e = tid; e < MD_NB * ld; e += MD_THREADS) m.VW[e] = float2{0.0f, 0.0f};
+#pragma unroll
+    for (int h = 0; h < MD_RB; h++) {
+      const int r = tid + MD_THREADS * h;
+      arow[h] = A + 1024 * (md_strip(r >> 4) + (j0 >> 6)) + (r & 15) * 64 + (j0 & 63);
+      an[h] = r >= j0 && r < n ? arow[h][0] : 0.0f;
+    }
+    __syncthreads();
+    const int kend = min(j0 + MD_NB, n);
+    for (int k = j0; k < kend; k++) {
+      // ---- 1: column k
+      const int cc = k - j0, s = k + 1;
+      float u[MD_RB], sq = 0.0f;
+#pragma unroll
+      for (int h = 0; h < MD_RB; h++) {
+        const int rb = 64 * (wv + MD_WAVES * h), r = rb + l;
+        u[h] = 0.0f;
+        if (rb >= n || rb + 63 < k) continue;  // (the same in every lane)
+        float x = r == k ? 2.0f * an[h] : an[h];
+        if (r >= s && r < n && cc + 1 < MD_NB) an[h] = arow[h][cc + 1];
+        for (int j = 0; j < cc; j += 8) {
+          float2 a[8], b[8];
+#pragma unroll
+          for (int i = 0; i < 8; i++) {
+            a[i] = m.VW[(j + i) * ld + r];
+            b[i] = m.VW[(j + i) * ld + k];
+          }
+#pragma unroll
+          for (int i = 0; i < 8; i++) x -= a[i].x * b[i].y + a[i].y * b[i].x;
+        }
+        if (r == k) dg[k] = ldexp((double)x, ex);
+        x = r < s || r >= n ? 0.0f : x;
+        m.us[r] = x;
+        if (r == s) s_alpha = x;
+        u[h] = x;
+        sq += r > s ? x * x : 0.0f;
+      }
+      if (s >= n) break;
+      sq = md_sum64(sq);
+      if (l == 0) nrm[wv] = sq;
+      __syncthreads();
+      // ---- the reflector, the same in every thread
+      const float x = md_sum16(nrm[li]), alpha = s_alpha;
+      float beta = alpha, tau = 0.0f, u0 = 0.0f, sc = 0.0f;
+      // (entries below 1e-12 of the block's largest are zero to FP32: squares of smaller ones would underflow)
+      const bool refl = __builtin_amdgcn_readfirstlane(__float_as_int(x)) > __float_as_int(1e-24f);  // (x >= 0)
+      if (refl) {
+        beta = -copysignf(__builtin_amdgcn_sqrtf(alpha * alpha + x), alpha);
+        u0 = alpha - beta;
+        tau = -u0 * __builtin_amdgcn_rcpf(beta);
+        sc = __builtin_amdgcn_rcpf(u0);
+      }
+      if (refl) {  // (the same in every thread)
+        // ---- 2: products with u.  More strips than waves: pairs of them, which share column sums
+        const int s0 = s >> 4, t0 = s >> 6, P = S >> 1;
+        const bool pairs = S - s0 > MD_WAVES;
+        const int last = pairs ? P : S, cnt = last - (pairs ? s0 >> 1 : s0);  // (pair or strip) last - 1 down
+        float* pw = m.part + wv * np + 4 * li + lk;
+        float asum = 0.0f;
+        for (int q = 0; q * MD_WAVES < cnt; q++) {
+          const int i0 = q * MD_WAVES + (q & 1 ? MD_WAVES - 1 - wv : wv);
+          if (i0 >= cnt) continue;
+          const int st = last - 1 - i0;
+          asum += pairs ? md_strip_product<2>(A, m, 2 * st, t0, s, u0, pw, q == 0, li, lk)
+                        : md_strip_product<1>(A, m, st, t0, s, u0, pw, q == 0, li, lk);
+        }
+        // panel columns wv and wv + MD_WAVES: V^T u and W^T u
+        for (int j = wv; j < cc; j += MD_WAVES) {
+          float pv = 0.0f, pq = 0.0f;
+          for (int r = 64 * t0 + l; r < np; r += 64) {
+            const float ur = r == s ? u0 : m.us[r];
+            const float2 z = m.VW[j * ld + r];
+            pv += z.x * ur;
+            pq += z.y * ur;
+          }
+          pv = md_sum64(pv);
+          pq = md_sum64(pq);
+          if (l == 0) dots[j] = float2{pv * sc, pq * sc};
+        }
+        asum = md_sum64(asum);
+        if (l == 0) ap[wv] = asum;
+        __syncthreads();
+        // ---- 3: w = tau (A v) - (tau^2 / 2) (v^T A v) v; row and column sums of u^T A u are equal
+        const float va = sc * sc * md_sum16(ap[li]);
+#pragma unroll
+        for (int h = 0; h < MD_RB; h++) {
+          const int cb = wv + MD_WAVES * h, rb = 64 * cb, r = rb + l;
+          if (rb >= n || rb + 63 < s) continue;
+          // the column sums of the waves whose first strips (their longest) reach these columns
+          const int pn = min(cnt, pairs ? P - 2 * cb : S - 4 * cb);
+          float y = m.ysum[r], vw = 0.0f, ps[MD_WAVES];
+#pragma unroll
+          for (int i = 0; i < MD_WAVES; i++) ps[i] = m.part[i * np + r];
+#pragma unroll
+          for (int i = 0; i < MD_WAVES; i++) y += i < pn ? ps[i] : 0.0f;
+          y *= sc;
+          for (int j = 0; j < cc; j += 8) {
+            float2 z[8], d[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+              z[i] = m.VW[(j + i) * ld + r];
+              d[i] = dots[j + i];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+              if (j + i < cc) {  // (dots beyond cc are an earlier panel's)
+                y -= z[i].x * d[i].y + z[i].y * d[i].x;
+                vw += d[i].x * d[i].y;
+              }
+          }
+          const bool in = r >= s && r < n;
+          const float v = r == s ? 1.0f : u[h] * sc;
+          const float w = in ? tau * (y - tau * (va - vw) * v) : 0.0f;
+          m.VW[cc * ld + r] = float2{in ? v : 0.0f, w};
+        }
+      }
+      // v to memory for the back-transformation (rows above the panel's first are not read there)
+#pragma unroll
+      for (int h = 0; h < MD_RB; h++) {
+        const int rb = 64 * (wv + MD_WAVES * h), r = rb + l;
+        if (r < 16 * S && rb + 63 >= j0) V[(long long)k * ldv + r] = refl && r >= s ? (r == s ? 1.0f : u[h] * sc) : 0.0f;
+      }
+      if (tid == 0) {
+        tau_g[k] = tau;
+        eg[k] = ldexp((double)beta, ex);
+      }
+      __syncthreads();
+    }
+    if (j0 + MD_NB >= n) break;
+    // ---- the panel's rank-2k update of the trailing strips on the matrix cores (16 x 16 x 4 steps): lane
+    // l supplies -V(row l%16, j) and W(column l%16, j), then -W and V, for j = 4 ks + l/16; entry (i, c)
+    // of a 16 x 16 piece lands in lane 16 (i/4) + c, register i%4.  The diagonal pieces keep zeros
+    // above the diagonal and half the change on it.
+    const int p1 = (j0 >> 4) + 1, Sa = S - p1;
+    for (int q = 0; q * MD_WAVES < Sa; q++) {
+      const int i0 = q * MD_WAVES + (q & 1 ? MD_WAVES - 1 - wv : wv);
+      if (i0 >= Sa) continue;
+      const int st = S - 1 - i0;
+      float2 ar[4];
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) ar[ks] = m.VW[(4 * ks + lk) * ld + 16 * st + li];
+      float* tb = A + 1024 * md_strip(st) + 256 * lk + li;
+      auto piece = [&](int cs) { return tb + 1024 * (cs >> 2) + 16 * (cs & 3); };
+      auto mac = [&](int cs, flt4 acc) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+          const float2 b = m.VW[(4 * ks + lk) * ld + 16 * cs + li];
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-ar[ks].x, b.y, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-ar[ks].y, b.x, acc, 0, 0, 0);
+        }
+        return acc;
+      };
+      int cs = p1;
+      for (; cs + 4 <= st; cs += 4) {  // four pieces in flight
+        flt4 acc[4];
+#pragma unroll
+        for (int f = 0; f < 4; f++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[f][r] = piece(cs + f)[64 * r];
+#pragma unroll
+        for (int f = 0; f < 4; f++) acc[f] = mac(cs + f, acc[f]);
+#pragma unroll
+        for (int f = 0; f < 4; f++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) piece(cs + f)[64 * r] = acc[f][r];
+      }
+      for (; cs <= st; cs++) {
+        flt4 old, acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int r = 0; r < 4; r++) old[r] = piece(cs)[64 * r];
+        acc = mac(cs, acc);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int i = 4 * lk + r;
+          piece(cs)[64 * r] = cs < st || i > li ? old[r] + acc[r] : i == li ? old[r] + 0.5f * acc[r] : 0.0f;
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The rest of the reduction, columns 0 .. n-1 of an n x n matrix (n <= MD_REG), with the matrix in
+// registers and updated after every column.  Wave w holds the strips S-1-w, S-16+w and S-17-w: NT tiles of
+// each, lane (lk, li) rows 4 lk .. + 3 and columns 4 li .. + 3 of a tile.  The 16 x 16 piece on a strip's
+// diagonal is held in full and counts for its rows only; lanes right of it hold nothing that is read.
+// Three barriers per column: the column (in cb), the products' partial sums, v and w.
+struct MdReg {
+  float cb[MD_REG], vb[MD_REG], wb[MD_REG], ysum[MD_REG], cpart[MD_WAVES][MD_REG], ap[16];
+};
+template <int NT>
+struct MdStrip {
+  flt4 a[NT][4];
+  flt4 x, y;  // the strip's rows of u and the row sums; of v and w
+  int st;     // < 0: none
+
+  // from the tiles in memory (lower triangle, diagonal halved, rows from r0 = b0 on)
+  __device__ __forceinline__ void load(const float* A, int b0, int strip, int li, int lk) {
+    st = strip;
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        a[t][i] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (st < 0 || t > st >> 2) continue;
+        const int r = 16 * st + 4 * lk + i, c = 64 * t + 4 * li;
+        if (c >> 4 < st) {
+          a[t][i] = *reinterpret_cast<const flt4*>(A + 1024 * (md_strip((b0 + r) >> 4) + ((b0 + c) >> 6)) +
+                                                   (r & 15) * 64 + (c & 63));
+        } else if (c >> 4 == st) {
+#pragma unroll
+          for (int j = 0; j < 4; j++) {
+            const int hi = max(r, c + j), lo = min(r, c + j);
+            const float z = A[1024 * (md_strip((b0 + hi) >> 4) + ((b0 + lo) >> 6)) + (hi & 15) * 64 + (lo & 63)];
+            a[t][i][j] = hi == lo ? 2.0f * z : z;
+          }
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // a tile at a time: the next ones' loads would cost registers
+    }
+  }
+  // the last tile while row s or a later one is in the strip (the tiles before s's are skipped by the caller)
+  __device__ __forceinline__ int last(int s) const { return st >= s >> 4 ? st >> 2 : -1; }
+  // u's rows of the strip (zero above s, u0 at s), no row sums yet
+  __device__ __forceinline__ void begin(const MdReg& m, int s, float u0, int lk) {
+    if (st < s >> 4) return;
+    const int r4 = 16 * st + 4 * lk;
+    x = *reinterpret_cast<const flt4*>(m.cb + r4);
+    if (st == s >> 4)
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = r4 + i < s ? 0.0f : r4 + i == s ? u0 : x[i];
+    y = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  // tile t: row sums with the columns' u (uc), column sums added to ca
+  __device__ __forceinline__ void product(int t, const flt4& uc, flt4& ca, int li) {
+    flt4 ur = x, uy = uc;
+    if (t == st >> 2) {
+      const int d = (li >> 2) - (st & 3);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        ur[i] = d >= 0 ? 0.0f : ur[i];
+        uy[i] = d > 0 ? 0.0f : uy[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        ca[j] += a[t][i][j] * ur[i];
+        y[i] += a[t][i][j] * uy[j];
+      }
+  }
+  // the row sums into ysum; this lane's share of u^T A u from them
+  __device__ __forceinline__ float end(MdReg& m, int s, int li, int lk) const {
+    if (st < s >> 4) return 0.0f;
+    const float rs = md_rows(y, li);
+    if (li < 4) m.ysum[16 * st + 4 * lk + md_row(li)] = rs;
+    return (y[0] * x[0] + y[1] * x[1]) + (y[2] * x[2] + y[3] * x[3]);
+  }
+  __device__ __forceinline__ void rows_vw(const MdReg& m, int s, int lk) {
+    if (st < s >> 4) return;
+    x = *reinterpret_cast<const flt4*>(m.vb + 16 * st + 4 * lk);
+    y = *reinterpret_cast<const flt4*>(m.wb + 16 * st + 4 * lk);
+  }
+  __device__ __forceinline__ void update(int t, const flt4& vc, const flt4& wc) {
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) a[t][i][j] -= x[i] * wc[j] + y[i] * vc[j];
+  }
+  // column c of tile t into cb
+  __device__ __forceinline__ void column(MdReg& m, int t, int c, int li, int lk) const {
+    flt4 z;
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      z[i] = (c & 2) ? ((c & 1) ? a[t][i][3] : a[t][i][2]) : ((c & 1) ? a[t][i][1] : a[t][i][0]);
+    if (li == (c & 63) >> 2) *reinterpret_cast<flt4*>(m.cb + 16 * st + 4 * lk) = z;
+  }
+};
+__device__ __forceinline__ void md_resident(MdReg& m, const float* A, int b0, int n, int ex, float* V, int ldv,
+                                            float* tau_g, double* dg, double* eg) {
+  constexpr int NT = MD_REG / 64;
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, lk = l >> 4;
+  const int S = md_strips(n), nr = 16 * S, T = (nr + 63) >> 6;
+  MdStrip<5> A0;
+  MdStrip<3> A1;
+  MdStrip<1> A2;
+  A0.load(A, b0, S - 1 - wv, li, lk);
+  A1.load(A, b0, S - 16 + wv, li, lk);
+  A2.load(A, b0, S - 17 - wv, li, lk);
+  if (tid < 16) m.ap[tid] = 0.0f;
+  for (int r = tid; r < MD_REG; r += MD_THREADS) m.cb[r] = m.vb[r] = m.wb[r] = 0.0f;
+  __syncthreads();
+  auto column = [&](int s) {
+    const int l0 = A0.last(s), l1 = A1.last(s), l2 = A2.last(s);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+      if (t != s >> 6) continue;
+      if (t <= l0) A0.column(m, t, s, li, lk);
+      if (t < 3 && t <= l1) A1.column(m, t < 3 ? t : 0, s, li, lk);
+      if (t < 1 && t <= l2) A2.column(m, 0, s, li, lk);
+    }
+  };
+  column(0);
+  for (int k = 0;; k++) {
+    __syncthreads();
+    const int s = k + 1, t0 = s >> 6;
+    if (tid == k) dg[k] = ldexp((double)m.cb[k], ex);
+    if (s >= n) break;
+    // ---- the reflector, the same in every wave
+    float x;
+    {
+      const float z = m.cb[64 * t0 + l];
+      x = 64 * t0 + l > s ? z * z : 0.0f;
+    }
+    for (int rb = 64 * (t0 + 1); rb < nr; rb += 64) x += m.cb[rb + l] * m.cb[rb + l];
+    const float alpha = m.cb[s];
+    x = md_sum64(x);
+    float beta = alpha, tau = 0.0f, u0 = 0.0f, sc = 0.0f;
+    const bool refl = __builtin_amdgcn_readfirstlane(__float_as_int(x)) > __float_as_int(1e-24f);  // (see md_columns)
+    if (refl) {
+      beta = -copysignf(__builtin_amdgcn_sqrtf(alpha * alpha + x), alpha);
+      u0 = alpha - beta;
+      tau = -u0 * __builtin_amdgcn_rcpf(beta);
+      sc = __builtin_amdgcn_rcpf(u0);
+    }
+    if (tid == 0) {
+      tau_g[k] = tau;
+      eg[k] = ldexp((double)beta, ex);
+    }
+    if (refl) {
+      float asum = 0.0f;
+      A0.begin(m, s, u0, lk);
+      A1.begin(m, s, u0, lk);
+      A2.begin(m, s, u0, lk);
+      const int l0 = A0.last(s), l1 = A1.last(s), l2 = A2.last(s);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        if (t < t0) continue;
+        if (t >= T) break;
+        flt4 uc = *reinterpret_cast<const flt4*>(m.cb + 64 * t + 4 * li), ca = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (t == t0)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int c = 64 * t + 4 * li + i;
+            uc[i] = c < s ? 0.0f : c == s ? u0 : uc[i];
+          }
+        if (t <= l0) A0.product(t, uc, ca, li);
+        if (t < 3 && t <= l1) A1.product(t < 3 ? t : 0, uc, ca, li);
+        if (t < 1 && t <= l2) A2.product(0, uc, ca, li);
+        asum += (ca[0] * uc[0] + ca[1] * uc[1]) + (ca[2] * uc[2] + ca[3] * uc[3]);
+        m.cpart[wv][64 * t + 4 * li + lk] = md_add16(md_add32(ca[0], ca[2]), md_add32(ca[1], ca[3]));
+      }
+      asum += A0.end(m, s, li, lk);
+      asum += A1.end(m, s, li, lk);
+      asum += A2.end(m, s, li, lk);
+      asum = md_sum64(asum);
+      if (l == 0) m.ap[wv] = asum;
+      __syncthreads();
+      // ---- w = tau (A v) - (tau^2 / 2) (v^T A v) v
+      if (64 * wv < nr && 64 * wv + 63 >= s) {
+        const float va = sc * sc * md_sum16(m.ap[li]);
+        const int r = tid;
+        float y = m.ysum[r], p[MD_WAVES];
+#pragma unroll
+        for (int i = 0; i < MD_WAVES; i++) p[i] = m.cpart[i][r];
+        const float u = m.cb[r];
+        y += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+        const bool in = r >= s && r < n;
+        const float v = in ? (r == s ? 1.0f : u * sc) : 0.0f;
+        const float w = in ? tau * (y * sc - 0.5f * tau * va * v) : 0.0f;
+        m.vb[r] = v;
+        m.wb[r] = w;
+        if (r < nr) V[(long long)k * ldv + r] = v;
+      }
+      __syncthreads();
+      A0.rows_vw(m, s, lk);
+      A1.rows_vw(m, s, lk);
+      A2.rows_vw(m, s, lk);
+#pragma unroll
+      for (int t = 0; t < NT; t++) {
+        if (t < t0) continue;
+        if (t >= T) break;
+        const flt4 vc = *reinterpret_cast<const flt4*>(m.vb + 64 * t + 4 * li);
+        const flt4 wc = *reinterpret_cast<const flt4*>(m.wb + 64 * t + 4 * li);
+        if (t <= l0) A0.update(t, vc, wc);
+        if (t < 3 && t <= l1) A1.update(t < 3 ? t : 0, vc, wc);
+        if (t < 1 && t <= l2) A2.update(0, vc, wc);
+      }
+    } else {
+      __syncthreads();  // every wave has read the column
+    }
+    // v's zero rows from the panel's first on (the back-transformation reads no earlier ones): those before
+    // the waves that store v, or all of them
+    if (tid >= (k & ~(MD_NB - 1)) && tid < (refl ? s & ~63 : nr)) V[(long long)k * ldv + tid] = 0.0f;
+    column(s);
+  }
+}
+
+// One block per workgroup.  While more than MD_REG rows are left the working matrix is read from L2 (one CU
+// takes 64 B per clock at best, 44 B achieved: 11 us per column at 620 rows, which bounds blocks of 400 rows
+// and more); the rest of the reduction runs on the trailing matrix in registers, 2.0 .. 2.9 us per column
+// for 100 .. 320 rows, bound by the chain of its three phases (from LDS it took 2.8 .. 4.5 us).  Whole blocks:
+// 0.19 ms at 96 rows, 0.44 at 192, 0.91 at 320, 2.5 at 512, 4.1 at 619, 6.4 at 768.
+__global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __restrict__ bl,
+                                                           const double* __restrict__ Ha, float* __restrict__ Aa,
+                                                           float* __restrict__ Va, float* __restrict__ taua,
+                                                           double* __restrict__ Wsa) {
+  extern __shared__ float4 lds4[];
+  float* lds = reinterpret_cast<float*>(lds4);
+  const MidBlock B = bl[blockIdx.x];
+  const int n = B.n, ldv = 16 * md_strips(n);
+  __shared__ double s_max[MD_WAVES];
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
+  const double* H = Ha + B.h_off;
+  float* A = Aa + B.p_off;
+  float* V = Va + B.v_off;
+  float* tau = taua + B.e_off;
+  const HtWs ws = ht_ws(Wsa + B.w_off, n, B.T);
+  // ---- the block scaled by a power of two to entries of at most one, in FP32
+  double mx = 0.0;
+  for (int r = wv; r < n; r += MD_WAVES)
+    for (int c = l; c <= r; c += 64) {
+      const double h = fabs(H[(long long)r * n + c]);
+      mx = h > mx || h != h ? h : mx;  // NaN stays
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const double h = __shfl_xor(mx, o, 64);
+    mx = h > mx || h != h ? h : mx;
+  }
+  if (l == 0) s_max[wv] = mx;
+  __syncthreads();
+  for (int w = 0; w < MD_WAVES; w++) mx = s_max[w] > mx || s_max[w] != s_max[w] ? s_max[w] : mx;
+  // (a NaN or an infinity goes on into X and the refinement, which leaves such a block unconverged)
+  const int ex = mx > 0.0 && mx <= 1.7976931348623157e308 ? ilogb(mx) + 1 : 0;
+  for (int r = wv; r < ldv; r += MD_WAVES) {
+    float* dst = A + 1024 * md_strip(r >> 4) + (r & 15) * 64;
+    for (int c = l, t = 0; t <= r >> 6; c += 64, t++) {
+      const double h = r < n && c <= r ? ldexp(H[(long long)r * n + c], -ex) : 0.0;
+      dst[t * 1024 + l] = (float)(c == r ? 0.5 * h : h);
+    }
+  }
+  __syncthreads();
+  const int b0 = n > MD_REG ? (n - MD_REG + 63) / 64 * 64 : 0;  // columns reduced in memory
+  if (b0 > 0) md_columns(A, md_lds(lds, n), n, b0, ex, V, ldv, tau, ws.d, ws.e);
+  md_resident(*reinterpret_cast<MdReg*>(lds), A, b0, n - b0, ex, V + (long long)b0 * ldv + b0, ldv, tau + b0,
+              ws.d + b0, ws.e + b0);
+}
+
+// The WY factor of panel p of each block: T_p upper triangular with H_{j0} .. H_{j0+nb-1} =
+// I - V_p T_p V_p^T (forward, columnwise); V_p T_p goes to VT beside V (columns of zeros past the last
+// reflector).
+__global__ void __launch_bounds__(256) k_mid_larft(const MidBlock* __restrict__ bl, int nblk,
+                                                   const float* __restrict__ Va, const float* __restrict__ taua,
+                                                   float* __restrict__ VTa) {
+  int g = blockIdx.x, b = -1;
+  for (int i = 0; i < nblk; i++) {
+    const int P = (bl[i].n + MD_NB - 2) / MD_NB;
+    if (g < P) {
+      b = i;
+      break;
+    }
+    g -= P;
+  }
+  if (b < 0) return;
+  const MidBlock B = bl[b];
+  const int n = B.n, ldv = 16 * md_strips(n), j0 = g * MD_NB, nb = min(MD_NB, n - 1 - j0);
+  const float* V = Va + B.v_off + (long long)j0 * ldv;
+  float* VT = VTa + B.v_off + (long long)j0 * ldv;
+  __shared__ float St[MD_NB][65], G[MD_NB][MD_NB + 1], T[MD_NB][MD_NB + 1];
+  const int tid = threadIdx.x, a = tid >> 4, c = tid & 15;
+  float acc = 0.0f;
+  for (int r0 = j0; r0 < ldv; r0 += 64) {
+    for (int e = tid; e < MD_NB * 64; e += 256) {
+      const int j = e >> 6, r = r0 + (e & 63);
+      St[j][e & 63] = j < nb && r < ldv ? V[(long long)j * ldv + r] : 0.0f;
+    }
+    __syncthreads();
+    for (int q = 0; q < 64; q++) acc += St[a][q] * St[c][q];
+    __syncthreads();
+  }
+  G[a][c] = acc;
+  T[a][c] = 0.0f;
+  __syncthreads();
+  for (int i = 0; i < nb; i++) {
+    const float ti = taua[B.e_off + j0 + i];
+    float x = 0.0f;
+    if (tid < i)
+      for (int q = tid; q < i; q++) x += T[tid][q] * G[q][i];
+    __syncthreads();
+    if (tid < i) T[tid][i] = -ti * x;
+    if (tid == i) T[i][i] = ti;
+    __syncthreads();
+  }
+  for (int e = tid; e < MD_NB * ldv; e += 256) {
+    const int j = e / ldv, r = e - j * ldv;
+    float x = 0.0f;
+    if (r > j0)
+      for (int i = 0; i <= min(j, nb - 1); i++) x += V[(long long)i * ldv + r] * T[i][j];
+    if (j0 + j < ldv) VT[(long long)j * ldv + r] = x;
+  }
+}
+
+// X = Q Z for 64 columns of one block: Z (FP64, the eigenvectors of T) in the matrix-core layout in
+// registers (wave w: row tiles w, w + 16, w + 32), the panels applied last first, Z -= (V_p T_p) (V_p^T Z).
+// Register r of a 16 x 16 piece holds rows 4 (l/16) + r of it, which is the right-hand operand of a
+// 4-row step over those rows as it stands, so Z never leaves the registers; each wave's share of
+// V_p^T Z meets the others' in LDS.
+constexpr int MB_THREADS = 1024;
+constexpr int MB_WAVES = MB_THREADS / 64;
+constexpr int MB_RT = MD_MAX / 16 / MB_WAVES;
+__global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restrict__ bl, int nblk,
+                                                         const float* __restrict__ Va, const float* __restrict__ VTa,
+                                                         double* __restrict__ Xa) {
+  __shared__ float Yp[MB_WAVES][MD_NB][64];
+  __shared__ float Ys[MD_NB][80];
+  int g = blockIdx.x, b = -1;
+  for (int i = 0; i < nblk; i++) {
+    const int ct = (bl[i].n + 63) / 64;
+    if (g < ct) {
+      b = i;
+      break;
+    }
+    g -= ct;
+  }
+  if (b < 0) return;
+  const MidBlock B = bl[b];
+  const int n = B.n, ldv = 16 * md_strips(n), NT = ldv / 16;
+  const float* V = Va + B.v_off;
+  const float* VT = VTa + B.v_off;
+  double* X = Xa + B.h_off;
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
+  flt4 z[MB_RT][4];
+#pragma unroll
+  for (int q = 0; q < MB_RT; q++)
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 64 * g + 16 * ct + li;
+        z[q][ct][r] = row < n && col < n ? (float)X[(long long)row * n + col] : 0.0f;
+      }
+  for (int p = n > 1 ? (n - 2) / MD_NB : -1; p >= 0; p--) {
+    const int j0 = p * MD_NB;  // panel column j0 + j beyond n - 2 has no reflector: V T is zero there
+    flt4 y[4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) y[ct] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int q = 0; q < MB_RT; q++) {
+      const int rt = wv + MB_WAVES * q;
+      if (rt < p || rt >= NT) continue;
+      flt4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (j0 + li < n - 1) a = *reinterpret_cast<const flt4*>(V + (long long)(j0 + li) * ldv + 16 * rt + 4 * lk);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++) y[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], z[q][ct][r], y[ct], 0, 0, 0);
+    }
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) Yp[wv][4 * lk + r][16 * ct + li] = y[ct][r];
+    __syncthreads();
+    {
+      float acc = 0.0f;
+#pragma unroll
+      for (int w = 0; w < MB_WAVES; w++) acc += Yp[w][tid >> 6][l];
+      Ys[tid >> 6][l] = acc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < MB_RT; q++) {
+      const int rt = wv + MB_WAVES * q;
+      if (rt < p || rt >= NT) continue;
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++) {
+        const int j = 4 * ks + lk;
+        const float a = j0 + j < ldv ? -VT[(long long)(j0 + j) * ldv + 16 * rt + li] : 0.0f;
+#pragma unroll
+        for (int ct = 0; ct < 4; ct++)
+          z[q][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Ys[j][16 * ct + li], z[q][ct], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < MB_RT; q++)
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 64 * g + 16 * ct + li;
+        if (row < n && col < n) X[(long long)row * n + col] = (double)z[q][ct][r];
+      }
+}
+
+// Eigenvalues of T (d, e) by multisection on Sturm counts: eight lanes per eigenvalue count at eight
+// inner points of its interval, which shrinks ninefold a pass, until it is rtol ||T|| wide.  The counts
+// run on the characteristic polynomials p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2} (a sign change per
+// eigenvalue below x): one fused operation on the dependent chain of a step, where the quotients
+// p_i / p_{i-1} of the usual form take a reciprocal and three more.  T is scaled to about unit norm, so
+// the polynomials stay in range over eight steps, after which they are rescaled by a power of two.
+constexpr int ST_LANES = 8;
+constexpr int ST_PER = 256 / ST_LANES;  // eigenvalues per workgroup
+constexpr int ST_UNROLL = 8;
+__global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
+                                                  double* __restrict__ lam, double rtol) {
+  extern __shared__ double2 de[];  // {d_i, e_{i-1}^2}, filled up to a multiple of ST_UNROLL
+  int g = blockIdx.x, b = -1;
+  for (int i = 0; i < nblk; i++) {
+    const int cw = (bl[i].n + ST_PER - 1) / ST_PER;
+    if (g < cw) {
+      b = i;
+      break;
+    }
+    g -= cw;
+  }
+  if (b < 0) return;
+  const HtBlock B = bl[b];
+  const int n = B.n, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
+  const HtWs w = ht_ws(const_cast<double*>(Wa) + B.w_off, n, B.T);
+  __shared__ double rlo[4], rhi[4];
+  double lo = 1e300, hi = -1e300;
+  for (int i = tid; i < n; i += 256) {
+    const double di = w.d[i], rad = (i < n - 1 ? fabs(w.e[i]) : 0.0) + (i > 0 ? fabs(w.e[i - 1]) : 0.0);
+    lo = fmin(lo, di - rad);
+    hi = fmax(hi, di + rad);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+  }
+  if (l == 0) {
+    rlo[wv] = lo;
+    rhi[wv] = hi;
+  }
+  __syncthreads();
+  lo = fmin(fmin(rlo[0], rlo[1]), fmin(rlo[2], rlo[3]));
+  hi = fmax(fmax(rhi[0], rhi[1]), fmax(rhi[2], rhi[3]));
+  const double tn = fmax(fabs(lo), fabs(hi));
+  const int j = g * ST_PER + tid / ST_LANES, ln = tid & (ST_LANES - 1);
+  if (!(tn > 0.0 && tn <= 1.7976931348623157e308)) {  // T = 0: every eigenvalue is exactly zero
+    if (j < n && ln == 0) lam[B.e_off + j] = 0.0;
+    return;
+  }
+  const int ex = ilogb(tn) + 1;  // ||T|| in [1/2, 1) after scaling
+  const int nf = (n + ST_UNROLL - 1) / ST_UNROLL * ST_UNROLL;
+  for (int i = tid; i < nf; i += 256) {
+    const double e = i > 0 && i < n ? ldexp(w.e[i - 1], -ex) : 0.0;
+    de[i] = double2{i < n ? ldexp(w.d[i], -ex) : 4.0, e * e};  // (rows past the end: a 1 x 1 block above all)
+  }
+  __syncthreads();
+  const double eps = 2.220446049250313e-16;
+  double a = ldexp(lo, -ex) - 4.0 * eps, c = ldexp(hi, -ex) + 4.0 * eps;
+  // a pivot p_i / p_{i-1} below this is moved to it from below (as the quotient form moves a vanishing one)
+  constexpr double PIV = 1e-32;
+  const bool mine = j < n;
+  const double tol = fmax(rtol, 0.5 * eps);
+  for (int it = 0; it < 24; it++) {
+    const bool go = mine && c - a > tol;
+    if (__ballot(go) == 0) break;
+    const double h = (c - a) * (1.0 / (ST_LANES + 1)), x = a + (ln + 1) * h;
+    int cnt = 0;
+    double p1 = 1.0, p2 = 0.0;
+    for (int i0 = 0; i0 < nf; i0 += ST_UNROLL) {
+      double2 t[ST_UNROLL];
+#pragma unroll
+      for (int i = 0; i < ST_UNROLL; i++) t[i] = de[i0 + i];
+#pragma unroll
+      for (int i = 0; i < ST_UNROLL; i++) {
+        double p = fma(t[i].x - x, p1, -t[i].y * p2);
+        p = fabs(p) < PIV * fabs(p1) ? -PIV * p1 : p;
+        cnt += (int)((unsigned)(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
+        p2 = p1;
+        p1 = p;
+      }
+      const int sh = -__builtin_amdgcn_frexp_exp(fmax(fabs(p1), fabs(p2)));
+      p1 = __builtin_amdgcn_ldexp(p1, sh);
+      p2 = __builtin_amdgcn_ldexp(p2, sh);
+    }
+    // points at or below the eigenvalue: those with at most j eigenvalues below them
+    const unsigned long long in = __ballot(cnt <= j);
+    const int m = __popc((unsigned)(in >> (l & ~(ST_LANES - 1))) & ((1u << ST_LANES) - 1));
+    if (go) {
+      const double na = a + m * h;
+      c = m == ST_LANES ? c : a + (m + 1) * h;
+      a = na;
+    }
+  }
+  if (mine && ln == 0) lam[B.e_off + j] = ldexp(0.5 * (a + c), ex);
+}
+
+// ----------------------------------------------------------------------------- launchers
+static size_t mid_reduce_lds(int n) {
+  const size_t mem = ((size_t)2 * MD_NB * md_ld(n) + (size_t)(MD_WAVES + 2) * md_np(n)) * sizeof(float);  // md_lds
+  return std::max(n > MD_REG ? mem : 0, sizeof(MdReg));
+}
+void launch_mid_reduce(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const double* H, float* A, float* V,
+                       float* tau, double* W, hipStream_t s) {
+  int nmax = 1;
+  for (const auto& b : bl) nmax = std::max(nmax, b.n);
+  NRGK_REQUIRE(nmax <= MD_MAX, NRGK_ERR_INVALID, "nrgk: block too wide for the batched tridiagonalisation");
+  NRGK_LAUNCH(k_mid_reduce, dim3((unsigned)bl.size()), dim3(MD_THREADS), mid_reduce_lds(nmax), s, d_bl, H, A, V, tau, W);
+  NRGK_HIP(hipGetLastError());
+}
+void launch_mid_back(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const float* V, const float* tau, float* VT,
+                     double* X, hipStream_t s) {
+  int gp = 0, gc = 0;
+  for (const auto& b : bl) {
+    gp += (b.n + MD_NB - 2) / MD_NB;
+    gc += (b.n + 63) / 64;
+  }
+  NRGK_LAUNCH(k_mid_larft, dim3(gp), dim3(256), 0, s, d_bl, (int)bl.size(), V, tau, VT);
+  NRGK_HIP(hipGetLastError());
+  NRGK_LAUNCH(k_mid_back, dim3(gc), dim3(MB_THREADS), 0, s, d_bl, (int)bl.size(), V, (const float*)VT, X);
+  NRGK_HIP(hipGetLastError());
+}
+void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
+                     hipStream_t s) {
+  int g = 0, nmax = 1;
+  for (const auto& b : bl) {
+    g += (b.n + ST_PER - 1) / ST_PER;
+    nmax = std::max(nmax, b.n);
+  }
+  if (!g) return;
+  NRGK_LAUNCH(k_ht_sturm, dim3(g), dim3(256), (size_t)(nmax + ST_UNROLL) * sizeof(double2), s, d_bl, (int)bl.size(), W,
+              lam, rtol);
+  NRGK_HIP(hipGetLastError());
+}
+void set_mid_lds_limits(int bytes) {
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_mid_reduce, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)mid_reduce_lds(MD_MAX)));
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm, hipFuncAttributeMaxDynamicSharedMemorySize, bytes - 8192));
+}
+
+}  // namespace nrgk

@@ -55,7 +55,7 @@ __device__ __forceinline__ dbl4 sm_tile(const double* A, const double* B, int ld
   return acc;
 }
 
-// status[b] is 1 if block b has a non-finite entry or did not converge; sweeps: the most of any block.
+// status[b] (zero before) is 1 if block b did not converge; sweeps: the most of any block.
 __global__ void __launch_bounds__(SM_THREADS) k_eig_small(const EigBlock* __restrict__ blocks,
                                                           const double* __restrict__ Ha, double* __restrict__ Ua,
                                                           double* __restrict__ lam, int* __restrict__ status,
@@ -90,8 +90,10 @@ __global__ void __launch_bounds__(SM_THREADS) k_eig_small(const EigBlock* __rest
     rad = fmax(rad, ev[k]);
     finite = finite && ev[k] <= 1.7976931348623157e308;
   }
-  if (!finite) {  // NaN or infinity: the block is left to the caller's fallback
-    if (tid == 0) status[blockIdx.x] = 1;
+  if (!finite) {  // NaN or infinity in: NaN out (a chain's truncation reports it)
+    const double nan = __longlong_as_double(0x7ff8000000000000ll);
+    for (int e = tid; e < n * n; e += SM_THREADS) Ua[blk.off + e] = nan;
+    if (tid < n) lam[blk.e_off + tid] = nan;
     return;
   }
   const int ex = rad > 0.0 ? ilogb(rad) + 1 : 0;

@@ -1,4 +1,4 @@
-// K3-K5: the eigensolver of the wide sector blocks (above the batched Jacobi's crossover), replacing
+// K3-K5: the eigensolver of the wide sector blocks (above the batched solver's crossover), replacing
 // per-block LAPACKE_dsyevd (nrgcore/include/utils/qmatrix.hpp:375-404) for those blocks.
 //
 // 1. Blocked Householder tridiagonalisation in FP64 (the lower-triangle form: reflector H_k = I -

@@ -8,14 +8,7 @@ namespace nrgk {
 void launch_assemble(const AsmSector* sectors, int n_sectors, int n_rows, const AsmSub* subs, const AsmCon* cons,
                      const double* e_prev, const double* e_bath, const double* f_prev, const double* f_bath,
                      double rescale, double* H, hipStream_t s);
-void launch_shift_convert(const EigBlock* blocks, const int* row_block, const int* row_local, int n_rows,
-                          const double* H, unsigned int* sigma_bits, float* sigma_out, float* W, hipStream_t s);
 // k_eig.hip
-void launch_jacobi_round(const JacTask* tasks, int n_tasks, float* W, int round, int* flags, double* dgram, int* dgv,
-                         float tol, float ang_tol, int max_inner, double jac_far, hipStream_t s);
-void launch_normalize_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_tiles, const int4* groups,
-                           int n_groups, const float* W, const float* sigma, double* X, double* lam, int* perm,
-                           double* nrm_s, double* nrm_g, size_t lds, hipStream_t s);
 void launch_oa(const EigBlock* blocks, int nb, const int4* sym_tiles, int n_sym, const int4* all_tiles, int n_all,
                double* S, double* Rp, double* E, double* lam, int* cid, int* sidx, double* offmax, int* stats,
                double* conv, double* scrW, double* scrG, double* scrT, double* rrv, int nmax, double e_tol,
@@ -24,7 +17,6 @@ void launch_copy_converged(const EigBlock* blocks, int nb, const double* conv, d
                            double e_pred, double d_pred, const double* src, double* dst, hipStream_t s);
 void launch_final_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_tiles, const double* X,
                        const double* lam_in, double* U, double* lam_out, int* perm, size_t lds, hipStream_t s);
-size_t normalize_sort_lds(int nmax);
 size_t final_sort_lds(int nmax);
 void set_kernel_lds_limits(int bytes);
 // k_small.hip: blocks of up to SM_MAX rows, solved whole by one workgroup each
@@ -32,6 +24,19 @@ constexpr int SM_MAX = 64;
 void launch_eig_small(const EigBlock* blocks, int nb, int nmax, const double* H, double* U, double* lam, int* status,
                       int* sweeps, hipStream_t s);
 void set_small_lds_limit();
+// k_mid.hip: FP32 start vectors of the wider blocks of the batched solve
+constexpr int MD_NB = 16;    // panel width
+constexpr int MD_MAX = 768;  // the widest block whose panel and column sums fit a workgroup's LDS
+long long md_matrix_floats(int n);  // floats of a block's working matrix
+int md_ldv(int n);                  // row stride (and rows) of its Householder vectors
+void launch_mid_reduce(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const double* H, float* A, float* V,
+                       float* tau, double* W, hipStream_t s);
+void launch_mid_back(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const float* V, const float* tau, float* VT,
+                     double* X, hipStream_t s);
+// eigenvalues of T to rtol ||T||
+void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
+                     hipStream_t s);
+void set_mid_lds_limits(int bytes);
 // k_gemm.hip
 int prepare_gemm(std::vector<GemmProb>& probs);
 void launch_gemm(const GemmProb* d_probs, int n_probs, int tiles, hipStream_t s);

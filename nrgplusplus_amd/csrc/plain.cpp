@@ -93,11 +93,11 @@ void Chain::eigensolve_plain() {
 }
 
 
-// The crossover of the batched solver: a block wider than its LDS-resident Jacobi panel (768 rows)
+// The crossover of the batched solver: a block wider than it takes (768 rows)
 // is solved by rocSOLVER dsyevd -- Householder tridiagonalisation with blocked (GEMM) trailing
 // updates, then divide and conquer, all in FP64 -- on side streams of the chain (largest blocks
 // first, each to the stream with the least n^3 so far), while the main stream runs the batched FP32
-// Jacobi and FP64 refinement of the other blocks.  The side streams write only the rows of their
+// solve and FP64 refinement of the other blocks.  The side streams write only the rows of their
 // blocks in X (scratch), U and the raw eigenvalues, and have their own work and info arrays, so no
 // two streams share memory.  All streams keep the default priority.
 void large_blocks_begin(Chain& c, const std::vector<int>& sectors) {

@@ -1,9 +1,9 @@
 // Autotuning of the eigensolver's crossover (no counterpart in the reference): the block width above
-// which a sector block leaves the batched FP32 Jacobi (+ FP64 refinement) for the FP64 Householder
+// which a sector block leaves the batched FP32 solve (+ FP64 refinement) for the FP64 Householder
 // path.  For each candidate width n, a batch of random symmetric n x n blocks is solved both ways on
-// the device -- the Jacobi path forming every eigenvector (the refinement needs them), the Householder
+// the device -- the batched path forming every eigenvector (the refinement needs them), the Householder
 // path the eigenvalues and the first n/4 eigenvectors (the kept columns an RG step reads) -- and the
-// crossover is the widest candidate at which the Jacobi path is not slower.  The result is cached in a
+// crossover is the widest candidate at which the batched path is not slower.  The result is cached in a
 // text file per GPU model and CU count, which every context reads when it is created.
 #include <chrono>
 #include <cstdio>
@@ -43,7 +43,7 @@ void tune_load(Ctx& c) {
   }
 }
 
-// one timed solve of the blocks: eigenvalues of all, eigenvectors of all (Jacobi) or of the first
+// one timed solve of the blocks: eigenvalues of all, eigenvectors of all (batched) or of the first
 // quarter of the columns (Householder), ms of device work between two stream synchronisations
 static double timed_solve(Ctx* ctx, const std::vector<int>& dims, const std::vector<double>& H, int mixed_max) {
   Chain c(ctx, NRGK_MODE_MIXED);
@@ -109,7 +109,7 @@ int tune_crossover(Ctx* ctx, const std::string& path, std::vector<std::vector<do
       f << "gpu " << ctx->arch << " " << ctx->n_cu << "\n";
       f << "crossover " << cross << "\n";
       for (auto& r : table)
-        f << "# n " << (int)r[0] << " blocks " << (int)r[1] << " jacobi_ms " << r[2] << " householder_ms " << r[3] << "\n";
+        f << "# n " << (int)r[0] << " blocks " << (int)r[1] << " batched_ms " << r[2] << " householder_ms " << r[3] << "\n";
     }
   }
   return cross;
