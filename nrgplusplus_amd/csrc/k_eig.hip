@@ -876,7 +876,7 @@ void launch_final_sort(const EigBlock* blocks, int nb, const int4* tiles, int n_
 void set_kernel_lds_limits(int bytes) {
   set_trunc_lds_limit();
   set_small_lds_limit();
-  set_mid_lds_limits(bytes);
+  set_mid_lds_limit();
   NRGK_HIP(hipFuncSetAttribute((const void*)k_oa_prep, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_oa_rr, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_final_sort, hipFuncAttributeMaxDynamicSharedMemorySize, bytes));

@@ -788,103 +788,6 @@ __global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restr
       }
 }
 
-// Eigenvalues of T (d, e) by multisection on Sturm counts: eight lanes per eigenvalue count at eight
-// inner points of its interval, which shrinks ninefold a pass, until it is rtol ||T|| wide.  The counts
-// run on the characteristic polynomials p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2} (a sign change per
-// eigenvalue below x): one fused operation on the dependent chain of a step, where the quotients
-// p_i / p_{i-1} of the usual form take a reciprocal and three more.  T is scaled to about unit norm, so
-// the polynomials stay in range over eight steps, after which they are rescaled by a power of two.
-constexpr int ST_LANES = 8;
-constexpr int ST_PER = 256 / ST_LANES;  // eigenvalues per workgroup
-constexpr int ST_UNROLL = 8;
-__global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
-                                                  double* __restrict__ lam, double rtol) {
-  extern __shared__ double2 de[];  // {d_i, e_{i-1}^2}, filled up to a multiple of ST_UNROLL
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int cw = (bl[i].n + ST_PER - 1) / ST_PER;
-    if (g < cw) {
-      b = i;
-      break;
-    }
-    g -= cw;
-  }
-  if (b < 0) return;
-  const HtBlock B = bl[b];
-  const int n = B.n, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
-  const HtWs w = ht_ws(const_cast<double*>(Wa) + B.w_off, n, B.T);
-  __shared__ double rlo[4], rhi[4];
-  double lo = 1e300, hi = -1e300;
-  for (int i = tid; i < n; i += 256) {
-    const double di = w.d[i], rad = (i < n - 1 ? fabs(w.e[i]) : 0.0) + (i > 0 ? fabs(w.e[i - 1]) : 0.0);
-    lo = fmin(lo, di - rad);
-    hi = fmax(hi, di + rad);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    lo = fmin(lo, __shfl_xor(lo, o, 64));
-    hi = fmax(hi, __shfl_xor(hi, o, 64));
-  }
-  if (l == 0) {
-    rlo[wv] = lo;
-    rhi[wv] = hi;
-  }
-  __syncthreads();
-  lo = fmin(fmin(rlo[0], rlo[1]), fmin(rlo[2], rlo[3]));
-  hi = fmax(fmax(rhi[0], rhi[1]), fmax(rhi[2], rhi[3]));
-  const double tn = fmax(fabs(lo), fabs(hi));
-  const int j = g * ST_PER + tid / ST_LANES, ln = tid & (ST_LANES - 1);
-  if (!(tn > 0.0 && tn <= 1.7976931348623157e308)) {  // T = 0: every eigenvalue is exactly zero
-    if (j < n && ln == 0) lam[B.e_off + j] = 0.0;
-    return;
-  }
-  const int ex = ilogb(tn) + 1;  // ||T|| in [1/2, 1) after scaling
-  const int nf = (n + ST_UNROLL - 1) / ST_UNROLL * ST_UNROLL;
-  for (int i = tid; i < nf; i += 256) {
-    const double e = i > 0 && i < n ? ldexp(w.e[i - 1], -ex) : 0.0;
-    de[i] = double2{i < n ? ldexp(w.d[i], -ex) : 4.0, e * e};  // (rows past the end: a 1 x 1 block above all)
-  }
-  __syncthreads();
-  const double eps = 2.220446049250313e-16;
-  double a = ldexp(lo, -ex) - 4.0 * eps, c = ldexp(hi, -ex) + 4.0 * eps;
-  // a pivot p_i / p_{i-1} below this is moved to it from below (as the quotient form moves a vanishing one)
-  constexpr double PIV = 1e-32;
-  const bool mine = j < n;
-  const double tol = fmax(rtol, 0.5 * eps);
-  for (int it = 0; it < 24; it++) {
-    const bool go = mine && c - a > tol;
-    if (__ballot(go) == 0) break;
-    const double h = (c - a) * (1.0 / (ST_LANES + 1)), x = a + (ln + 1) * h;
-    int cnt = 0;
-    double p1 = 1.0, p2 = 0.0;
-    for (int i0 = 0; i0 < nf; i0 += ST_UNROLL) {
-      double2 t[ST_UNROLL];
-#pragma unroll
-      for (int i = 0; i < ST_UNROLL; i++) t[i] = de[i0 + i];
-#pragma unroll
-      for (int i = 0; i < ST_UNROLL; i++) {
-        double p = fma(t[i].x - x, p1, -t[i].y * p2);
-        p = fabs(p) < PIV * fabs(p1) ? -PIV * p1 : p;
-        cnt += (int)((unsigned)(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
-        p2 = p1;
-        p1 = p;
-      }
-      const int sh = -__builtin_amdgcn_frexp_exp(fmax(fabs(p1), fabs(p2)));
-      p1 = __builtin_amdgcn_ldexp(p1, sh);
-      p2 = __builtin_amdgcn_ldexp(p2, sh);
-    }
-    // points at or below the eigenvalue: those with at most j eigenvalues below them
-    const unsigned long long in = __ballot(cnt <= j);
-    const int m = __popc((unsigned)(in >> (l & ~(ST_LANES - 1))) & ((1u << ST_LANES) - 1));
-    if (go) {
-      const double na = a + m * h;
-      c = m == ST_LANES ? c : a + (m + 1) * h;
-      a = na;
-    }
-  }
-  if (mine && ln == 0) lam[B.e_off + j] = ldexp(0.5 * (a + c), ex);
-}
-
 // ----------------------------------------------------------------------------- launchers
 static size_t mid_reduce_lds(int n) {
   const size_t mem = ((size_t)2 * MD_NB * md_ld(n) + (size_t)(MD_WAVES + 2) * md_np(n)) * sizeof(float);  // md_lds
@@ -910,22 +813,9 @@ void launch_mid_back(const MidBlock* d_bl, const std::vector<MidBlock>& bl, cons
   NRGK_LAUNCH(k_mid_back, dim3(gc), dim3(MB_THREADS), 0, s, d_bl, (int)bl.size(), V, (const float*)VT, X);
   NRGK_HIP(hipGetLastError());
 }
-void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
-                     hipStream_t s) {
-  int g = 0, nmax = 1;
-  for (const auto& b : bl) {
-    g += (b.n + ST_PER - 1) / ST_PER;
-    nmax = std::max(nmax, b.n);
-  }
-  if (!g) return;
-  NRGK_LAUNCH(k_ht_sturm, dim3(g), dim3(256), (size_t)(nmax + ST_UNROLL) * sizeof(double2), s, d_bl, (int)bl.size(), W,
-              lam, rtol);
-  NRGK_HIP(hipGetLastError());
-}
-void set_mid_lds_limits(int bytes) {
+void set_mid_lds_limit() {
   NRGK_HIP(hipFuncSetAttribute((const void*)k_mid_reduce, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)mid_reduce_lds(MD_MAX)));
-  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm, hipFuncAttributeMaxDynamicSharedMemorySize, bytes - 8192));
 }
 
 }  // namespace nrgk

@@ -19,8 +19,7 @@
 //    Every scalar a later launch needs (the reflector of column k from the norm partials) is
 //    recomputed by each workgroup from the same partials in the same order, so all agree bit for bit
 //    and no launch waits on a single-workgroup reduction.
-// 2. Eigenvalues of T by bisection on Sturm counts (one thread per eigenvalue, T in LDS), ascending
-//    as dsyevd returns them.
+// 2. Eigenvalues of T by multisection on Sturm counts (T in LDS), ascending as dsyevd returns them.
 // 3. Eigenvectors of T by inverse iteration with partial-pivoting LU of T - lambda I (one lane per
 //    eigenvector, all iterated at once; after every step the members of each cluster of eigenvalues
 //    closer than ctol are made orthonormal by modified Gram-Schmidt, one workgroup per cluster from
@@ -605,14 +604,24 @@ __global__ void __launch_bounds__(256) k_ht_syr2k(const HtBlock* __restrict__ bl
   }
 }
 
-// Eigenvalues of T (d, e) by bisection on the Sturm count, the j-th smallest by thread j; T is read
-// from LDS (every thread walks the same entries).
-__global__ void __launch_bounds__(256) k_ht_stebz(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
-                                                  double* __restrict__ lam) {
-  extern __shared__ double lds[];
+// Eigenvalues of T (d, e) by multisection on Sturm counts: LANES lanes per eigenvalue count at as many
+// inner points of its interval, which shrinks (LANES + 1)-fold a pass, until it is rtol ||T|| wide.  The counts
+// run on the characteristic polynomials p_i = (d_i - x) p_{i-1} - e_{i-1}^2 p_{i-2} (a sign change per
+// eigenvalue below x): one fused operation on the dependent chain of a step, where the quotients
+// p_i / p_{i-1} of the usual form take a reciprocal and three more.  T is scaled to about unit norm, so
+// the polynomials stay in range over eight steps, after which they are rescaled by a power of two.
+// A pass costs a wavefront about nine operations a row whatever LANES is, so eight lanes pay while the
+// wavefronts still find free SIMDs (17 passes instead of 52: five blocks of ~1 000 rows 2.3 -> 0.4 ms); where
+// the eigenvalues alone fill the chip, one lane each does the least work.
+constexpr int ST_UNROLL = 8;
+template <int ST_LANES>
+__global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
+                                                  double* __restrict__ lam, double rtol) {
+  extern __shared__ double2 de[];  // {d_i, e_{i-1}^2}, filled up to a multiple of ST_UNROLL
+  constexpr int ST_PER = 256 / ST_LANES;  // eigenvalues per workgroup
   int g = blockIdx.x, b = -1;
   for (int i = 0; i < nblk; i++) {
-    const int cw = (bl[i].n + 255) / 256;
+    const int cw = (bl[i].n + ST_PER - 1) / ST_PER;
     if (g < cw) {
       b = i;
       break;
@@ -621,67 +630,78 @@ __global__ void __launch_bounds__(256) k_ht_stebz(const HtBlock* __restrict__ bl
   }
   if (b < 0) return;
   const HtBlock B = bl[b];
-  const int n = B.n;
+  const int n = B.n, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
   const HtWs w = ht_ws(const_cast<double*>(Wa) + B.w_off, n, B.T);
-  double* d = lds;
-  double* e2 = lds + n;
-  __shared__ double rlo[256], rhi[256], rnm[256];
-  const int tid = threadIdx.x;
-  double lo = 1e300, hi = -1e300, nm = 0.0;
+  __shared__ double rlo[4], rhi[4];
+  double lo = 1e300, hi = -1e300;
   for (int i = tid; i < n; i += 256) {
-    const double di = w.d[i];
-    const double ei = i < n - 1 ? w.e[i] : 0.0, ep = i > 0 ? w.e[i - 1] : 0.0;
-    d[i] = di;
-    e2[i] = ei * ei;
-    const double rad = fabs(ei) + fabs(ep);
+    const double di = w.d[i], rad = (i < n - 1 ? fabs(w.e[i]) : 0.0) + (i > 0 ? fabs(w.e[i - 1]) : 0.0);
     lo = fmin(lo, di - rad);
     hi = fmax(hi, di + rad);
-    nm = fmax(nm, fabs(di) + rad);
   }
-  rlo[tid] = lo;
-  rhi[tid] = hi;
-  rnm[tid] = nm;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, o, 64));
+    hi = fmax(hi, __shfl_xor(hi, o, 64));
+  }
+  if (l == 0) {
+    rlo[wv] = lo;
+    rhi[wv] = hi;
+  }
   __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (tid < o) {
-      rlo[tid] = fmin(rlo[tid], rlo[tid + o]);
-      rhi[tid] = fmax(rhi[tid], rhi[tid + o]);
-      rnm[tid] = fmax(rnm[tid], rnm[tid + o]);
-    }
-    __syncthreads();
-  }
-  const double tnorm = rnm[0];
-  const double eps = 2.220446049250313e-16;
-  const double pivmin = 2.2250738585072014e-308 * fmax(1.0, tnorm * tnorm);
-  const double atol = 0.25 * eps * tnorm;
-  const int j = g * 256 + tid;
-  if (j >= n) return;
-  if (tnorm == 0.0) {  // T = 0: every eigenvalue is exactly zero
-    lam[B.e_off + j] = 0.0;
+  lo = fmin(fmin(rlo[0], rlo[1]), fmin(rlo[2], rlo[3]));
+  hi = fmax(fmax(rhi[0], rhi[1]), fmax(rhi[2], rhi[3]));
+  const double tn = fmax(fabs(lo), fabs(hi));
+  const int j = g * ST_PER + tid / ST_LANES, ln = tid & (ST_LANES - 1);
+  if (!(tn > 0.0 && tn <= 1.7976931348623157e308)) {  // T = 0: every eigenvalue is exactly zero
+    if (j < n && ln == 0) lam[B.e_off + j] = 0.0;
     return;
   }
-  double a = rlo[0] - 2.0 * eps * tnorm - pivmin, c = rhi[0] + 2.0 * eps * tnorm + pivmin;
-  for (int it = 0; it < 200; it++) {
-    const double mid = 0.5 * (a + c);
-    if (c - a <= 2.0 * eps * fmax(fabs(a), fabs(c)) + atol || mid <= a || mid >= c) break;
-    // Sturm count: eigenvalues below mid.  e_{i-1}^2 / q by the hardware reciprocal and one Newton
-    // step (|q| >= pivmin keeps it finite, and e^2 / pivmin below the overflow threshold), which
-    // shortens the dependent chain of each step to three fused operations
-    int cnt = 0;
-    double q = d[0] - mid;
-    if (fabs(q) < pivmin) q = -pivmin;
-    cnt += q < 0.0;
-    for (int i = 1; i < n; i++) {
-      double r = __builtin_amdgcn_rcp(q);
-      r = fma(r, fma(-q, r, 1.0), r);
-      q = fma(-e2[i - 1], r, d[i] - mid);
-      if (fabs(q) < pivmin) q = -pivmin;
-      cnt += q < 0.0;
-    }
-    if (cnt <= j) a = mid;
-    else c = mid;
+  const int ex = ilogb(tn) + 1;  // ||T|| in [1/2, 1) after scaling
+  const int nf = (n + ST_UNROLL - 1) / ST_UNROLL * ST_UNROLL;
+  for (int i = tid; i < nf; i += 256) {
+    const double e = i > 0 && i < n ? ldexp(w.e[i - 1], -ex) : 0.0;
+    de[i] = double2{i < n ? ldexp(w.d[i], -ex) : 4.0, e * e};  // (rows past the end: a 1 x 1 block above all)
   }
-  lam[B.e_off + j] = 0.5 * (a + c);
+  __syncthreads();
+  const double eps = 2.220446049250313e-16;
+  double a = ldexp(lo, -ex) - 4.0 * eps, c = ldexp(hi, -ex) + 4.0 * eps;
+  // a pivot p_i / p_{i-1} below this is moved to it from below (as the quotient form moves a vanishing one)
+  constexpr double PIV = 1e-32;
+  const bool mine = j < n;
+  const double tol = fmax(rtol, 0.5 * eps);
+  for (int it = 0; it < 64; it++) {
+    const bool go = mine && c - a > fmax(tol, 2.0 * eps * fmin(fabs(a), fabs(c)));
+    if (__ballot(go) == 0) break;
+    const double h = (c - a) * (1.0 / (ST_LANES + 1)), x = a + (ln + 1) * h;
+    int cnt = 0;
+    double p1 = 1.0, p2 = 0.0;
+    for (int i0 = 0; i0 < nf; i0 += ST_UNROLL) {
+      double2 t[ST_UNROLL];
+#pragma unroll
+      for (int i = 0; i < ST_UNROLL; i++) t[i] = de[i0 + i];
+#pragma unroll
+      for (int i = 0; i < ST_UNROLL; i++) {
+        double p = fma(t[i].x - x, p1, -t[i].y * p2);
+        p = fabs(p) < PIV * fabs(p1) ? -PIV * p1 : p;
+        cnt += (int)((unsigned)(__double2hiint(p) ^ __double2hiint(p1)) >> 31);
+        p2 = p1;
+        p1 = p;
+      }
+      const int sh = -__builtin_amdgcn_frexp_exp(fmax(fabs(p1), fabs(p2)));
+      p1 = __builtin_amdgcn_ldexp(p1, sh);
+      p2 = __builtin_amdgcn_ldexp(p2, sh);
+    }
+    // points at or below the eigenvalue: those with at most j eigenvalues below them
+    const unsigned long long in = __ballot(cnt <= j);
+    const int m = __popc((unsigned)(in >> (l & ~(ST_LANES - 1))) & ((1u << ST_LANES) - 1));
+    if (go) {
+      const double na = a + m * h;
+      c = m == ST_LANES ? c : a + (m + 1) * h;
+      a = na;
+    }
+  }
+  if (mine && ln == 0) lam[B.e_off + j] = ldexp(0.5 * (a + c), ex);
 }
 
 // deterministic start vector entries in [-1, 1)
@@ -1311,13 +1331,26 @@ int launch_ht_syr2k(const HtBlock* d_bl, const std::vector<HtBlock>& bl, int k, 
   NRGK_HIP(hipGetLastError());
   return g;
 }
-void launch_ht_stebz(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, hipStream_t s) {
-  int g = 0, nmax = 1;
+void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
+                     hipStream_t s) {
+  int nmax = 1;
+  long long total = 0;
   for (const auto& b : bl) {
-    g += (b.n + 255) / 256;
+    total += b.n;
     nmax = std::max(nmax, b.n);
   }
-  if (g) NRGK_LAUNCH(k_ht_stebz, dim3(g), dim3(256), (size_t)nmax * 2 * sizeof(double), s, d_bl, (int)bl.size(), W, lam);
+  if (!total) return;
+  const size_t lds = (size_t)(nmax + ST_UNROLL) * sizeof(double2);
+  auto grid = [&](int lanes) {
+    int g = 0;
+    for (const auto& b : bl) g += (b.n + 256 / lanes - 1) / (256 / lanes);
+    return g;
+  };
+  // (1 024 SIMDs; a wavefront holds 64 / lanes eigenvalues)
+  if (total * 8 <= 2 * 64 * 1024)
+    NRGK_LAUNCH(k_ht_sturm<8>, dim3(grid(8)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
+  else
+    NRGK_LAUNCH(k_ht_sturm<1>, dim3(grid(1)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
   NRGK_HIP(hipGetLastError());
 }
 void launch_ht_stein(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, const double* lam, double* U,
@@ -1369,13 +1402,15 @@ void launch_ht_larft(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const 
   if (g) NRGK_LAUNCH(k_ht_larft, dim3(g), dim3(256), 0, s, d_bl, (int)bl.size(), V, W, A);
   NRGK_HIP(hipGetLastError());
 }
-// dynamic LDS of the bisection and inverse-iteration kernels (d and e^2, or d and e, of the widest
+// dynamic LDS of the multisection and inverse-iteration kernels (d and e^2, or d and e, of the widest
 // block); their static LDS (below 8 KB) comes on top of it
 constexpr int HT_STATIC_LDS = 8192;
 int ht_max_n(int lds_bytes) { return (lds_bytes - HT_STATIC_LDS) / (int)(2 * sizeof(double)); }
 void set_ht_lds_limits(int bytes) {
   const int dyn = bytes - HT_STATIC_LDS;
-  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_stebz, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
+  const int dyn_st = dyn + ST_UNROLL * (int)sizeof(double2);
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm<8>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn_st));
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm<1>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn_st));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_stein_step, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
 }
 

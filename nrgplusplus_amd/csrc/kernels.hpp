@@ -33,10 +33,7 @@ void launch_mid_reduce(const MidBlock* d_bl, const std::vector<MidBlock>& bl, co
                        float* tau, double* W, hipStream_t s);
 void launch_mid_back(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const float* V, const float* tau, float* VT,
                      double* X, hipStream_t s);
-// eigenvalues of T to rtol ||T||
-void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
-                     hipStream_t s);
-void set_mid_lds_limits(int bytes);
+void set_mid_lds_limit();
 // k_gemm.hip
 int prepare_gemm(std::vector<GemmProb>& probs);
 void launch_gemm(const GemmProb* d_probs, int n_probs, int tiles, hipStream_t s);
@@ -51,7 +48,9 @@ int launch_ht_update(const HtBlock* d_bl, const std::vector<HtBlock>& bl, int k,
                      hipStream_t s);
 int launch_ht_syr2k(const HtBlock* d_bl, const std::vector<HtBlock>& bl, int k, double* A, const double* V, double* W,
                     hipStream_t s);
-void launch_ht_stebz(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, hipStream_t s);
+// eigenvalues of T to rtol ||T|| (0: to rounding)
+void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, double* lam, double rtol,
+                     hipStream_t s);
 // list: 3 ints per cluster of more than one member (at most the wanted columns), count: one int
 void launch_ht_stein(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, const double* lam, double* U,
                      double* S, double ctol_rel, int* list, int* count, hipStream_t s);

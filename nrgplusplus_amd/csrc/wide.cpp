@@ -156,7 +156,7 @@ void Chain::wide_begin(const std::vector<int>& sectors) {
       hipEvent_t g0 = nullptr, g1 = nullptr;
       const bool fe = want("tridiag_eigenvalues");
       if (fe) mark(g0);
-      launch_ht_stebz(d, ht, W, dlam_raw.as<double>(), s2);
+      launch_ht_sturm(d, ht, W, dlam_raw.as<double>(), 0.0, s2);
       if (fe) {
         mark(g1);
         wide_prof.push_back(ProfRun{"tridiag_eigenvalues", g0, g1, 1, 0.0, 0.0});
