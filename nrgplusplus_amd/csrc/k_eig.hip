@@ -93,13 +93,14 @@ __device__ void rr_jacobi(double* Wm, int k, double* mu, int* perm, double* nrm)
     if (lane == 0) nrm[c] = sqrt(s);
   }
   __syncthreads();
-  // ascending order of the norms by rank (ties by column index)
+  // ascending order of the norms by rank (ties by column index; sort_key: every rank is taken once, so that
+  // perm is a permutation, also where norms are NaN)
   for (int c = threadIdx.x; c < k; c += blockDim.x) {
-    const double v = nrm[c];
+    const double v = nrm[c], kv = sort_key(v);
     int r = 0;
     for (int c2 = 0; c2 < k; c2++) {
-      const double u = nrm[c2];
-      r += (u < v) || (u == v && c2 < c);
+      const double u = sort_key(nrm[c2]);
+      r += (u < kv) || (u == kv && c2 < c);
     }
     perm[r] = c;
     mu[r] = v;

@@ -55,6 +55,18 @@ __device__ __forceinline__ dbl4 sm_tile(const double* A, const double* B, int ld
   return acc;
 }
 
+// rank of v[i] among v[0 .. n-1], ascending, ties by index, NaN last: every rank is taken once
+__device__ __forceinline__ int sm_rank(const double* v, int n, int i) {
+  auto key = [](double x) { return x < 1e308 ? x : 1e308; };
+  const double k = key(v[i]);
+  int rank = 0;
+  for (int c = 0; c < n; c++) {
+    const double u = key(v[c]);
+    rank += u < k || (u == k && c < i);
+  }
+  return rank;
+}
+
 // status[b] (zero before) is 1 if block b did not converge; sweeps: the most of any block.
 __global__ void __launch_bounds__(SM_THREADS) k_eig_small(const EigBlock* __restrict__ blocks,
                                                           const double* __restrict__ Ha, double* __restrict__ Ua,
@@ -199,12 +211,7 @@ __global__ void __launch_bounds__(SM_THREADS) k_eig_small(const EigBlock* __rest
     if (l == 0) ev[c] = s;
   }
   __syncthreads();
-  if (tid < n) {
-    const double v = ev[tid];
-    int rank = 0;
-    for (int c = 0; c < n; c++) rank += ev[c] < v || (ev[c] == v && c < tid);
-    perm[rank] = tid;
-  }
+  if (tid < n) perm[sm_rank(ev, n, tid)] = tid;
   __syncthreads();
   for (int e = tid; e < n * n; e += SM_THREADS) {
     const int c = e / n, r = e - c * n, p = perm[c];
@@ -265,11 +272,9 @@ __global__ void __launch_bounds__(SM_THREADS) k_eig_small(const EigBlock* __rest
   }
   // eigenvalues ascending (the refinement may exchange neighbours by an ulp)
   if (tid < n) {
-    const double v = lt[tid];
-    int rank = 0;
-    for (int c = 0; c < n; c++) rank += lt[c] < v || (lt[c] == v && c < tid);
+    const int rank = sm_rank(lt, n, tid);
     perm[tid] = rank;
-    lam[blk.e_off + rank] = ldexp(v, ex);
+    lam[blk.e_off + rank] = ldexp(lt[tid], ex);
   }
   __syncthreads();
   double* U = Ua + blk.off;

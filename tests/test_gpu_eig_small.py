@@ -68,3 +68,16 @@ def test_non_finite_block_gives_nan(nk):
     assert np.isnan(w).all()
     np.testing.assert_allclose(w0, np.ones(5), atol=1e-15)
     np.testing.assert_allclose(U0 @ U0.T, np.eye(5), atol=1e-15)
+
+
+def test_nan_block(nk):
+    """a NaN entry: every eigenvalue of that block is NaN, as the wider blocks' are, and the others' stand"""
+    rng = np.random.default_rng(4)
+    lams = [np.sort(rng.uniform(-1, 1, n)) for n in (64, 20, 33)]
+    blocks = [_block(rng, lam) for lam in lams]
+    nk.eigh_batched(blocks)
+    blocks[1][3, 5] = blocks[1][5, 3] = np.nan
+    out = nk.eigh_batched(blocks)
+    assert np.isnan(out[1][0]).all()
+    for i in (0, 2):
+        _check(blocks[i], lams[i], *out[i], 1.0)
