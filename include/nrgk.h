@@ -116,7 +116,9 @@ const char* nrgk_version(void);
 /* opens HIP device `device`; no reference counterpart (the reference has no device) */
 int nrgk_ctx_create(int device, nrgk_ctx** out);
 int nrgk_ctx_destroy(nrgk_ctx* ctx);
-/* bytes of device memory the context may hand to chains (0 = 90% of the free HBM) */
+/* bytes of device memory the context may hand to chains (0 = 90% of the free HBM).  Memory of chains that
+ * are gone is kept for the next ones, up to 1/32 of the capacity and not counted as used; it is freed by this
+ * call, with the context, and where an allocation needs the room */
 int nrgk_ctx_set_capacity(nrgk_ctx* ctx, size_t bytes);
 int nrgk_ctx_used_bytes(nrgk_ctx* ctx, size_t* used, size_t* capacity);
 

@@ -76,7 +76,7 @@ int nrgk_ctx_create(int device, nrgk_ctx** out) {
     tune_load(h->c);
     size_t fr = 0, tot = 0;
     NRGK_HIP(hipMemGetInfo(&fr, &tot));
-    h->c.capacity = (size_t)(0.9 * (double)fr);
+    h->c.set_capacity((size_t)(0.9 * (double)fr));
     *out = h;
   });
 }
@@ -108,12 +108,13 @@ int nrgk_ctx_destroy(nrgk_ctx* ctx) {
 int nrgk_ctx_set_capacity(nrgk_ctx* ctx, size_t bytes) {
   return guard([&] {
     NRGK_REQUIRE(ctx, NRGK_ERR_INVALID, "null context");
+    ctx->c.pool.trim();
     if (bytes == 0) {
       size_t fr = 0, tot = 0;
       NRGK_HIP(hipMemGetInfo(&fr, &tot));
       bytes = (size_t)(0.9 * (double)fr) + ctx->c.used;
     }
-    ctx->c.capacity = bytes;
+    ctx->c.set_capacity(bytes);
   });
 }
 int nrgk_ctx_used_bytes(nrgk_ctx* ctx, size_t* used, size_t* capacity) {

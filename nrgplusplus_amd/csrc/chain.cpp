@@ -23,23 +23,47 @@ ThreadCounts& thread_counts() {
 void DevBuf::ensure(size_t bytes) {
   if (bytes <= cap) return;
   release();
-  size_t want = bytes + bytes / 4 + 256;
+  const size_t want = bytes + bytes / 4 + 256;
+  size = retired ? MemPool::size_class(want) : want;
   if (ctx) ctx->charge(want);
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess) {
-    if (ctx) ctx->refund(want);
-    p = nullptr;
-    throw Error(NRGK_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(want) + "): " + hipGetErrorString(e));
+  if (ctx && retired) p = ctx->pool.take(size);
+  if (!p) {
+    if (ctx && ctx->capacity && ctx->used + ctx->pool.held() > ctx->capacity) ctx->pool.trim();
+    hipError_t e = hipMalloc(&p, size);
+    if (e != hipSuccess && ctx) {
+      // the device waits, as hipFree made it, and everything idle is freed
+      if (retired && hipDeviceSynchronize() == hipSuccess) retired->give_all();
+      ctx->pool.trim();
+      size = want;
+      e = hipMalloc(&p, size);
+    }
+    if (e != hipSuccess) {
+      if (ctx) ctx->refund(want);
+      p = nullptr;
+      throw Error(NRGK_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(want) + "): " + hipGetErrorString(e));
+    }
   }
   cap = want;
 }
 void DevBuf::release() {
   if (p) {
-    (void)hipFree(p);
+    if (retired) retired->add(p, size);
+    else (void)hipFree(p);
     if (ctx) ctx->refund(cap);
   }
   p = nullptr;
   cap = 0;
+}
+void Retired::give_all() {
+  std::vector<std::pair<void*, size_t>> b;
+  {
+    std::lock_guard<std::mutex> lk(m);
+    b.swap(bufs);
+  }
+  for (auto& [p, size] : b) {
+    if (ctx) ctx->pool.give(p, size);
+    else (void)hipFree(p);
+  }
 }
 
 template <class T>
@@ -101,10 +125,16 @@ void Chain::init_device() {
                     &dY, &dC, &dlam_tmp, &dlam_raw, &dlam_prev, &dlam_shift[0], &dlam_shift[1], &d_eig, &d_stats, &d_kept,
                     &d_trunc, &d_eig_act, &d_rrv, &d_cid, &d_sidx, &d_mid_A, &d_mid_tau, &d_mid_ws, &d_mid_q, &d_ht,
                     &d_wide_ws, &d_wide_s, &d_wide_q, &d_wide_A, &d_wide_V})
-    b->ctx = ctx;
+    b->ctx = ctx, b->retired = &retired;
+  for (DevBuf& b : d_big_work) b.ctx = ctx, b.retired = &retired;
+  d_big_info.ctx = ctx, d_big_info.retired = &retired;
   stg.ctx = ctx;
   NRGK_HIP(hipSetDevice(ctx->device));
-  NRGK_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+  hold = std::make_shared<StreamHold>();
+  NRGK_HIP(hipStreamCreateWithFlags(&hold->st, hipStreamNonBlocking));
+  st = hold->st;
+  retired.ctx = ctx;
+  retired.st = st;
   for (auto& e : ev) NRGK_HIP(hipEventCreate(&e));
 }
 
@@ -163,6 +193,15 @@ void Chain::sync() {
   NRGK_HIP(stream_sync(st));
   stg.reset();
   prof_resolve();
+  reclaim();
+}
+
+void Chain::reclaim() {
+  // not under the worker, which is enqueueing on a side stream
+  if (retired.empty() || wide_thread.joinable()) return;
+  for (hipStream_t s : st_big)
+    if (s) NRGK_HIP(hipStreamSynchronize(s));
+  retired.give_all();
 }
 
 hipEvent_t Chain::take_event() {
@@ -214,7 +253,6 @@ Chain::~Chain() {
   }
   if (prof_open) ev_pool.push_back(prof_open);
   for (auto& e : ev_pool) (void)hipEventDestroy(e);
-  if (st) (void)hipStreamDestroy(st);
 }
 
 void Chain::set_bath(const nrgk_site_desc* b) {

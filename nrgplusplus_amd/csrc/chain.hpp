@@ -82,9 +82,21 @@ struct SiteData {
 
 struct Obs;
 
+// A chain's stream, kept by the chain and by its observables and recorders: whichever goes last drains it.
+struct StreamHold {
+  hipStream_t st = nullptr;
+  ~StreamHold() {
+    if (!st) return;
+    (void)hipStreamSynchronize(st);
+    (void)hipStreamDestroy(st);
+  }
+};
+
 struct Chain {
   Ctx* ctx = nullptr;
-  hipStream_t st = nullptr;
+  std::shared_ptr<StreamHold> hold;
+  hipStream_t st = nullptr;  // hold->st
+  Retired retired;           // before the buffers: their memory outlives them until the streams have drained
   SiteData imp, bath;
   size_t K = 1024;
   int mode = NRGK_MODE_MIXED;
@@ -196,6 +208,8 @@ struct Chain {
   // drains the stream and recycles it
   Staging stg;
   void sync();
+  // outgrown buffers back to the context's pool; the chain's stream has drained
+  void reclaim();
   // host data to a persistent device buffer, without blocking the host (staged, then copied)
   template <class T>
   T* upload_to(DevBuf& buf, const T* src, size_t n, size_t byte_off = 0) {

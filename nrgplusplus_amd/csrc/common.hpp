@@ -8,7 +8,11 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
+#include <tuple>
+#include <utility>
 #include <vector>
 
 #include "../../include/nrgk.h"
@@ -57,18 +61,137 @@ inline hipError_t stream_sync(hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ device buffers
-// A device allocation that only grows; per-iteration scratch reuses it without hipMalloc in the
-// steady state.  Every allocation is charged to the owning context's capacity (HBM admission).
 struct Ctx;
+
+// Idle device and page-locked memory of a context, for its next chains.  A chain's buffers come and go with
+// it (one request of the server, one eigh call, one of the chains of a z-average), and hipMalloc, hipFree and
+// hipHostMalloc each wait for the whole device: 16 chains at K = 512 spent 25 ms growing their buffers in the
+// first sites and 54 ms giving them back, of 187 ms.  Memory is given here only when no stream uses it any
+// more.  Bounded: beyond `limit` bytes memory is freed; what is held is freed when an allocation
+// fails or would take the context past its capacity, when the capacity is set, and with the context.
+class MemPool {
+ public:
+  size_t limit = 0;         // device bytes held at most
+  size_t host_limit = 256u << 20;  // page-locked bytes held at most (staging: as many device bytes)
+  MemPool() = default;
+  MemPool(const MemPool&) = delete;
+  MemPool& operator=(const MemPool&) = delete;
+  ~MemPool() { trim(); }
+  // Size of the allocation behind a request: eight classes to the octave, so that chains whose sectors differ
+  // a little fit each other's buffers; at most an eighth more than was asked for.
+  static size_t size_class(size_t bytes) {
+    size_t step = 4096;
+    while (step * 16 < bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+  }
+  void* take(size_t size) {
+    std::lock_guard<std::mutex> lk(m_);
+    auto it = dev_.find(size);
+    if (it == dev_.end()) return nullptr;
+    void* p = it->second;
+    dev_.erase(it);
+    held_ -= size;
+    return p;
+  }
+  void give(void* p, size_t size) {
+    {
+      std::lock_guard<std::mutex> lk(m_);
+      if (held_ + size <= limit) {
+        dev_.emplace(size, p);
+        held_ += size;
+        return;
+      }
+    }
+    (void)hipFree(p);
+  }
+  std::pair<char*, char*> take_staging(size_t size) {
+    std::lock_guard<std::mutex> lk(m_);
+    auto it = staging_.find(size);
+    if (it == staging_.end()) return {nullptr, nullptr};
+    auto p = it->second;
+    staging_.erase(it);
+    held_ -= size;
+    host_held_ -= size;
+    return p;
+  }
+  void give_staging(char* host, char* dev, size_t size) {
+    {
+      std::lock_guard<std::mutex> lk(m_);
+      if (held_ + size <= limit && host_held_ + size <= host_limit) {
+        staging_.emplace(size, std::make_pair(host, dev));
+        held_ += size;
+        host_held_ += size;
+        return;
+      }
+    }
+    (void)hipHostFree(host);
+    (void)hipFree(dev);
+  }
+  size_t held() const { return held_; }
+  void trim() {
+    std::multimap<size_t, void*> d;
+    std::multimap<size_t, std::pair<char*, char*>> s;
+    {
+      std::lock_guard<std::mutex> lk(m_);
+      d.swap(dev_);
+      s.swap(staging_);
+      held_ = 0;
+      host_held_ = 0;
+    }
+    for (auto& e : d) (void)hipFree(e.second);
+    for (auto& e : s) {
+      (void)hipHostFree(e.second.first);
+      (void)hipFree(e.second.second);
+    }
+  }
+
+ private:
+  std::mutex m_;
+  std::multimap<size_t, void*> dev_;
+  std::multimap<size_t, std::pair<char*, char*>> staging_;
+  std::atomic<size_t> held_{0}, host_held_{0};
+};
+
+// Buffers that their owner has let go of while its stream may still use them: given to the context's pool
+// when the owner, having drained its streams, says so, or with the owner.
+struct Retired {
+  Ctx* ctx = nullptr;
+  hipStream_t st = nullptr;
+  std::mutex m;
+  std::vector<std::pair<void*, size_t>> bufs;
+  Retired() = default;
+  Retired(const Retired&) = delete;
+  Retired& operator=(const Retired&) = delete;
+  ~Retired() {
+    if (!bufs.empty() && st) (void)hipStreamSynchronize(st);
+    give_all();
+  }
+  void add(void* p, size_t size) {
+    std::lock_guard<std::mutex> lk(m);
+    bufs.emplace_back(p, size);
+  }
+  bool empty() {
+    std::lock_guard<std::mutex> lk(m);
+    return bufs.empty();
+  }
+  void give_all();
+};
+
+// A device allocation that only grows; per-iteration scratch reuses it without hipMalloc in the
+// steady state.  Every allocation is charged to the owning context's capacity (HBM admission).  With an
+// owner's Retired list it comes from and goes back to the context's pool; without one (temporaries) it is
+// allocated and freed directly.
 struct DevBuf {
   void* p = nullptr;
   size_t cap = 0;
+  size_t size = 0;  // of the allocation (cap, rounded up to the pool's size class)
   Ctx* ctx = nullptr;
+  Retired* retired = nullptr;
   DevBuf() = default;
-  explicit DevBuf(Ctx* c) : ctx(c) {}
+  explicit DevBuf(Ctx* c, Retired* r = nullptr) : ctx(c), retired(r) {}
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), cap(o.cap), ctx(o.ctx) {
+  DevBuf(DevBuf&& o) noexcept : p(o.p), cap(o.cap), size(o.size), ctx(o.ctx), retired(o.retired) {
     o.p = nullptr;
     o.cap = 0;
   }
@@ -77,7 +200,9 @@ struct DevBuf {
       release();
       p = o.p;
       cap = o.cap;
+      size = o.size;
       ctx = o.ctx;
+      retired = o.retired;
       o.p = nullptr;
       o.cap = 0;
     }
@@ -96,6 +221,7 @@ struct Ctx {
   int device = 0;
   size_t capacity = 0;
   std::atomic<size_t> used{0};  // chains of one context may be stepped from several host threads
+  MemPool pool;                 // idle memory, beside `used`
   int lds_max = 65536;  // bytes of LDS one workgroup may allocate
   int n_cu = 0;
   std::string arch;     // gcnArchName of the device
@@ -103,6 +229,10 @@ struct Ctx {
   // path (768, MD_MAX, unless the autotuner's cache says otherwise)
   int mixed_max = 768;
   bool tuned = false;
+  void set_capacity(size_t bytes) {
+    capacity = bytes;
+    pool.limit = bytes / 32;  // 8 GiB of a whole device
+  }
   void charge(size_t bytes) {
     size_t u = used.load();
     do {
@@ -136,29 +266,47 @@ struct Staging {
   Staging(const Staging&) = delete;
   Staging& operator=(const Staging&) = delete;
   ~Staging() { release(); }
+  // the owner has drained the streams that use it
   void release() {
     for (auto& c : chunks) {
-      if (c.host) (void)hipHostFree(c.host);
-      if (c.dev) {
+      if (ctx) {
+        ctx->pool.give_staging(c.host, c.dev, c.cap);
+        ctx->refund(c.cap);
+      } else {
+        (void)hipHostFree(c.host);
         (void)hipFree(c.dev);
-        if (ctx) ctx->refund(c.cap);
       }
     }
     chunks.clear();
   }
-  void add_chunk(size_t cap) {
+  void add_chunk(size_t bytes) {
     Chunk c;
-    c.cap = cap;
-    if (ctx) ctx->charge(cap);
-    hipError_t e = hipHostMalloc((void**)&c.host, cap, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMalloc((void**)&c.dev, cap);
-    if (e != hipSuccess) {
-      if (c.host) (void)hipHostFree(c.host);
-      if (ctx) ctx->refund(cap);
-      throw Error(NRGK_ERR_NOMEM, std::string("nrgk: staging allocation (") + std::to_string(cap) + "): " +
-                                      hipGetErrorString(e));
+    c.cap = MemPool::size_class(bytes);
+    if (ctx) ctx->charge(c.cap);
+    if (ctx) std::tie(c.host, c.dev) = ctx->pool.take_staging(c.cap);
+    if (!c.host) {
+      if (ctx && ctx->capacity && ctx->used + ctx->pool.held() > ctx->capacity) ctx->pool.trim();
+      hipError_t e = allocate(c);
+      if (e != hipSuccess && ctx) {
+        ctx->pool.trim();
+        e = allocate(c);
+      }
+      if (e != hipSuccess) {
+        if (ctx) ctx->refund(c.cap);
+        throw Error(NRGK_ERR_NOMEM, std::string("nrgk: staging allocation (") + std::to_string(c.cap) + "): " +
+                                        hipGetErrorString(e));
+      }
     }
     chunks.push_back(c);
+  }
+  static hipError_t allocate(Chunk& c) {
+    hipError_t e = hipHostMalloc((void**)&c.host, c.cap, hipHostMallocDefault);
+    if (e == hipSuccess) {
+      e = hipMalloc((void**)&c.dev, c.cap);
+      if (e != hipSuccess) (void)hipHostFree(c.host);
+    }
+    if (e != hipSuccess) c.host = c.dev = nullptr;
+    return e;
   }
   // an aligned region of `bytes`: (host, device) addresses
   std::pair<char*, char*> take(size_t bytes) {

@@ -19,7 +19,10 @@
 namespace nrgk {
 
 Obs::Obs(Chain* c, int n_ops, const int* nblocks, const int* bi, const int* bj, const double* data) : ch(c), nops(n_ops) {
-  for (DevBuf* b : {&buf[0], &buf[1], &dseg, &dC, &dY}) b->ctx = ch->ctx;
+  hold = ch->hold;
+  retired.ctx = ch->ctx;
+  retired.st = ch->st;
+  for (DevBuf* b : {&buf[0], &buf[1], &dseg, &dC, &dY}) b->ctx = ch->ctx, b->retired = &retired;
   NRGK_REQUIRE(ch->phase == Chain::FRESH, NRGK_ERR_STATE, "nrgk: observables are created before the first site");
   ch->need_full_u = true;  // the rotation reads every column of U
   blocks.assign(nops, OpMap());
@@ -122,6 +125,7 @@ void Obs::update() {
   c.run_gemms(g1);
   c.run_gemms(g2);
   c.sync();
+  retired.give_all();
   blocks = std::move(nbk);
   cur = nbuf;
 }
@@ -130,14 +134,17 @@ void Obs::update() {
 Fdm::Fdm(Chain* c, Obs* o, int nb, double emin, double emax) : ch(c), obs(o), nbins(nb), e_min(emin), e_max(emax) {
   NRGK_REQUIRE(nb > 0 && emin > 0 && emax > emin, NRGK_ERR_INVALID, "nrgk: bad FDM binning");
   delE = (nbins - 1.0) / std::log(e_max / e_min);  // fdmSpectrum.hpp:351-354
+  hold = ch->hold;
+  retired.ctx = ch->ctx;
+  retired.st = ch->st;
   for (DevBuf* b : {&dpos, &dneg, &dsum, &dbf, &dred[0], &dred[1], &dRA, &dAR, &dT1, &drho, &ditems, &dpt, &dE, &dth, &dQ})
-    b->ctx = ch->ctx;
+    b->ctx = ch->ctx, b->retired = &retired;
 }
 
 void* Fdm::arena_alloc(size_t bytes) {
   bytes = (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
   if (chunks.empty() || chunk_used + bytes > chunks.back()->cap) {
-    auto b = std::make_unique<DevBuf>(ch->ctx);
+    auto b = std::make_unique<DevBuf>(ch->ctx, &retired);
     b->ensure(std::max<size_t>(bytes, size_t(512) << 20));
     chunks.push_back(std::move(b));
     chunk_used = 0;
@@ -612,6 +619,7 @@ void Fdm::backward_shells(const std::vector<std::pair<Shell*, double>>& list, do
   signed_tot.assign(nops, 0.0);
   d2h(signed_tot.data(), dsum.as<double>() + 1, nops, st);
   NRGK_HIP(stream_sync(st));
+  retired.give_all();
   if (n_shells) *n_shells = ns;
 }
 

@@ -10,6 +10,8 @@ namespace nrgk {
 // System operators rotated along the chain (update_system_operator, sysOperator.hpp:35-133).
 struct Obs {
   Chain* ch = nullptr;
+  std::shared_ptr<StreamHold> hold;  // of the chain's stream
+  Retired retired;
   int nops = 0;
   std::vector<OpMap> blocks;  // full n_i x n_j blocks in the current basis
   DevBuf buf[2];
@@ -47,6 +49,8 @@ struct Shell {
 
 struct Fdm {
   Chain* ch = nullptr;
+  std::shared_ptr<StreamHold> hold;  // of the chain's stream
+  Retired retired;
   Obs* obs = nullptr;
   Obs* sysop = nullptr;  // fdmThermodynamics::setSystemOperator
   int nbins = 0;

@@ -111,9 +111,7 @@ void large_blocks_begin(Chain& c, const std::vector<int>& sectors) {
       NRGK_REQUIRE(rocblas_create_handle(&h) == rocblas_status_success, NRGK_ERR_HIP, "rocblas_create_handle failed");
       rocblas_set_stream(h, c.st_big[k]);
       c.rocblas_big[k] = h;
-      c.d_big_work[k].ctx = c.ctx;
     }
-  c.d_big_info.ctx = c.ctx;
   std::vector<int> order(sectors);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return c.cur_n[x] > c.cur_n[y]; });
   double load[Chain::N_SIDE] = {0};
