@@ -9,10 +9,11 @@
 //   k_mid_back    X = Q Z, a workgroup per 64 columns, every panel in one launch
 //
 // The whole sequence takes a dozen launches whatever the block widths; the one-sided block Jacobi it
-// replaces took n/16 dependent launches per sweep and nine sweeps for the widest blocks (n = 330, a SIAM step
-// at K = 1024: 2.7 -> 1.7 ms; n = 190, K = 500: 1.3 -> 0.75 ms; n = 619, K = 2048: 6.8 -> 5.0 ms).
+// replaces took n/16 dependent launches per sweep and nine sweeps for the widest blocks.
 #include "common.hpp"
 #include "kernels.hpp"
+
+#include <type_traits>
 
 namespace nrgk {
 
@@ -37,8 +38,8 @@ long long md_matrix_floats(int n) { return 1024LL * md_strip(md_strips(n)); }
 __host__ __device__ __forceinline__ int md_np(int n) { return (n + 63) & ~63; }
 // row stride of the staged panel columns: the four 16-lane groups of a matrix-core operand 16 banks apart
 __host__ __device__ __forceinline__ int md_ld(int n) { return md_np(n) + 16; }
-// the widest trailing matrix held in registers: 20 strips of up to 5 tiles, three strips to a wave
-constexpr int MD_REG = 320;
+// the widest trailing matrix held in registers, in tiles of 64 rows and in rows
+constexpr int MD_T = 6, MD_REG = 64 * MD_T;
 
 template <int CTRL>
 __device__ __forceinline__ float md_dpp(float v) {
@@ -374,228 +375,270 @@ __device__ __forceinline__ void md_columns(float* A, const MdLds& m, int n, int 
   }
 }
 
-// The rest of the reduction, columns 0 .. n-1 of an n x n matrix (n <= MD_REG), with the matrix in
-// registers and updated after every column.  Wave w holds the strips S-1-w, S-16+w and S-17-w: NT tiles of
-// each, lane (lk, li) rows 4 lk .. + 3 and columns 4 li .. + 3 of a tile.  The 16 x 16 piece on a strip's
-// diagonal is held in full and counts for its rows only; lanes right of it hold nothing that is read.
-// Three barriers per column: the column (in cb), the products' partial sums, v and w.
+// The rest of the reduction, columns 0 .. n-1 of an n x n matrix (n <= MD_REG), with the matrix in registers
+// and updated after every column.  Its last row is the last of T tiles of 64 rows (rows of zeros before the
+// first one), so that a phase of 64 columns has the pivot row in the first of the tiles left and everything
+// but that row's place in it is known to the compiler.  Of the S = 4 T strips of 16 rows left, wave w holds
+// the strips S-1-w, S-16+w and S-17-w: register 4 b + i of lane (lk, li) of a tile is row 4 lk + i, column
+// 16 b + li of it (the layout of the matrix cores' 16 x 16 results).  The 16 x 16 piece on a strip's diagonal
+// is held in full and counts for its rows only; nothing right of it is read.
+// Two barriers per column: w of the pivot row, which all the next column's entries wait for, is formed by
+// every wave for itself, and the rank-two update of the tiles (matrix cores) runs under the next reflector.
 struct MdReg {
-  float cb[MD_REG], vb[MD_REG], wb[MD_REG], ysum[MD_REG], cpart[MD_WAVES][MD_REG], ap[16];
+  float cb[MD_REG], vb[MD_REG], wb[MD_REG], ysum[MD_REG], an[MD_REG], cpart[MD_WAVES][MD_REG], ap[16];
+  float d[MD_REG], e[MD_REG], tau[MD_REG];  // by row, the results
 };
+typedef float flt16 __attribute__((ext_vector_type(16)));
+
+// A strip's first NT tiles (the last of them holds its diagonal); NT <= 0: no strip
 template <int NT>
 struct MdStrip {
-  flt4 a[NT][4];
-  flt4 x, y;  // the strip's rows of u and the row sums; of v and w
-  int st;     // < 0: none
-
-  // from the tiles in memory (lower triangle, diagonal halved, rows from r0 = b0 on)
-  __device__ __forceinline__ void load(const float* A, int b0, int strip, int li, int lk) {
-    st = strip;
+  static constexpr bool any = NT > 0;
+  flt4 x, y;  // the strip's rows of u and the row sums
+  // u's rows (first tile: zero above row s, u0 at s)
+  __device__ __forceinline__ void begin(const float* cb, int st, int s, float u0, int lk) {
+    if constexpr (any) {
+      const int r4 = 16 * st + 4 * lk;
+      x = *reinterpret_cast<const flt4*>(cb + r4);
+      if constexpr (NT == 1)
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
+        for (int i = 0; i < 4; i++) x[i] = r4 + i < s ? 0.0f : r4 + i == s ? u0 : x[i];
+      y = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  }
+  // tile t: row sums with the columns' u (uc), column sums added to ca; q: the diagonal's piece of its tile
+  template <int t>
+  __device__ __forceinline__ void product(const flt16& a, const flt4& uc, flt4& ca, int q) {
+    if constexpr (t < NT) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        a[t][i] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (st < 0 || t > st >> 2) continue;
-        const int r = 16 * st + 4 * lk + i, c = 64 * t + 4 * li;
-        if (c >> 4 < st) {
-          a[t][i] = *reinterpret_cast<const flt4*>(A + 1024 * (md_strip((b0 + r) >> 4) + ((b0 + c) >> 6)) +
-                                                   (r & 15) * 64 + (c & 63));
-        } else if (c >> 4 == st) {
+      for (int b = 0; b < 4; b++) {
+        float c = 0.0f, ub = uc[b];
+        if constexpr (t == NT - 1) ub = b <= q ? ub : 0.0f;
 #pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const int hi = max(r, c + j), lo = min(r, c + j);
-            const float z = A[1024 * (md_strip((b0 + hi) >> 4) + ((b0 + lo) >> 6)) + (hi & 15) * 64 + (lo & 63)];
-            a[t][i][j] = hi == lo ? 2.0f * z : z;
-          }
+        for (int i = 0; i < 4; i++) {
+          c += a[4 * b + i] * x[i];
+          y[i] += a[4 * b + i] * ub;
         }
-      }
-      __builtin_amdgcn_sched_barrier(0);  // a tile at a time: the next ones' loads would cost registers
-    }
-  }
-  // the last tile while row s or a later one is in the strip (the tiles before s's are skipped by the caller)
-  __device__ __forceinline__ int last(int s) const { return st >= s >> 4 ? st >> 2 : -1; }
-  // u's rows of the strip (zero above s, u0 at s), no row sums yet
-  __device__ __forceinline__ void begin(const MdReg& m, int s, float u0, int lk) {
-    if (st < s >> 4) return;
-    const int r4 = 16 * st + 4 * lk;
-    x = *reinterpret_cast<const flt4*>(m.cb + r4);
-    if (st == s >> 4)
-#pragma unroll
-      for (int i = 0; i < 4; i++) x[i] = r4 + i < s ? 0.0f : r4 + i == s ? u0 : x[i];
-    y = flt4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  // tile t: row sums with the columns' u (uc), column sums added to ca
-  __device__ __forceinline__ void product(int t, const flt4& uc, flt4& ca, int li) {
-    flt4 ur = x, uy = uc;
-    if (t == st >> 2) {
-      const int d = (li >> 2) - (st & 3);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        ur[i] = d >= 0 ? 0.0f : ur[i];
-        uy[i] = d > 0 ? 0.0f : uy[i];
+        if constexpr (t == NT - 1) c = b < q ? c : 0.0f;
+        ca[b] += c;
       }
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        ca[j] += a[t][i][j] * ur[i];
-        y[i] += a[t][i][j] * uy[j];
-      }
   }
   // the row sums into ysum; this lane's share of u^T A u from them
-  __device__ __forceinline__ float end(MdReg& m, int s, int li, int lk) const {
-    if (st < s >> 4) return 0.0f;
-    const float rs = md_rows(y, li);
-    if (li < 4) m.ysum[16 * st + 4 * lk + md_row(li)] = rs;
-    return (y[0] * x[0] + y[1] * x[1]) + (y[2] * x[2] + y[3] * x[3]);
+  __device__ __forceinline__ float end(float* ysum, int st, int li, int lk) const {
+    if constexpr (any) {
+      const float rs = md_rows(y, li);
+      if (li < 4) ysum[16 * st + 4 * lk + md_row(li)] = rs;
+      return (y[0] * x[0] + y[1] * x[1]) + (y[2] * x[2] + y[3] * x[3]);
+    }
+    return 0.0f;
   }
-  __device__ __forceinline__ void rows_vw(const MdReg& m, int s, int lk) {
-    if (st < s >> 4) return;
-    x = *reinterpret_cast<const flt4*>(m.vb + 16 * st + 4 * lk);
-    y = *reinterpret_cast<const flt4*>(m.wb + 16 * st + 4 * lk);
-  }
-  __device__ __forceinline__ void update(int t, const flt4& vc, const flt4& wc) {
+  // column c of the first tile
+  static __device__ __forceinline__ void column(float* dst, const flt16& a, int st, int c, int li, int lk) {
+    if constexpr (any) {
+      flt4 z;
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) a[t][i][j] -= x[i] * wc[j] + y[i] * vc[j];
-  }
-  // column c of tile t into cb
-  __device__ __forceinline__ void column(MdReg& m, int t, int c, int li, int lk) const {
-    flt4 z;
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-      z[i] = (c & 2) ? ((c & 1) ? a[t][i][3] : a[t][i][2]) : ((c & 1) ? a[t][i][1] : a[t][i][0]);
-    if (li == (c & 63) >> 2) *reinterpret_cast<flt4*>(m.cb + 16 * st + 4 * lk) = z;
+      for (int i = 0; i < 4; i++)
+        z[i] = (c & 32) ? ((c & 16) ? a[12 + i] : a[8 + i]) : ((c & 16) ? a[4 + i] : a[i]);
+      if (li == (c & 15)) *reinterpret_cast<flt4*>(dst + 16 * st + 4 * lk) = z;
+    }
   }
 };
-__device__ __forceinline__ void md_resident(MdReg& m, const float* A, int b0, int n, int ex, float* V, int ldv,
-                                            float* tau_g, double* dg, double* eg) {
-  constexpr int NT = MD_REG / 64;
-  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, lk = l >> 4;
-  const int S = md_strips(n), nr = 16 * S, T = (nr + 63) >> 6;
-  MdStrip<5> A0;
-  MdStrip<3> A1;
-  MdStrip<1> A2;
-  A0.load(A, b0, S - 1 - wv, li, lk);
-  A1.load(A, b0, S - 16 + wv, li, lk);
-  A2.load(A, b0, S - 17 - wv, li, lk);
-  if (tid < 16) m.ap[tid] = 0.0f;
-  for (int r = tid; r < MD_REG; r += MD_THREADS) m.cb[r] = m.vb[r] = m.wb[r] = 0.0f;
-  __syncthreads();
-  auto column = [&](int s) {
-    const int l0 = A0.last(s), l1 = A1.last(s), l2 = A2.last(s);
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-      if (t != s >> 6) continue;
-      if (t <= l0) A0.column(m, t, s, li, lk);
-      if (t < 3 && t <= l1) A1.column(m, t < 3 ? t : 0, s, li, lk);
-      if (t < 1 && t <= l2) A2.column(m, 0, s, li, lk);
-    }
-  };
-  column(0);
-  for (int k = 0;; k++) {
+template <int I, int N, class F>
+__device__ __forceinline__ void md_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    md_for<I + 1, N>(f);
+  }
+}
+
+struct MdOut {
+  float* V;
+  int n, ldv, nr;  // nr: rows of V (n rounded up to 32)
+};
+// Pivot rows s0 .. s1 (row r is at place r + MD_REG - n of the LDS vectors), all in the first of T tiles, by
+// the waves of class C (0: waves 0 .. 3, 1: 4 .. 7), whose strips have T - C, T - 3 + C and T - 4 - C tiles.
+template <int T, int C>
+__device__ __forceinline__ void md_phase(MdReg& m, const MdOut& o, flt16 (&a0)[MD_T], flt16 (&a1)[MD_T - 2],
+                                         flt16 (&a2)[MD_T - 4], int s0,
+                                         int s1) {
+  constexpr int N0 = T - C, N1 = T - 3 + C, N2 = T - 4 - C, off = 64 * (MD_T - T);
+  // (opaque: addresses formed from it are formed again in each phase, not kept in registers through all of them)
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, li = l & 15, lk = l >> 4;
+  const int st0 = 4 * T - 1 - wv, st1 = 4 * T - 16 + wv, st2 = 4 * T - 17 - wv, sh = MD_REG - o.n;
+  const float* cb = m.cb + off;
+  const float *vb = m.vb + off, *wb = m.wb + off;
+  for (int sm = s0; sm <= s1; sm++) {
+    const int s = sm + sh - off;
     __syncthreads();
-    const int s = k + 1, t0 = s >> 6;
-    if (tid == k) dg[k] = ldexp((double)m.cb[k], ex);
-    if (s >= n) break;
-    // ---- the reflector, the same in every wave
-    float x;
-    {
-      const float z = m.cb[64 * t0 + l];
-      x = 64 * t0 + l > s ? z * z : 0.0f;
+    // ---- the last column's update of the tiles; meanwhile the reflector, the same in every wave
+    float z[T], vc[T], wc[T];
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      z[t] = cb[64 * t + l];
+      if (t < N0) {
+        vc[t] = vb[64 * t + l];
+        wc[t] = wb[64 * t + l];
+      }
     }
-    for (int rb = 64 * (t0 + 1); rb < nr; rb += 64) x += m.cb[rb + l] * m.cb[rb + l];
-    const float alpha = m.cb[s];
+    auto update = [&](auto nt, flt16* a, int st) {
+      if constexpr (decltype(nt)::value > 0) {
+        const float vr = -vb[16 * st + li], wr = -wb[16 * st + li];
+        md_for<0, decltype(nt)::value>([&](auto t) {
+          a[t] = __builtin_amdgcn_mfma_f32_16x16x1f32(vr, wc[t], a[t], 0, 0, 0);
+          a[t] = __builtin_amdgcn_mfma_f32_16x16x1f32(wr, vc[t], a[t], 0, 0, 0);
+        });
+      }
+    };
+    update(std::integral_constant<int, N0>{}, a0, st0);
+    update(std::integral_constant<int, N1>{}, a1, st1);
+    update(std::integral_constant<int, N2>{}, a2, st2);
+    float x = l > s ? z[0] * z[0] : 0.0f;
+#pragma unroll
+    for (int t = 1; t < T; t++) x += z[t] * z[t];
+    const float alpha = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(z[0]), s));
     x = md_sum64(x);
-    float beta = alpha, tau = 0.0f, u0 = 0.0f, sc = 0.0f;
-    const bool refl = __builtin_amdgcn_readfirstlane(__float_as_int(x)) > __float_as_int(1e-24f);  // (see md_columns)
-    if (refl) {
+    float beta = alpha, tau = 0.0f, u0 = 0.0f, sc = 0.0f;  // (no reflector: v = e_s with tau = 0)
+    if (__builtin_amdgcn_readfirstlane(__float_as_int(x)) > __float_as_int(1e-24f)) {  // (see md_columns)
       beta = -copysignf(__builtin_amdgcn_sqrtf(alpha * alpha + x), alpha);
       u0 = alpha - beta;
       tau = -u0 * __builtin_amdgcn_rcpf(beta);
       sc = __builtin_amdgcn_rcpf(u0);
     }
-    if (tid == 0) {
-      tau_g[k] = tau;
-      eg[k] = ldexp((double)beta, ex);
+    if constexpr (T == MD_T) __builtin_amdgcn_sched_barrier(0);
+    // ---- products with u = v / sc; the column that comes next, not yet updated with this v and w
+    MdStrip<N0> r0;
+    MdStrip<N1> r1;
+    MdStrip<N2> r2;
+    r0.begin(cb, st0, s, u0, lk);
+    r1.begin(cb, st1, s, u0, lk);
+    r2.begin(cb, st2, s, u0, lk);
+    r0.column(m.an + off, a0[0], st0, s, li, lk);
+    r1.column(m.an + off, a1[0], st1, s, li, lk);
+    r2.column(m.an + off, a2[0], st2, s, li, lk);
+    float asum = 0.0f;
+    md_for<0, N0>([&](auto t) {
+      flt4 uc, ca = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        const int c = 16 * b + li;
+        uc[b] = cb[64 * t + c];
+        if constexpr (t == 0) uc[b] = c < s ? 0.0f : c == s ? u0 : uc[b];
+      }
+      r0.template product<t>(a0[t], uc, ca, st0 & 3);
+      r1.template product<t>(a1[t < MD_T - 2 ? t : 0], uc, ca, st1 & 3);
+      r2.template product<t>(a2[t < MD_T - 4 ? t : 0], uc, ca, st2 & 3);
+      asum += (ca[0] * uc[0] + ca[1] * uc[1]) + (ca[2] * uc[2] + ca[3] * uc[3]);
+      m.cpart[wv][off + 64 * t + l] = md_add16(md_add32(ca[0], ca[2]), md_add32(ca[1], ca[3]));
+      if constexpr (T == MD_T) __builtin_amdgcn_sched_barrier(0);
+    });
+    asum += r0.end(m.ysum + off, st0, li, lk);
+    asum += r1.end(m.ysum + off, st1, li, lk);
+    asum += r2.end(m.ysum + off, st2, li, lk);
+    if constexpr (N0 > 0) asum = md_sum64(asum);
+    if (l == 0) m.ap[wv] = asum;
+    __syncthreads();
+    // ---- w = tau (A v) - (tau^2 / 2) (v^T A v) v, and the next column
+    if constexpr (T == MD_T) asm volatile("" : "+v"(tid));
+    if (64 * wv < o.nr && 64 * wv + 63 >= ((sm - 1) & ~(MD_NB - 1))) {
+      const int p = min(tid + sh, MD_REG - 1), ps = off + s;
+      float y = m.ysum[p], ys = m.ysum[ps], c[MD_WAVES], cs[MD_WAVES];
+#pragma unroll
+      for (int i = 0; i < MD_WAVES; i++) {
+        c[i] = m.cpart[i][p];
+        cs[i] = m.cpart[i][ps];
+      }
+      const float a = m.an[p], u = m.cb[p];
+      const float va = 0.5f * tau * sc * sc * md_sum16(m.ap[li]);
+      y += ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+      ys += ((cs[0] + cs[1]) + (cs[2] + cs[3])) + ((cs[4] + cs[5]) + (cs[6] + cs[7]));
+      const bool in = tid >= sm && tid < o.n;
+      const float v = in ? (tid == sm ? 1.0f : u * sc) : 0.0f;
+      const float w = in ? tau * (y * sc - va * v) : 0.0f, ws = tau * (ys * sc - va);
+      const float nx = a - v * ws - w;
+      if (tid < o.n) {
+        m.vb[p] = v;
+        m.wb[p] = w;
+        m.cb[p] = nx;
+      }
+      if (tid >= ((sm - 1) & ~(MD_NB - 1)) && tid < o.nr) o.V[(unsigned)((sm - 1) * o.ldv + tid)] = v;
+      if (tid == sm) {
+        m.tau[sm - 1] = tau;
+        m.e[sm - 1] = beta;
+        m.d[sm] = nx;
+      }
     }
-    if (refl) {
-      float asum = 0.0f;
-      A0.begin(m, s, u0, lk);
-      A1.begin(m, s, u0, lk);
-      A2.begin(m, s, u0, lk);
-      const int l0 = A0.last(s), l1 = A1.last(s), l2 = A2.last(s);
+  }
+}
+// the waves of class C
+template <int C, class G>
+__device__ __forceinline__ void md_tiles(MdReg& m, const MdOut& o, const G& get) {
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = threadIdx.x & 63, li = l & 15, lk = l >> 4;
+  const int T0 = (o.n + 63) >> 6, S = 4 * T0, sh = MD_REG - o.n, pad = 64 * T0 - o.n;
+  flt16 a0[MD_T], a1[MD_T - 2], a2[MD_T - 4];
+  auto load = [&](flt16& a, int t, int st) {
 #pragma unroll
-      for (int t = 0; t < NT; t++) {
-        if (t < t0) continue;
-        if (t >= T) break;
-        flt4 uc = *reinterpret_cast<const flt4*>(m.cb + 64 * t + 4 * li), ca = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (t == t0)
+    for (int b = 0; b < 4; b++)
 #pragma unroll
-          for (int i = 0; i < 4; i++) {
-            const int c = 64 * t + 4 * li + i;
-            uc[i] = c < s ? 0.0f : c == s ? u0 : uc[i];
-          }
-        if (t <= l0) A0.product(t, uc, ca, li);
-        if (t < 3 && t <= l1) A1.product(t < 3 ? t : 0, uc, ca, li);
-        if (t < 1 && t <= l2) A2.product(0, uc, ca, li);
-        asum += (ca[0] * uc[0] + ca[1] * uc[1]) + (ca[2] * uc[2] + ca[3] * uc[3]);
-        m.cpart[wv][64 * t + 4 * li + lk] = md_add16(md_add32(ca[0], ca[2]), md_add32(ca[1], ca[3]));
+      for (int i = 0; i < 4; i++) {
+        const int r = 16 * st + 4 * lk + i - pad, c = 64 * t + 16 * b + li - pad;
+        a[4 * b + i] = 4 * t + b <= st && r >= 0 && c >= 0 ? get(max(r, c), min(r, c)) : 0.0f;
       }
-      asum += A0.end(m, s, li, lk);
-      asum += A1.end(m, s, li, lk);
-      asum += A2.end(m, s, li, lk);
-      asum = md_sum64(asum);
-      if (l == 0) m.ap[wv] = asum;
-      __syncthreads();
-      // ---- w = tau (A v) - (tau^2 / 2) (v^T A v) v
-      if (64 * wv < nr && 64 * wv + 63 >= s) {
-        const float va = sc * sc * md_sum16(m.ap[li]);
-        const int r = tid;
-        float y = m.ysum[r], p[MD_WAVES];
+    __builtin_amdgcn_sched_barrier(0);  // a tile at a time: the next ones' loads would cost registers
+  };
+  md_for<0, MD_T - C>([&](auto t) { load(a0[t], t, S - 1 - wv); });
+  md_for<0, MD_T - 3 + C>([&](auto t) { load(a1[t], t, S - 16 + wv); });
+  md_for<0, MD_T - 4 - C>([&](auto t) { load(a2[t], t, S - 17 - wv); });
+  md_for<0, MD_T>([&](auto p) {
+    constexpr int T = MD_T - p, off = 64 * p;
+    if (T > T0) return;
+    md_phase<T, C>(m, o, a0, a1, a2, max(1, off - sh), min(o.n - 1, off + 63 - sh));
 #pragma unroll
-        for (int i = 0; i < MD_WAVES; i++) p[i] = m.cpart[i][r];
-        const float u = m.cb[r];
-        y += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
-        const bool in = r >= s && r < n;
-        const float v = in ? (r == s ? 1.0f : u * sc) : 0.0f;
-        const float w = in ? tau * (y * sc - 0.5f * tau * va * v) : 0.0f;
-        m.vb[r] = v;
-        m.wb[r] = w;
-        if (r < nr) V[(long long)k * ldv + r] = v;
-      }
-      __syncthreads();
-      A0.rows_vw(m, s, lk);
-      A1.rows_vw(m, s, lk);
-      A2.rows_vw(m, s, lk);
+    for (int t = 0; t < MD_T - 1 - C; t++) a0[t] = a0[t + 1];
 #pragma unroll
-      for (int t = 0; t < NT; t++) {
-        if (t < t0) continue;
-        if (t >= T) break;
-        const flt4 vc = *reinterpret_cast<const flt4*>(m.vb + 64 * t + 4 * li);
-        const flt4 wc = *reinterpret_cast<const flt4*>(m.wb + 64 * t + 4 * li);
-        if (t <= l0) A0.update(t, vc, wc);
-        if (t < 3 && t <= l1) A1.update(t < 3 ? t : 0, vc, wc);
-        if (t < 1 && t <= l2) A2.update(0, vc, wc);
-      }
-    } else {
-      __syncthreads();  // every wave has read the column
-    }
-    // v's zero rows from the panel's first on (the back-transformation reads no earlier ones): those before
-    // the waves that store v, or all of them
-    if (tid >= (k & ~(MD_NB - 1)) && tid < (refl ? s & ~63 : nr)) V[(long long)k * ldv + tid] = 0.0f;
-    column(s);
+    for (int t = 0; t < MD_T - 4 + C; t++) a1[t] = a1[t + 1];
+#pragma unroll
+    for (int t = 0; t < MD_T - 5 - C; t++) a2[t] = a2[t + 1];
+  });
+}
+__device__ __forceinline__ float* md_uniform(float* p) {  // into scalar registers
+  const unsigned long long a = reinterpret_cast<unsigned long long>(p);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((int)a), hi = __builtin_amdgcn_readfirstlane((int)(a >> 32));
+  return reinterpret_cast<float*>((unsigned long long)hi << 32 | lo);
+}
+template <class G>
+__device__ __forceinline__ void md_resident(MdReg& m, const MdOut& o, int ex, float* tau, double* dg, double* eg,
+                                            const G& get) {
+  const int tid = threadIdx.x, sh = MD_REG - o.n;
+  if (tid < 16) m.ap[tid] = 0.0f;
+  for (int r = tid; r < MD_REG; r += MD_THREADS) {
+    m.vb[r] = m.wb[r] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < MD_WAVES; w++) m.cpart[w][r] = 0.0f;  // (a wave adds nothing to tiles it has no part of)
+    if (r >= sh) m.cb[r] = get(r - sh, 0);
+  }
+  if (tid == 0) m.d[0] = get(0, 0);
+  // (both sides pass the same number of barriers)
+  if (__builtin_amdgcn_readfirstlane(tid >> 6) < 4) md_tiles<0>(m, o, get);
+  else md_tiles<1>(m, o, get);
+  __syncthreads();
+  if (tid < o.n) dg[tid] = ldexp((double)m.d[tid], ex);
+  if (tid < o.n - 1) {
+    eg[tid] = ldexp((double)m.e[tid], ex);
+    tau[tid] = m.tau[tid];
   }
 }
 
 // One block per workgroup.  While more than MD_REG rows are left the working matrix is read from L2 (one CU
 // takes 64 B per clock at best, 44 B achieved: 11 us per column at 620 rows, which bounds blocks of 400 rows
-// and more); the rest of the reduction runs on the trailing matrix in registers, 2.0 .. 2.9 us per column
-// for 100 .. 320 rows, bound by the chain of its three phases (from LDS it took 2.8 .. 4.5 us).  Whole blocks:
-// 0.19 ms at 96 rows, 0.44 at 192, 0.91 at 320, 2.5 at 512, 4.1 at 619, 6.4 at 768.
+// and more); the rest of the reduction runs on the trailing matrix in registers, 1.2 .. 1.9 us per column
+// for 100 .. 330 rows: at the narrow end the chain reflector - products - w with its two barriers, at the
+// wide end the products' 32 multiply-adds per tile and lane.  (The update on the vector units and a third barrier
+// in the place of the repeated w: 2.0 .. 2.9 us; from LDS: 2.8 .. 4.5 us.)  384 rows are what the registers
+// hold; a seventh tile would spill.  Whole blocks: 0.11 ms at 96 rows, 0.26 at 192, 0.56 at 320, 0.61 at 330,
+// 2.0 at 512, 3.5 at 619, 5.9 at 768.
 __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __restrict__ bl,
                                                            const double* __restrict__ Ha, float* __restrict__ Aa,
                                                            float* __restrict__ Va, float* __restrict__ taua,
@@ -628,6 +671,12 @@ __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __res
   for (int w = 0; w < MD_WAVES; w++) mx = s_max[w] > mx || s_max[w] != s_max[w] ? s_max[w] : mx;
   // (a NaN or an infinity goes on into X and the refinement, which leaves such a block unconverged)
   const int ex = mx > 0.0 && mx <= 1.7976931348623157e308 ? ilogb(mx) + 1 : 0;
+  MdReg& m = *reinterpret_cast<MdReg*>(lds);
+  if (n <= MD_REG) {
+    md_resident(m, MdOut{md_uniform(V), n, ldv, ldv}, ex, tau, ws.d, ws.e,
+                [&](int r, int c) { return (float)ldexp(H[(long long)r * n + c], -ex); });
+    return;
+  }
   for (int r = wv; r < ldv; r += MD_WAVES) {
     float* dst = A + 1024 * md_strip(r >> 4) + (r & 15) * 64;
     for (int c = l, t = 0; t <= r >> 6; c += 64, t++) {
@@ -636,10 +685,14 @@ __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __res
     }
   }
   __syncthreads();
-  const int b0 = n > MD_REG ? (n - MD_REG + 63) / 64 * 64 : 0;  // columns reduced in memory
-  if (b0 > 0) md_columns(A, md_lds(lds, n), n, b0, ex, V, ldv, tau, ws.d, ws.e);
-  md_resident(*reinterpret_cast<MdReg*>(lds), A, b0, n - b0, ex, V + (long long)b0 * ldv + b0, ldv, tau + b0,
-              ws.d + b0, ws.e + b0);
+  const int b0 = (n - MD_REG + 63) / 64 * 64;  // columns reduced in memory
+  md_columns(A, md_lds(lds, n), n, b0, ex, V, ldv, tau, ws.d, ws.e);
+  md_resident(m, MdOut{md_uniform(V + (long long)b0 * ldv + b0), n - b0, ldv, ldv - b0}, ex, tau + b0, ws.d + b0,
+              ws.e + b0,
+              [&](int r, int c) {
+                const float z = A[1024 * (md_strip((b0 + r) >> 4) + ((b0 + c) >> 6)) + (r & 15) * 64 + (c & 63)];
+                return r == c ? 2.0f * z : z;
+              });
 }
 
 // The WY factor of panel p of each block: T_p upper triangular with H_{j0} .. H_{j0+nb-1} =

@@ -1,5 +1,5 @@
 """The batched solver's FP32 Householder stage with its FP64 refinement, at the widths where its kernels
-change course: whole and partial strips (16 rows), tiles (64) and register blocks (320 rows and more are
+change course: whole and partial strips (16 rows), tiles (64) and register blocks (more than 384 rows are
 reduced in memory first), one-column panels, the widest block it takes (768).
 
 H = Q diag(lam) Q^T with Haar Q.  Bounds, in units of the largest |lam|: forming H rounds it by about n eps
