@@ -176,17 +176,25 @@ void Chain::prepare_blocks(const std::vector<int>& dims, const double* H) {
   NRGK_HIP(hipSetDevice(ctx->device));
   // LAPACKE_dsyevd(ROW_MAJOR, 'U') reads only the upper triangle of each block (qmatrix.hpp:390-391):
   // it is mirrored into the lower one, which the batched solver also reads
-  std::vector<double> Hs(H, H + tot_elems);
-  for (int s = 0; s < S; s++) {
-    double* A = Hs.data() + cur_off[s];
-    const int n = dims[s];
-    for (int i = 0; i < n; i++)
-      for (int j = 0; j < i; j++) A[(size_t)i * n + j] = A[(size_t)j * n + i];
-  }
   dH.ensure((size_t)tot_elems * sizeof(double));
-  NRGK_HIP(hipMemcpyAsync(dH.p, Hs.data(), (size_t)tot_elems * sizeof(double), hipMemcpyHostToDevice, st));
-  // the host copy must outlive the asynchronous copy
-  NRGK_HIP(stream_sync(st));
+  NRGK_HIP(hipMemcpyAsync(dH.p, H, (size_t)tot_elems * sizeof(double), hipMemcpyHostToDevice, st));
+  std::vector<EigBlock> blks;
+  std::vector<int4> tiles;
+  for (int s = 0; s < S; s++) {
+    EigBlock b{};
+    b.off = cur_off[s];
+    b.n = dims[s];
+    const int T = (b.n + 63) / 64;
+    for (int i = 0; i < T; i++)
+      for (int j = i; j < T; j++) tiles.push_back(int4{s, i, j, 0});
+    blks.push_back(b);
+  }
+  Staging::Region rg = stg.open(Staging::span<EigBlock>(blks.size()) + Staging::span<int4>(tiles.size()));
+  const EigBlock* db = stg.place(rg, blks);
+  const int4* dt = stg.place(rg, tiles);
+  stg.commit(rg, st);
+  launch_mirror(db, dt, (int)tiles.size(), dH.as<double>(), st);
+  sync();  // the caller's array is read no more
 }
 
 void Chain::sync() {

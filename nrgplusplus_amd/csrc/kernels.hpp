@@ -5,6 +5,7 @@
 namespace nrgk {
 
 // k_assemble.hip
+void launch_mirror(const EigBlock* blocks, const int4* tiles, int n_tiles, double* H, hipStream_t s);
 void launch_assemble(const AsmSector* sectors, int n_sectors, int n_rows, const AsmSub* subs, const AsmCon* cons,
                      const double* e_prev, const double* e_bath, const double* f_prev, const double* f_bath,
                      double rescale, double* H, hipStream_t s);
