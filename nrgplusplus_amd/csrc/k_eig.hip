@@ -333,7 +333,7 @@ __device__ void rr_small_wave(const double* Sb, const double* Rb, double* Eb, in
 //   k_oa_entries  32x32 tiles: E_ij (coalesced), largest out-of-cluster residual |rho_ij|
 // conv[4b..4b+3] = (largest residual, largest orthogonality defect, noise level, largest out-of-cluster
 // rotation |rho_ij / (lt_j - lt_i)|) of active block b.
-//   k_oa_rr       one workgroup per block: Rayleigh-Ritz of every cluster of two or more
+//   k_oa_rr       a workgroup per 32 rows of a block: Rayleigh-Ritz of every cluster of two or more
 constexpr int OT = 32;
 constexpr int OA_CONV = 4;  // entries of conv per block
 
@@ -599,7 +599,9 @@ __global__ void __launch_bounds__(256) k_oa_entries(const EigBlock* __restrict__
 
 // Rayleigh-Ritz on every cluster of two or more: M = 1.5 I - 0.5 Rp_JJ, (M S_JJ M) Q = Q mu,
 // E_JJ = M Q - I and the out-of-cluster rows of E(:,J) mapped through M Q.  Clusters of up to
-// RR_SMALL members one wave each, the wider ones in turn by the whole workgroup.
+// RR_SMALL members one wave each, the wider ones in turn by a whole workgroup, of which a block has one to
+// 32 rows: the blocks of a two-channel step
+__host__ __device__ __forceinline__ int oa_rr_parts(int n) { return n < 64 ? 1 : n < 1024 ? n / 32 : 32; }
 __global__ void __launch_bounds__(1024) k_oa_rr(const EigBlock* __restrict__ blocks, const double* __restrict__ S,
                                                 const double* __restrict__ Rp, double* __restrict__ E,
                                                 double* __restrict__ lam, const int* __restrict__ cid_g,
@@ -609,8 +611,10 @@ __global__ void __launch_bounds__(1024) k_oa_rr(const EigBlock* __restrict__ blo
                                                 double e_tol, double d_tol) {
   extern __shared__ double sh[];
   const EigBlock blk = blocks[blockIdx.x];
-  const int n = blk.n;
-  if (n < 2) return;
+  // the block's clusters are shared out over oa_rr_parts(n) workgroups by their first member's place (they
+  // touch disjoint columns of E); those wider than RR_MAX, which share scratch, go to the first
+  const int n = blk.n, part = blockIdx.y, parts = oa_rr_parts(n);
+  if (n < 2 || part >= parts) return;
   const bool last = oa_converged(conv, blockIdx.x, e_tol, d_tol);
   const double* Sb = S + blk.off;
   const double* Rb = Rp + blk.off;
@@ -636,7 +640,7 @@ __global__ void __launch_bounds__(1024) k_oa_rr(const EigBlock* __restrict__ blo
     if (s > 0 && csort[s] == csort[s - 1]) continue;
     int e = s + 1;
     while (e < n && csort[e] == csort[s]) e++;
-    if (e - s >= 2) {
+    if (e - s >= 2 && part == (e - s > RR_MAX ? 0 : (s >> 3) % parts)) {
       const int slot = atomicAdd(&s_nc, 1);
       cstart[2 * slot] = s;
       cstart[2 * slot + 1] = e;
@@ -859,7 +863,7 @@ void launch_oa(const EigBlock* blocks, int nb, const int4* sym_tiles, int n_sym,
   NRGK_HIP(hipGetLastError());
   NRGK_LAUNCH(k_oa_entries, dim3(n_all), dim3(256), 0, s, blocks, all_tiles, S, Rp, lam, cid, E, conv);
   NRGK_HIP(hipGetLastError());
-  NRGK_LAUNCH(k_oa_rr, dim3(nb), dim3(1024), oa_rr_lds(nmax), s, blocks, S, Rp, E, lam, cid, sidx, scrW, scrG,
+  NRGK_LAUNCH(k_oa_rr, dim3(nb, oa_rr_parts(nmax)), dim3(1024), oa_rr_lds(nmax), s, blocks, S, Rp, E, lam, cid, sidx, scrW, scrG,
                      scrT, rrv, conv, e_tol, d_tol);
   NRGK_HIP(hipGetLastError());
   NRGK_LAUNCH(k_oa_mask, dim3(n_all), dim3(256), 0, s, blocks, all_tiles, cid, conv, e_tol, d_tol, E);

@@ -79,3 +79,19 @@ def test_blocks_that_fall_apart(nk):
     for H, (w, U) in zip(blocks, out):
         _check(H, w, U, np.linalg.eigvalsh(H))
     np.testing.assert_array_equal(out[4][0], np.zeros(70))
+
+
+def test_multiplets(nk):
+    """clusters of one to 70 members, many of each size in a block: those of up to 8, up to 64 and more take
+    different paths, and a block's are shared out over its workgroups"""
+    rng = np.random.default_rng(13)
+    blocks, lams = [], []
+    for n in (66, 95, 96, 127, 128, 500, 768):
+        sizes = []
+        while sum(sizes) < n:
+            sizes.append(int(rng.choice([1, 2, 3, 8, 9, 20, 64, 65, 70])))
+        lam = np.repeat(rng.permutation(np.linspace(-1, 1, len(sizes))), sizes)[:n]
+        lams.append(np.sort(lam))
+        blocks.append(_block(rng, lam))
+    for H, lam, (w, U) in zip(blocks, lams, nk.eigh_batched(blocks)):
+        _check(H, w, U, lam)
