@@ -700,7 +700,7 @@ void Chain::eigensolve_mixed() {
     // eigenpairs of T: eigenvalues far closer than FP32 resolves them, then inverse iteration
     prof_begin("mid_tridiag");
     launch_ht_sturm(dht, mht, W, dlam_tmp.as<double>(), 1e-11, st);
-    launch_ht_stein(dht, mht, W, dlam_tmp.as<double>(), dX.as<double>(), scr, 1e-6,
+    launch_ht_stein(dht, mht, W, dlam_tmp.as<double>(), dX.as<double>(), scr, 1e-6, 1,
                     d_mid_q.as<int>() + 64, d_mid_q.as<int>(), st);
     prof_end("mid_tridiag", 7, 0.0, 0.0);
     prof_begin("mid_back");

@@ -610,9 +610,9 @@ __global__ void __launch_bounds__(256) k_ht_syr2k(const HtBlock* __restrict__ bl
 // eigenvalue below x): one fused operation on the dependent chain of a step, where the quotients
 // p_i / p_{i-1} of the usual form take a reciprocal and three more.  T is scaled to about unit norm, so
 // the polynomials stay in range over eight steps, after which they are rescaled by a power of two.
-// A pass costs a wavefront about nine operations a row whatever LANES is, so eight lanes pay while the
-// wavefronts still find free SIMDs (17 passes instead of 52: five blocks of ~1 000 rows 2.3 -> 0.4 ms); where
-// the eigenvalues alone fill the chip, one lane each does the least work.
+// A pass costs a wavefront about nine operations a row whatever LANES is, so more lanes pay while the
+// wavefronts still find free SIMDs: sixteen for 4 100 eigenvalues in blocks of up to 360 rows take 85 us where
+// eight take 117 and one takes 600; where the eigenvalues alone fill the chip, one lane each does the least work.
 constexpr int ST_UNROLL = 8;
 template <int ST_LANES>
 __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
@@ -633,6 +633,7 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
   const int n = B.n, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
   const HtWs w = ht_ws(const_cast<double*>(Wa) + B.w_off, n, B.T);
   __shared__ double rlo[4], rhi[4];
+  __shared__ unsigned short grid[256];
   double lo = 1e300, hi = -1e300;
   for (int i = tid; i < n; i += 256) {
     const double di = w.d[i], rad = (i < n - 1 ? fabs(w.e[i]) : 0.0) + (i > 0 ? fabs(w.e[i - 1]) : 0.0);
@@ -670,10 +671,7 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
   constexpr double PIV = 1e-32;
   const bool mine = j < n;
   const double tol = fmax(rtol, 0.5 * eps);
-  for (int it = 0; it < 64; it++) {
-    const bool go = mine && c - a > fmax(tol, 2.0 * eps * fmin(fabs(a), fabs(c)));
-    if (__ballot(go) == 0) break;
-    const double h = (c - a) * (1.0 / (ST_LANES + 1)), x = a + (ln + 1) * h;
+  auto count = [&](double x) {  // eigenvalues below x
     int cnt = 0;
     double p1 = 1.0, p2 = 0.0;
     for (int i0 = 0; i0 < nf; i0 += ST_UNROLL) {
@@ -692,6 +690,27 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
       p1 = __builtin_amdgcn_ldexp(p1, sh);
       p2 = __builtin_amdgcn_ldexp(p2, sh);
     }
+    return cnt;
+  };
+  // the first pass for the whole workgroup: 256 points, between two of which each eigenvalue starts
+  {
+    const double h = (c - a) * (1.0 / 257.0), a0 = a;
+    grid[tid] = (unsigned short)count(a0 + (tid + 1) * h);
+    __syncthreads();
+    int m0 = -1, m1 = 256;  // points m0 (at or below the eigenvalue) and m1 (above it)
+    while (m1 - m0 > 1) {
+      const int m = (m0 + m1) >> 1;
+      if (grid[m] <= j) m0 = m;
+      else m1 = m;
+    }
+    a = m0 >= 0 ? a0 + (m0 + 1) * h : a0;
+    c = m1 < 256 ? a0 + (m1 + 1) * h : c;
+  }
+  for (int it = 0; it < 64; it++) {
+    const bool go = mine && c - a > fmax(tol, 2.0 * eps * fmin(fabs(a), fabs(c)));
+    if (__ballot(go) == 0) break;
+    const double h = (c - a) * (1.0 / (ST_LANES + 1));
+    const int cnt = count(a + (ln + 1) * h);
     // points at or below the eigenvalue: those with at most j eigenvalues below them
     const unsigned long long in = __ballot(cnt <= j);
     const int m = __popc((unsigned)(in >> (l & ~(ST_LANES - 1))) & ((1u << ST_LANES) - 1));
@@ -706,12 +725,11 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
 
 // deterministic start vector entries in [-1, 1)
 __device__ __forceinline__ double ht_start(unsigned p, unsigned i) {
-  unsigned long long x = ((unsigned long long)p << 32) ^ (unsigned long long)(i + 0x9E3779B9u);
-  x += 0x9E3779B97F4A7C15ull;
-  x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
-  x = (x ^ (x >> 27)) * 0x94D049BB133111EBull;
-  x ^= x >> 31;
-  return (double)(x >> 11) * (2.0 / 9007199254740992.0) - 1.0;
+  unsigned x = p * 0x9E3779B9u ^ (i + 1u) * 0x85EBCA6Bu;
+  x ^= x >> 16;
+  x *= 0x7FEB352Du;
+  x ^= x >> 15;
+  return (double)(int)x * (1.0 / 2147483648.0);
 }
 
 // Rows per register tile of the column loops below: each tile's loads are issued together, so a
@@ -756,6 +774,29 @@ __device__ __forceinline__ void ht_bwd_load(const double* __restrict__ U, int n,
 // perturbation), which bounds the growth of one step by about 1 / piv0.
 // Each pass requests the next HT_RT rows before it stores the current ones: a wait on vector memory
 // also waits for every store issued before the awaited load, so the loads are not held behind them.
+// 1 / x to an ulp or so: the pivots' reciprocals stand in the elimination's dependent chain, where the IEEE
+// division takes three times as long
+__device__ __forceinline__ double ht_rcp(double x) {
+  double r = __builtin_amdgcn_rcp(x);
+  r = fma(fma(-x, r, 1.0), r, r);
+  return fma(fma(-x, r, 1.0), r, r);
+}
+// row i of the forward elimination (sub, nu: T's entries below and right of the next row's diagonal, nd: that
+// less the eigenvalue, x: the next row's right-hand side; f0 .. and ur: row i of the factors and of U).  Without
+// branches: lanes that exchange rows i and i + 1 stand beside lanes that do not.
+__device__ __forceinline__ void ht_fwd_row(double sub, double nd, double nu, double x, double piv0, double* f0, double* f1,
+                                           double* f2, double* ur, int p, int slot, double& cd, double& cu, double& xi) {
+  const bool sw = fabs(cd) < fabs(sub);
+  const double pc = fabs(cd) < piv0 ? (cd < 0.0 ? -piv0 : piv0) : cd;
+  const double r = ht_rcp(sw ? sub : pc), ml = (sw ? cd : sub) * r;
+  f0[slot] = r;
+  f1[slot] = sw ? nd : cu;
+  f2[slot] = sw ? nu : 0.0;
+  ur[p] = sw ? x : xi;
+  xi = (sw ? xi : x) - ml * (sw ? x : xi);
+  cd = (sw ? cu : nd) - ml * (sw ? nd : cu);
+  cu = sw ? -ml * nu : nu;
+}
 // the forward elimination over rows i0 .. i0 + HT_RT - 1 (cd, cu: the pivot row's diagonal and
 // superdiagonal, xi: its right-hand side)
 __device__ __forceinline__ void ht_fwd_rows(int n, double lp, double piv0, double* __restrict__ U, int p,
@@ -767,56 +808,76 @@ __device__ __forceinline__ void ht_fwd_rows(int n, double lp, double piv0, doubl
   for (int j = 0; j < HT_RT; j++) {
     const int i = i0 + j;
     if (i >= n - 1) continue;
-    const double sub = sb[j], nd = dn[j] - lp, nu = en[j];
-    const long long o = (long long)i * mp + slot;
-    if (fabs(cd) >= fabs(sub)) {
-      if (fabs(cd) < piv0) cd = cd < 0.0 ? -piv0 : piv0;
-      const double r = 1.0 / cd, ml = sub * r;
-      f0[o] = r;
-      f1[o] = cu;
-      f2[o] = 0.0;
-      U[(long long)i * n + p] = xi;
-      xi = xn[j] - ml * xi;
-      cd = nd - ml * cu;
-      cu = nu;
-    } else {  // rows i and i + 1 exchanged
-      const double r = 1.0 / sub, ml = cd * r;
-      f0[o] = r;
-      f1[o] = nd;
-      f2[o] = nu;
-      U[(long long)i * n + p] = xn[j];
-      xi = xi - ml * xn[j];
-      cd = cu - ml * nd;
-      cu = -ml * nu;
-    }
+    ht_fwd_row(sb[j], dn[j] - lp, en[j], xn[j], piv0, f0 + (long long)i * mp, f1 + (long long)i * mp,
+               f2 + (long long)i * mp, U + (long long)i * n, p, slot, cd, cu, xi);
   }
 }
 // the back substitution over rows i1, i1 - 1, .. i1 - HT_RT + 1 (x1, x2: the solution's next two rows)
 __device__ __forceinline__ void ht_bwd_rows(int n, double* __restrict__ U, int p, int i1, const double* uu,
                                             const double* a0, const double* a1, const double* a2, double& x1,
-                                            double& x2) {
+                                            double& x2, double& mx, double& s2) {
 #pragma unroll
   for (int j = 0; j < HT_RT; j++) {
     const int i = i1 - j;
     if (i < 0) continue;
     const double v = (uu[j] - a1[j] * x1 - a2[j] * x2) * a0[j];
     U[(long long)i * n + p] = v;
+    mx = fmax(mx, fabs(v));
+    s2 += v * v;
     x2 = x1;
     x1 = v;
   }
 }
-__device__ void ht_inverse_step(const double* __restrict__ d, const double* __restrict__ e, int n, double lp,
-                                double piv0, double* __restrict__ U, int p, double* __restrict__ f0,
-                                double* __restrict__ f1, double* __restrict__ f2, long long mp, int slot) {
+// The bulk of the rows goes through tiles without bounds, their addresses a scalar row pointer and the lane's own
+// offset and T's entries (gd, ge, in memory) scalar loads; the last ones through the bounded tiles above (d, e in
+// LDS).  One wavefront per SIMD runs this, so instructions count: blocks of up to 360 rows, 158 -> 87 us a step.
+template <bool FIRST>
+__device__ void ht_inverse_step(const double* __restrict__ d, const double* __restrict__ e, const double* __restrict__ gd,
+                                const double* __restrict__ ge, int n, double lp, double piv0, double* __restrict__ U,
+                                int p, double* __restrict__ f0, double* __restrict__ f1, double* __restrict__ f2,
+                                long long mp, int slot, double& mx, double& s2) {
   double cd = d[0] - lp, cu = n > 1 ? e[0] : 0.0;
-  double xi = U[p];
+  double xi = FIRST ? ht_start((unsigned)p, 0u) : U[p];
+  const long long sn = n;
+  int i0 = 0;
+  if (n - 1 >= 3 * HT_RT) {
+    auto load = [&](double* x, int i) {
+      const double* ur = U + (i + 1) * sn;
+#pragma unroll
+      for (int j = 0; j < HT_RT; j++) x[j] = FIRST ? ht_start((unsigned)p, (unsigned)(i + 1 + j)) : (ur + j * sn)[p];
+    };
+    auto rows = [&](const double* x, int i) {
+      double tile_d[HT_RT], tile_e[HT_RT + 1];
+#pragma unroll
+      for (int j = 0; j < HT_RT; j++) tile_d[j] = gd[i + 1 + j];
+#pragma unroll
+      for (int j = 0; j <= HT_RT; j++) tile_e[j] = ge[i + j];
+      double *q0 = f0 + i * mp, *q1 = f1 + i * mp, *q2 = f2 + i * mp, *ur = U + i * sn;
+#pragma unroll
+      for (int j = 0; j < HT_RT; j++)
+        ht_fwd_row(tile_e[j], tile_d[j] - lp, tile_e[j + 1], x[j], piv0, q0 + j * mp, q1 + j * mp, q2 + j * mp,
+                   ur + j * sn, p, slot, cd, cu, xi);
+    };
+    double xa[HT_RT], xb[HT_RT];
+    load(xa, 0);
+    for (; i0 + 3 * HT_RT <= n - 1; i0 += 2 * HT_RT) {
+      load(xb, i0 + HT_RT);
+      __builtin_amdgcn_sched_barrier(0);  // keep these loads ahead of the stores below
+      rows(xa, i0);
+      load(xa, i0 + 2 * HT_RT);
+      __builtin_amdgcn_sched_barrier(0);
+      rows(xb, i0 + HT_RT);
+    }
+  }
+  if (FIRST)
+    for (int i = i0 + 1; i < n; i++) U[i * sn + p] = ht_start((unsigned)p, (unsigned)i);
   if (n >= 2) {
     // two register tiles in turn: each is refilled while the other one's rows are eliminated
     double xa[HT_RT], sa[HT_RT], da[HT_RT], ea[HT_RT], xb[HT_RT], sb[HT_RT], db[HT_RT], eb[HT_RT];
-    ht_fwd_load(d, e, n, U, p, 0, xa, sa, da, ea);
-    for (int i0 = 0; i0 < n - 1; i0 += 2 * HT_RT) {
+    ht_fwd_load(d, e, n, U, p, i0, xa, sa, da, ea);
+    for (; i0 < n - 1; i0 += 2 * HT_RT) {
       ht_fwd_load(d, e, n, U, p, i0 + HT_RT, xb, sb, db, eb);
-      __builtin_amdgcn_sched_barrier(0);  // keep these loads ahead of the stores below
+      __builtin_amdgcn_sched_barrier(0);
       ht_fwd_rows(n, lp, piv0, U, p, f0, f1, f2, mp, slot, i0, xa, sa, da, ea, cd, cu, xi);
       ht_fwd_load(d, e, n, U, p, i0 + 2 * HT_RT, xa, sa, da, ea);
       __builtin_amdgcn_sched_barrier(0);
@@ -825,26 +886,58 @@ __device__ void ht_inverse_step(const double* __restrict__ d, const double* __re
   }
   if (fabs(cd) < piv0) cd = cd < 0.0 ? -piv0 : piv0;
   const long long ol = (long long)(n - 1) * mp + slot;
-  f0[ol] = 1.0 / cd;
+  f0[ol] = ht_rcp(cd);
   f1[ol] = 0.0;
   f2[ol] = 0.0;
   U[(long long)(n - 1) * n + p] = xi;
   double x1 = 0.0, x2 = 0.0;
+  mx = s2 = 0.0;
+  int i1 = n - 1;
+  if (n >= 3 * HT_RT) {
+    auto load = [&](double* uu, double* a0, double* a1, double* a2, int i) {
+      const double *q0 = f0 + i * mp, *q1 = f1 + i * mp, *q2 = f2 + i * mp, *ur = U + i * sn;
+#pragma unroll
+      for (int j = 0; j < HT_RT; j++) {
+        uu[j] = (ur - j * sn)[p];
+        a0[j] = (q0 - j * mp)[slot];
+        a1[j] = (q1 - j * mp)[slot];
+        a2[j] = (q2 - j * mp)[slot];
+      }
+    };
+    auto rows = [&](const double* uu, const double* a0, const double* a1, const double* a2, int i) {
+      double* ur = U + i * sn;
+#pragma unroll
+      for (int j = 0; j < HT_RT; j++) {
+        const double v = (uu[j] - a1[j] * x1 - a2[j] * x2) * a0[j];
+        (ur - j * sn)[p] = v;
+        mx = fmax(mx, fabs(v));
+        s2 += v * v;
+        x2 = x1;
+        x1 = v;
+      }
+    };
+    double ua[HT_RT], a0[HT_RT], a1[HT_RT], a2[HT_RT], ub[HT_RT], b0[HT_RT], b1[HT_RT], b2[HT_RT];
+    load(ua, a0, a1, a2, i1);
+    for (; i1 - 3 * HT_RT >= -1; i1 -= 2 * HT_RT) {
+      load(ub, b0, b1, b2, i1 - HT_RT);
+      __builtin_amdgcn_sched_barrier(0);
+      rows(ua, a0, a1, a2, i1);
+      load(ua, a0, a1, a2, i1 - 2 * HT_RT);
+      __builtin_amdgcn_sched_barrier(0);
+      rows(ub, b0, b1, b2, i1 - HT_RT);
+    }
+  }
   double ua[HT_RT], a0[HT_RT], a1[HT_RT], a2[HT_RT], ub[HT_RT], b0[HT_RT], b1[HT_RT], b2[HT_RT];
-  ht_bwd_load(U, n, p, n - 1, f0, f1, f2, mp, slot, ua, a0, a1, a2);
-  for (int i1 = n - 1; i1 >= 0; i1 -= 2 * HT_RT) {
+  ht_bwd_load(U, n, p, i1, f0, f1, f2, mp, slot, ua, a0, a1, a2);
+  for (; i1 >= 0; i1 -= 2 * HT_RT) {
     ht_bwd_load(U, n, p, i1 - HT_RT, f0, f1, f2, mp, slot, ub, b0, b1, b2);
     __builtin_amdgcn_sched_barrier(0);
-    ht_bwd_rows(n, U, p, i1, ua, a0, a1, a2, x1, x2);
+    ht_bwd_rows(n, U, p, i1, ua, a0, a1, a2, x1, x2, mx, s2);
     ht_bwd_load(U, n, p, i1 - 2 * HT_RT, f0, f1, f2, mp, slot, ua, a0, a1, a2);
     __builtin_amdgcn_sched_barrier(0);
-    ht_bwd_rows(n, U, p, i1 - HT_RT, ub, b0, b1, b2, x1, x2);
+    ht_bwd_rows(n, U, p, i1 - HT_RT, ub, b0, b1, b2, x1, x2, mx, s2);
   }
 }
-
-// inverse-iteration steps per eigenvector: from a random start one step leaves the vector off by about
-// eps ||T|| / gap along its neighbours (below 5e-12 outside the clusters), the second polishes it
-constexpr int HT_ITERS = 2;
 
 // the infinity norm of T (d, e in memory p)
 __device__ __forceinline__ double ht_tnorm_entry(const double* d, const double* e, int n, int i) {
@@ -857,24 +950,10 @@ __device__ __forceinline__ int ht_cluster_start_at(const double* L, int n, int x
   return x;
 }
 
-// column p normalised, scaled by its largest entry first so that the squares of an iterate of any
-// size stay finite
-__device__ void ht_col_normalise(double* __restrict__ U, int n, int p) {
-  // one read-only pass forms the largest magnitude and the plain sum of squares (sixteen rows a
-  // batch); only when that sum over- or underflows does a second pass form it from the scaled
-  // entries; then the column is scaled
+// column p, its largest magnitude mx and plain sum of squares s2 given, normalised; only when that sum over-
+// or underflows does another pass form it from the scaled entries
+__device__ void ht_col_normalise(double* __restrict__ U, int n, int p, double mx, double s2) {
   constexpr int RB = 2 * HT_RT;
-  double mx = 0.0, s2 = 0.0;
-  for (int i0 = 0; i0 < n; i0 += RB) {
-    double a[RB];
-#pragma unroll
-    for (int j = 0; j < RB; j++) a[j] = i0 + j < n ? U[(long long)(i0 + j) * n + p] : 0.0;
-#pragma unroll
-    for (int j = 0; j < RB; j++) {
-      mx = fmax(mx, fabs(a[j]));
-      s2 += a[j] * a[j];
-    }
-  }
   if (mx == 0.0) return;
   double inv;
   if (s2 > 1e-280 && s2 < 1e280) {
@@ -903,11 +982,13 @@ __device__ void ht_col_normalise(double* __restrict__ U, int n, int p) {
 
 // Eigenvectors of T for the eigenvalues 0 .. m-1 of each block (and the rest of a cluster that
 // starts below m), into the columns of U.  Clusters are runs of eigenvalues each within ctol of the
-// one before.  The host runs HT_ITERS rounds of
+// one before.  The host runs `iters` rounds of
 //   k_ht_stein_step  one inverse-iteration step for every wanted eigenvector (normalised), from a fixed
 //                    pseudo-random start in the first round
 //   k_ht_stein_mgs   every cluster of more than one member made orthonormal
-// and one more k_ht_stein_mgs at the end.  Orthogonalising after every step matters: the members of a
+// and one more k_ht_stein_mgs at the end.  From a random start one step leaves a vector off along its neighbours
+// by about the eigenvalue's error over the gap: 5e-12 outside the clusters where that is eps ||T||, and the second
+// step polishes it.  Start vectors of the FP64 refinement take one step: their T is itself off by FP32 rounding.  Orthogonalising after every step matters: the members of a
 // numerically degenerate cluster (copies of an eigenvalue in different split blocks of T) are all
 // pulled toward the copy their shifts sit closest to, so steps without it leave them nearly
 // dependent, and their orthogonalisation would then blow up the components outside the cluster;
@@ -925,10 +1006,10 @@ __device__ __forceinline__ double ht_tnorm_wave(const HtWs& w, int n, int lane) 
   for (int o = 32; o > 0; o >>= 1) nm = fmax(nm, __shfl_xor(nm, o, 64));
   return nm;
 }
+template <bool FIRST>
 __global__ void __launch_bounds__(64) k_ht_stein_step(const HtBlock* __restrict__ bl, int nblk,
                                                       const double* __restrict__ Wa, const double* __restrict__ lam,
-                                                      double* __restrict__ Ua, double* __restrict__ Sa, double ctol_rel,
-                                                      int first) {
+                                                      double* __restrict__ Ua, double* __restrict__ Sa, double ctol_rel) {
   int g = blockIdx.x, b = -1;
   for (int i = 0; i < nblk; i++) {
     const int cw = (bl[i].m + HT_CHUNK - 1) / HT_CHUNK;
@@ -967,10 +1048,9 @@ __global__ void __launch_bounds__(64) k_ht_stein_step(const HtBlock* __restrict_
   }
   __syncthreads();
   for (int p = a + lane; p < bend; p += 64) {
-    if (first)
-      for (int i = 0; i < n; i++) U[(long long)i * n + p] = ht_start((unsigned)p, (unsigned)i);
-    ht_inverse_step(td, te, n, L[p], piv0, U, p, f0, f1, f2, mp, slot);
-    ht_col_normalise(U, n, p);
+    double mx, s2;
+    ht_inverse_step<FIRST>(td, te, w.d, w.e, n, L[p], piv0, U, p, f0, f1, f2, mp, slot, mx, s2);
+    ht_col_normalise(U, n, p, mx, s2);
   }
 }
 
@@ -1347,14 +1427,16 @@ void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const 
     return g;
   };
   // (1 024 SIMDs; a wavefront holds 64 / lanes eigenvalues)
-  if (total * 8 <= 2 * 64 * 1024)
+  if (total * 16 <= 80 * 1024)
+    NRGK_LAUNCH(k_ht_sturm<16>, dim3(grid(16)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
+  else if (total * 8 <= 2 * 64 * 1024)
     NRGK_LAUNCH(k_ht_sturm<8>, dim3(grid(8)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
   else
     NRGK_LAUNCH(k_ht_sturm<1>, dim3(grid(1)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
   NRGK_HIP(hipGetLastError());
 }
 void launch_ht_stein(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, const double* lam, double* U,
-                     double* S, double ctol_rel, int* list, int* count, hipStream_t s) {
+                     double* S, double ctol_rel, int iters, int* list, int* count, hipStream_t s) {
   int g = 0, nmax = 1;
   for (const auto& b : bl) {
     g += (b.m + HT_CHUNK - 1) / HT_CHUNK;
@@ -1365,9 +1447,10 @@ void launch_ht_stein(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const 
   const size_t tl = (size_t)nmax * 2 * sizeof(double);  // d and e of the widest block
   NRGK_HIP(hipMemsetAsync(count, 0, sizeof(int), s));
   NRGK_LAUNCH(k_ht_stein_clusters, dim3(nb), dim3(256), 0, s, d_bl, W, lam, ctol_rel, list, count);
-  for (int it = 0; it <= HT_ITERS; it++) {
-    if (it < HT_ITERS)
-      NRGK_LAUNCH(k_ht_stein_step, dim3(g), dim3(64), tl, s, d_bl, nb, W, lam, U, S, ctol_rel, it == 0 ? 1 : 0);
+  for (int it = 0; it <= iters; it++) {
+    if (it < iters)
+      NRGK_LAUNCH(it == 0 ? k_ht_stein_step<true> : k_ht_stein_step<false>, dim3(g), dim3(64), tl, s, d_bl, nb, W, lam, U, S,
+                  ctol_rel);
     // a fixed grid that walks the cluster list (its length is read on the device)
     NRGK_LAUNCH(k_ht_stein_mgs, dim3(1024), dim3(256), 0, s, d_bl, (const int*)list, (const int*)count, U);
   }
@@ -1409,9 +1492,11 @@ int ht_max_n(int lds_bytes) { return (lds_bytes - HT_STATIC_LDS) / (int)(2 * siz
 void set_ht_lds_limits(int bytes) {
   const int dyn = bytes - HT_STATIC_LDS;
   const int dyn_st = dyn + ST_UNROLL * (int)sizeof(double2);
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm<16>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn_st));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm<8>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn_st));
   NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_sturm<1>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn_st));
-  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_stein_step, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_stein_step<true>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
+  NRGK_HIP(hipFuncSetAttribute((const void*)k_ht_stein_step<false>, hipFuncAttributeMaxDynamicSharedMemorySize, dyn));
 }
 
 }  // namespace nrgk

@@ -54,7 +54,7 @@ void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const 
                      hipStream_t s);
 // list: 3 ints per cluster of more than one member (at most the wanted columns), count: one int
 void launch_ht_stein(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const double* W, const double* lam, double* U,
-                     double* S, double ctol_rel, int* list, int* count, hipStream_t s);
+                     double* S, double ctol_rel, int iters, int* list, int* count, hipStream_t s);
 int ht_stein_slots(int m);  // scratch slots (HtBlock::mpad) of the inverse iteration for m columns
 int launch_ht_wy(const HtBlock* d_bl, const std::vector<HtBlock>& bl, int step, const double* V, const double* VT,
                  double* U, double* Ys, hipStream_t s);

@@ -227,7 +227,7 @@ void Chain::wide_vectors(bool all) {
   // bar; 5e-5 brings them to 1.3e-12 for 3.5 ms more orthogonalisation per step)
   const double ctol = env_knob("NRGK_WIDE_CLUSTER", 5e-5);
   prof_begin("tridiag_vectors");
-  launch_ht_stein(d, bl, W, dlam_raw.as<double>(), U, d_wide_s.as<double>(), ctol, d_wide_q.as<int>() + 64,
+  launch_ht_stein(d, bl, W, dlam_raw.as<double>(), U, d_wide_s.as<double>(), ctol, 2, d_wide_q.as<int>() + 64,
                   d_wide_q.as<int>(), st);
   prof_end("tridiag_vectors", 6, 0.0, 0.0);  // the cluster list, two steps, three orthogonalisations
   // V_p T_p over each block's working matrix (no longer needed), then per panel, last first:
