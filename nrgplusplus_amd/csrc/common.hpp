@@ -580,4 +580,31 @@ struct TruncOut {
   int nonfinite;  // eigenvalues that are not finite (the step fails)
 };
 
+#ifdef __HIPCC__
+// The entry that task g of a launch falls to, of n entries with count(i) tasks each in order; g becomes the task's
+// index within it; -1 past the last.  The lanes read 64 counts at once: a scan by scalar loads waits for memory at
+// every entry (half a microsecond each).
+template <class F>
+__device__ __forceinline__ int find_task(int n, int& g, const F& count) {
+  const int lane = threadIdx.x & 63;
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    const int c = i0 + lane < n ? count(i0 + lane) : 0;
+    int end = c;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(end, o, 64);
+      end += lane >= o ? y : 0;
+    }
+    const unsigned long long m = __ballot(g < end);
+    if (m) {
+      const int l = __ffsll(m) - 1;
+      g -= __builtin_amdgcn_readlane(end - c, l);
+      return i0 + l;
+    }
+    g -= __builtin_amdgcn_readlane(end, 63);
+  }
+  return -1;
+}
+#endif
+
 }  // namespace nrgk

@@ -701,15 +701,8 @@ __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __res
 __global__ void __launch_bounds__(256) k_mid_larft(const MidBlock* __restrict__ bl, int nblk,
                                                    const float* __restrict__ Va, const float* __restrict__ taua,
                                                    float* __restrict__ VTa) {
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int P = (bl[i].n + MD_NB - 2) / MD_NB;
-    if (g < P) {
-      b = i;
-      break;
-    }
-    g -= P;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n + MD_NB - 2) / MD_NB; });
   if (b < 0) return;
   const MidBlock B = bl[b];
   const int n = B.n, ldv = 16 * md_strips(n), j0 = g * MD_NB, nb = min(MD_NB, n - 1 - j0);
@@ -762,15 +755,8 @@ __global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restr
                                                          double* __restrict__ Xa) {
   __shared__ float Yp[MB_WAVES][MD_NB][64];
   __shared__ float Ys[MD_NB][80];
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int ct = (bl[i].n + 63) / 64;
-    if (g < ct) {
-      b = i;
-      break;
-    }
-    g -= ct;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n + 63) / 64; });
   if (b < 0) return;
   const MidBlock B = bl[b];
   const int n = B.n, ldv = 16 * md_strips(n), NT = ldv / 16;

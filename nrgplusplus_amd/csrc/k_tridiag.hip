@@ -180,15 +180,8 @@ __device__ __forceinline__ double ht_v(const double* u, const HtRefl& R, int s, 
 // (entries beyond n zero): one workgroup per tile, a row of 64 entries per 64 lanes.
 __global__ void __launch_bounds__(256) k_ht_tile_in(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ H,
                                                     double* __restrict__ Aa) {
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int nt = bl[i].T * (bl[i].T + 1) / 2;
-    if (g < nt) {
-      b = i;
-      break;
-    }
-    g -= nt;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return bl[i].T * (bl[i].T + 1) / 2; });
   if (b < 0) return;
   const HtBlock B = bl[b];
   const int n = B.n;
@@ -619,15 +612,8 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
                                                   double* __restrict__ lam, double rtol) {
   extern __shared__ double2 de[];  // {d_i, e_{i-1}^2}, filled up to a multiple of ST_UNROLL
   constexpr int ST_PER = 256 / ST_LANES;  // eigenvalues per workgroup
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int cw = (bl[i].n + ST_PER - 1) / ST_PER;
-    if (g < cw) {
-      b = i;
-      break;
-    }
-    g -= cw;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n + ST_PER - 1) / ST_PER; });
   if (b < 0) return;
   const HtBlock B = bl[b];
   const int n = B.n, tid = threadIdx.x, l = tid & 63, wv = tid >> 6;
@@ -1010,15 +996,8 @@ template <bool FIRST>
 __global__ void __launch_bounds__(64) k_ht_stein_step(const HtBlock* __restrict__ bl, int nblk,
                                                       const double* __restrict__ Wa, const double* __restrict__ lam,
                                                       double* __restrict__ Ua, double* __restrict__ Sa, double ctol_rel) {
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int cw = (bl[i].m + HT_CHUNK - 1) / HT_CHUNK;
-    if (g < cw) {
-      b = i;
-      break;
-    }
-    g -= cw;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].m + HT_CHUNK - 1) / HT_CHUNK; });
   if (b < 0) return;
   const HtBlock B = bl[b];
   const int n = B.n;
@@ -1144,15 +1123,8 @@ __global__ void __launch_bounds__(256) k_ht_stein_mgs(const HtBlock* __restrict_
 // matrix (columns j0 .. j0 + nbp - 1, rows j0 + 1 .. n - 1).
 __global__ void __launch_bounds__(256) k_ht_larft(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Va,
                                                   const double* __restrict__ Wa, double* __restrict__ Aa) {
-  int g = blockIdx.x, b = -1;
-  for (int i = 0; i < nblk; i++) {
-    const int P = (bl[i].n - 1 + HT_NB - 1) / HT_NB;
-    if (g < P) {
-      b = i;
-      break;
-    }
-    g -= P;
-  }
+  int g = blockIdx.x;
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n - 1 + HT_NB - 1) / HT_NB; });
   if (b < 0) return;
   const HtBlock B = bl[b];
   const int n = B.n, j0 = g * HT_NB, nbp = min(HT_NB, n - 1 - j0);
