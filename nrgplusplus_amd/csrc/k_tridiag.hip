@@ -39,11 +39,35 @@ namespace nrgk {
 
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ double ht_wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// Sum over the wavefront, in every lane: DPP exchanges within 16 lanes, then swaps of 16- and 32-lane halves.  The
+// column launches wait for two of these in turn, and shuffles through LDS take three times as long.
+template <int CTRL>
+__device__ __forceinline__ double ht_dpp(double v) {
+  return __builtin_amdgcn_update_dpp(0.0, v, CTRL, 0xF, 0xF, false);
+}
+template <bool HALF>
+__device__ __forceinline__ double ht_swap_add(double v) {  // the two 32-lane halves (else 16-lane rows) added
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  if constexpr (HALF) {
+    const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false), b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+  } else {
+    const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false), b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+  }
+}
+__device__ __forceinline__ double ht_quad_sum(double v) {  // over aligned groups of four lanes
+  v += ht_dpp<0xB1>(v);
+  v += ht_dpp<0x4E>(v);
   return v;
 }
+__device__ __forceinline__ double ht_half_sum(double v) {  // over each half of the wavefront
+  v = ht_quad_sum(v);
+  v += ht_dpp<0x141>(v);
+  v += ht_dpp<0x140>(v);
+  return ht_swap_add<false>(v);
+}
+__device__ __forceinline__ double ht_wave_sum(double v) { return ht_swap_add<true>(ht_half_sum(v)); }
 
 // tiles of the lower triangle of the trailing matrix that starts at row/column s, and its tile-rows
 __host__ __device__ __forceinline__ int ht_rows(int T, int s) {
@@ -171,9 +195,6 @@ __device__ void ht_reflector_wave(const HtWs& w, int n, int T, int k, int lane, 
 // entry r of v_k (v[k+1] = 1, zero above) from the column's entry ur = u[r]
 __device__ __forceinline__ double ht_v_of(double ur, const HtRefl& R, int s, int n, int r) {
   return (r < s || r >= n) ? 0.0 : (r == s ? 1.0 : ur * R.sc);
-}
-__device__ __forceinline__ double ht_v(const double* u, const HtRefl& R, int s, int n, int r) {
-  return (r < s || r >= n) ? 0.0 : (r == s ? 1.0 : u[r] * R.sc);
 }
 
 // Every block's H (row-major, n x n, from the assembled blocks) into its working matrix's lower tiles
@@ -305,6 +326,17 @@ __global__ void __launch_bounds__(256) k_ht_symv(const HtBlock* __restrict__ bl,
   ht_rs_step<2, 0xB1>(a, (p & 1) != 0);
   ht_rs_step<1, 0x4E>(a, (p & 2) != 0);
   red[wv][lane >> 4][((p >> 3) << 3) | (((p >> 2) & 1) << 2) | ((p & 1) << 1) | ((p >> 1) & 1)] = a[0];
+  __builtin_amdgcn_sched_barrier(0);
+  // (a diagonal tile's rows of V and W for the shares below, lane: V or W, column j of the panel: asked for ahead
+  // of the barrier; before the products their registers would cost every tile two waves per SIMD)
+  const int j0 = (k / HT_NB) * HT_NB, cc = k - j0, arr = lane >> 5, pj = lane & 31;
+  double x[16];
+  if (diag && pj < cc)
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int r = r0 + i;
+      x[i] = r >= s && r < n ? (arr == 0 ? V[r * ld + j0 + pj] : w.W[(long long)r * HT_NB + pj]) : 0.0;
+    }
   __syncthreads();
   const long long ix = ht_tidx(I, J);
   double myv = 0.0;
@@ -325,26 +357,17 @@ __global__ void __launch_bounds__(256) k_ht_symv(const HtBlock* __restrict__ bl,
   if (tid == 0) w.sp[t] = sp2[0] + sp2[1];  // by tile index within the launch
   if (diag) {
     // this tile-row's shares of V^T v and W^T v over the panel's earlier columns: wave h sums rows
-    // 16 h .. 16 h + 15 (lane: V or W, column j; all sixteen loads at once), then the quarters in order
-    const int j0 = (k / HT_NB) * HT_NB, cc = k - j0;
-    const int arr = lane >> 5, j = lane & 31;
+    // 16 h .. 16 h + 15, then the quarters in order
     double acc = 0.0;
-    if (j < cc) {
-      double x[16];
+    if (pj < cc)
 #pragma unroll
-      for (int l = 0; l < 16; l++) {
-        const int r = I * HT_TB + wv * 16 + l;
-        x[l] = r >= s && r < n ? (arr == 0 ? V[r * ld + j0 + j] : w.W[(long long)r * HT_NB + j]) : 0.0;
-      }
-#pragma unroll
-      for (int l = 0; l < 16; l++) acc += x[l] * vr[wv * 16 + l];
-    }
+      for (int i = 0; i < 16; i++) acc += x[i] * vr[wv * 16 + i];
     cred[wv][lane] = acc;
     __syncthreads();
-    if (tid < 64 && j < cc) {
+    if (tid < 64 && pj < cc) {
       const double q = (cred[0][tid] + cred[1][tid]) + (cred[2][tid] + cred[3][tid]);
-      if (arr == 0) w.qv[I * HT_NB + j] = q;
-      else w.qw[I * HT_NB + j] = q;
+      if (arr == 0) w.qv[I * HT_NB + pj] = q;
+      else w.qw[I * HT_NB + pj] = q;
     }
   }
 }
@@ -366,20 +389,14 @@ __device__ __forceinline__ double ht_ypart(const HtWs& w, int T, int t0, int r, 
   }
   return y;
 }
-// V(r,:) W^T v + W(r,:) V^T v over the panel's cc earlier columns
-__device__ __forceinline__ double ht_corr(const HtWs& w, const double* V, long long ld, int j0, int cc,
-                                          const double* Vv, const double* Wv, int r) {
-  double corr = 0.0;
-#pragma unroll 8
-  for (int j = 0; j < cc; j++) corr += V[r * ld + j0 + j] * Wv[j] + w.W[(long long)r * HT_NB + j] * Vv[j];
-  return corr;
-}
-
 // One workgroup per 64-row tile-row of the trailing matrix: w(r) = tau (y(r) - V(r,:) W^T v -
 // W(r,:) V^T v) - (tau/2) (w^T v) v(r) for its rows, v and w stored, then the next column with the
-// panel corrections and its norm partial.  Threads 0..255 split each row's partial sums in quarters
-// (thread 4 q + h: row q, quarter h); threads 256..259 do the same for row k + 1, whose w every
-// workgroup needs, so its value is the same bits as the one its owner stores.
+// panel corrections and its norm partial.  Thread 4 q + h takes row q: a quarter of its partial sums and of its
+// panel columns (8 h .. 8 h + 7).  Row k + 1, whose w every workgroup needs, is done by every wave in the same
+// order (threads 256 .. 259 take its quarters), also in the workgroup that stores it, so all have the same bits.
+// A launch is one chain of memory and barrier latencies, so whatever the workgroup reads is asked for at once.
+// (Four blocks of ~1 080 rows: 8.4 -> 6.4 us; with the panel's rows read where they were used, twice, by one
+// thread a row, and four barriers before w.)
 __global__ void __launch_bounds__(320) k_ht_update(const HtBlock* __restrict__ bl, int nblk, const HtLaunch L, int k,
                                                    const double* __restrict__ Aa, double* __restrict__ Va,
                                                    double* __restrict__ Wa) {
@@ -397,12 +414,35 @@ __global__ void __launch_bounds__(320) k_ht_update(const HtBlock* __restrict__ b
   __shared__ HtRefl R;
   __shared__ double Vv[HT_NB], Wv[HT_NB];
   __shared__ double qpart[4][2][HT_NB];
-  __shared__ double sred[4];
-  __shared__ double ypart[4][HT_TB], yspart[4];
-  __shared__ double sh_wv, sh_w1;
+  __shared__ double sred[4], sqr[4];
+  __shared__ double yspart[4];
+  __shared__ double sh_vw;
   __shared__ double sh_ws[HT_NB], sh_vs[HT_NB];  // W(s, :) and V(s, j0 + :), the panel's row k + 1
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  if (wv == 4) ht_reflector_wave(w, n, T, k, lane, &R);
+  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63, q = tid >> 2, h = tid & 3;
+  const int r = I * HT_TB + q;
+  const bool own = tid < 256 && r < n && r >= s;
+  double vp[8], wp[8], ur = 0.0, ars = 0.0, y = 0.0;
+  if (own) {
+    const double *vrow = V + r * ld + j0 + 8 * h, *wrow = w.W + (long long)r * HT_NB + 8 * h;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const bool in = 8 * h + j < cc;
+      vp[j] = in ? vrow[j] : 0.0;
+      wp[j] = in ? wrow[j] : 0.0;
+    }
+    ur = u[r];
+    if (!pend) ars = A[ht_at(r, s)];
+  }
+  if (wv == 4) {
+    if (!pend) {
+      if (lane < 4) yspart[lane] = ht_ypart(w, T, t0, s, lane);
+      if (lane < HT_NB) {
+        sh_ws[lane] = lane < cc ? w.W[(long long)s * HT_NB + lane] : 0.0;
+        sh_vs[lane] = lane < cc ? V[s * ld + j0 + lane] : 0.0;
+      }
+    }
+    ht_reflector_wave(w, n, T, k, lane, &R);
+  }
   // v^T A v over the launch's tiles (partials by tile index): a fixed partition and order, the same in
   // every workgroup
   const int m = T - t0, NTa = m * (m + 1) / 2;
@@ -415,10 +455,8 @@ __global__ void __launch_bounds__(320) k_ht_update(const HtBlock* __restrict__ b
 #pragma unroll
       for (int j = 0; j < 8; j++) acc += x[j];
     }
-    acc = ht_wave_sum(acc);
-    if (lane == 0) sred[wv] = acc;
     // the panel's V^T v and W^T v: thread 4 p + h sums quarter h of the tile-rows of pair p
-    const int pr = tid >> 2, h = tid & 3, arr = pr >> 5, j = pr & 31;
+    const int arr = q >> 5, j = q & 31;
     if (j < cc) {
       const double* src = arr == 0 ? w.qv : w.qw;
       double a = 0.0;
@@ -435,69 +473,65 @@ __global__ void __launch_bounds__(320) k_ht_update(const HtBlock* __restrict__ b
       qpart[h][arr][j] = a;
     }
     // the partial sums of this workgroup's rows
-    const int r = I * HT_TB + pr;
-    ypart[h][pr] = r < n && r >= s ? ht_ypart(w, T, t0, r, h) : 0.0;
-  } else if (tid < 260 && !pend) {
-    yspart[tid - 256] = ht_ypart(w, T, t0, s, tid - 256);
+    if (own) y = ht_ypart(w, T, t0, r, h);
+    acc = ht_wave_sum(acc);
+    if (lane == 0) sred[wv] = acc;
+    y = ht_quad_sum(y);
   }
   __syncthreads();
-  if (tid < 2 * HT_NB) {
+  if (tid < 64) {  // lanes 0 .. 31: V^T v, 32 .. 63: W^T v
     const int arr = tid >> 5, j = tid & 31;
-    if (j < cc) {
-      const double a = (qpart[0][arr][j] + qpart[1][arr][j]) + (qpart[2][arr][j] + qpart[3][arr][j]);
-      if (arr == 0) Vv[j] = a;
-      else Wv[j] = a;
-    }
-  } else if (tid < 2 * HT_NB + HT_NB && !pend) {
-    const int j = tid - 2 * HT_NB;
-    if (j < cc) {
-      sh_ws[j] = w.W[(long long)s * HT_NB + j];
-      sh_vs[j] = V[s * ld + j0 + j];
-    }
+    const double a = j < cc ? (qpart[0][arr][j] + qpart[1][arr][j]) + (qpart[2][arr][j] + qpart[3][arr][j]) : 0.0;
+    if (arr == 0) Vv[j] = a;
+    else Wv[j] = a;
+    const double vw = ht_half_sum(a * __shfl_xor(a, 32, 64));
+    if (tid == 0) sh_vw = vw;
   }
   __syncthreads();
-  if (tid == 0) {
-    double vw = 0.0;
-    for (int j = 0; j < cc; j++) vw += Vv[j] * Wv[j];
-    sh_wv = R.tau * ((sred[0] + sred[1]) + (sred[2] + sred[3]) - 2.0 * vw);
+  if (tid >= 256) return;
+  const double wvs = R.tau * ((sred[0] + sred[1]) + (sred[2] + sred[3]) - 2.0 * sh_vw);
+  double w1 = 0.0;
+  if (!pend) {
+    const int j = lane & 31;
+    const double c = ht_half_sum(sh_vs[j] * Wv[j] + sh_ws[j] * Vv[j]);
+    w1 = R.tau * (((yspart[0] + yspart[1]) + (yspart[2] + yspart[3])) - c) - 0.5 * R.tau * wvs;  // (v(s) = 1)
   }
-  __syncthreads();
-  const double wvs = sh_wv;
-  const int r = I * HT_TB + tid;
-  double wr = 0.0, vrr = 0.0;
-  const bool own = tid < 64 && r < n && r >= s;
+  double corr = 0.0, next = 0.0;
+  if (own)
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      corr += vp[j] * Wv[8 * h + j] + wp[j] * Vv[8 * h + j];
+      if (!pend) next += vp[j] * sh_ws[8 * h + j] + wp[j] * sh_vs[8 * h + j];
+    }
+  corr = ht_quad_sum(corr);
+  next = ht_quad_sum(next);
+  double sq = 0.0;
   if (own) {
-    const double y = (ypart[0][tid] + ypart[1][tid]) + (ypart[2][tid] + ypart[3][tid]);
-    vrr = ht_v(u, R, s, n, r);
-    wr = R.tau * (y - ht_corr(w, V, ld, j0, cc, Vv, Wv, r)) - 0.5 * R.tau * wvs * vrr;
-    w.W[(long long)r * HT_NB + cc] = wr;
-    V[r * ld + k] = vrr;
-  } else if (tid == 256 && !pend) {
-    const double y = (yspart[0] + yspart[1]) + (yspart[2] + yspart[3]);
-    sh_w1 = R.tau * (y - ht_corr(w, V, ld, j0, cc, Vv, Wv, s)) - 0.5 * R.tau * wvs * 1.0;
+    const double vrr = ht_v_of(ur, R, s, n, r);
+    double wr = R.tau * (y - corr) - 0.5 * R.tau * wvs * vrr;
+    if (!pend && r == s) wr = w1;
+    // the next column (k + 1 = s) with the panel's corrections, its diagonal entry and norm partial; column
+    // k's is V(r, k) W(s, k) + W(r, k) V(s, k), V(s, k) = 1
+    const double un = ars - next - (vrr * w1 + wr);
+    if (h == 0) {
+      w.W[(long long)r * HT_NB + cc] = wr;
+      V[r * ld + k] = vrr;
+      if (!pend) {
+        if (r == s) w.d[s] = un;
+        else w.u[(long long)(s & 1) * n + r] = un;
+        if (r >= s + 2) sq = un * un;
+      }
+    }
   }
   if (t == 0 && tid == 0) {
     w.tau[k] = R.tau;
     w.e[k] = R.beta;
   }
-  __syncthreads();
   if (pend) return;
-  // the next column (k + 1 = s) with the panel's corrections, its diagonal entry and norm partial
-  const double w1 = sh_w1;
-  double sq = 0.0;
-  if (own) {
-    double un = A[ht_at(r, s)];
-#pragma unroll 8
-    for (int j = 0; j < cc; j++) un -= V[r * ld + j0 + j] * sh_ws[j] + w.W[(long long)r * HT_NB + j] * sh_vs[j];
-    un -= vrr * w1 + wr;  // column k: V(r, k) W(s, k) + W(r, k) V(s, k), V(s, k) = 1
-    if (r == s) w.d[s] = un;
-    else w.u[(long long)(s & 1) * n + r] = un;
-    if (r >= s + 2) sq = un * un;
-  }
-  if (tid < 64) {
-    sq = ht_wave_sum(sq);
-    if (tid == 0) w.ss[(long long)(s & 1) * T + I] = sq;
-  }
+  sq = ht_wave_sum(sq);
+  if (lane == 0) sqr[wv] = sq;
+  __syncthreads();
+  if (tid == 0) w.ss[(long long)(s & 1) * T + I] = (sqr[0] + sqr[1]) + (sqr[2] + sqr[3]);
 }
 
 // Rank-2k update of the trailing lower triangle (rows and columns >= s = k + 1) at the end of a panel:
