@@ -122,8 +122,8 @@ Chain::Chain(Ctx* c, int mode_) : ctx(c), mode(mode_) { init_device(); }
 void Chain::init_device() {
   NRGK_REQUIRE(mode == NRGK_MODE_MIXED || mode == NRGK_MODE_PLAIN64, NRGK_ERR_INVALID, "nrgk: unknown mode");
   for (DevBuf* b : {&eprev_own, &fbuf[0], &fbuf[1], &d_bathE, &d_bathF, &dH, &dX, &dX2, &d_oa, &dU,
-                    &dY, &dC, &dlam_tmp, &dlam_raw, &dlam_prev, &dlam_shift[0], &dlam_shift[1], &d_eig, &d_stats, &d_kept,
-                    &d_trunc, &d_eig_act, &d_rrv, &d_cid, &d_sidx, &d_mid_A, &d_mid_tau, &d_mid_ws, &d_mid_q, &d_ht,
+                    &dY, &dC, &dlam_tmp, &dlam_raw, &dlam_prev, &dlam_shift[0], &dlam_shift[1], &d_stats, &d_kept,
+                    &d_trunc, &d_rrv, &d_cid, &d_sidx, &d_mid_A, &d_mid_tau, &d_mid_ws, &d_mid_q, &d_ht,
                     &d_wide_ws, &d_wide_s, &d_wide_q, &d_wide_A, &d_wide_V})
     b->ctx = ctx, b->retired = &retired;
   for (DevBuf& b : d_big_work) b.ctx = ctx, b.retired = &retired;
@@ -509,17 +509,20 @@ void Chain::run_gemms(std::vector<GemmProb>& probs) {
   }
   if (live.empty()) return;
   const int tiles = prepare_gemm(live);
-  const GemmProb* dprobs = stg.put(live, st);
+  launch_products(live, stg.put(live, st), tiles);
+}
+
+void Chain::launch_products(const std::vector<GemmProb>& probs, const GemmProb* d, int tiles) {
   double fl = 0, by = 0;
   if (prof_on)
-    for (auto& p : live) {
+    for (auto& p : probs) {
       // a symmetric product computes (and counts) the n (n + 1) / 2 entries on and above the diagonal
       const double outs = p.sym ? 0.5 * (double)p.m * (p.m + 1) : (double)p.m * p.n;
       fl += 2.0 * outs * p.k;
       by += 8.0 * ((double)p.m * p.k + (double)p.k * p.n + (p.C0 ? 2.0 : 1.0) * outs);
     }
   prof_begin("gemm_f64");
-  launch_gemm(dprobs, (int)live.size(), tiles, st);
+  launch_gemm(d, (int)probs.size(), tiles, st);
   prof_end("gemm_f64", 1, fl, by);
 }
 
@@ -636,7 +639,6 @@ void Chain::eigensolve_mixed() {
   }
   int nmax_m = 1;  // widest block of the batched solve (LDS sizes)
   for (auto& b : blks) nmax_m = std::max(nmax_m, b.n);
-  const EigBlock* dblk = upload_to(d_eig, blks.data(), nb);
   // ---- FP32 stage (k_mid.hip): every block's start vectors in a dozen launches, widest blocks first
   // (each is one workgroup's work in the reduction)
   const size_t bytes64 = std::max<long long>(1, tot_elems) * sizeof(double);
@@ -707,15 +709,6 @@ void Chain::eigensolve_mixed() {
     launch_mid_back(dm, mid, V, d_mid_tau.as<float>(), V + vo, dX.as<double>(), st);
     prof_end("mid_back", 2, 1.5 * fl, 0.0);
   }
-  // 32 x 32 tiles of every block, for the gather into U
-  std::vector<int4> tiles_blk;
-  for (int bi = 0; bi < nb; bi++) {
-    const int T = (blks[bi].n + 31) / 32;
-    for (int ti = 0; ti < T; ti++)
-      for (int tj = 0; tj < T; tj++) tiles_blk.push_back(int4{bi, ti, tj, 0});
-  }
-  const size_t n_tiles_blk = tiles_blk.size();
-  const int4* d_tiles_blk = upload_to(d_eig_act, tiles_blk.data(), tiles_blk.size());
   // NRGK_DEBUG_FINITE=1: the first stage and block that produces a non-finite value fail the call
   // with NRGK_ERR_NOCONV (the stage and block are in the message)
   const bool dbg = knob("NRGK_DEBUG_FINITE", 0) != 0;
@@ -751,6 +744,7 @@ void Chain::eigensolve_mixed() {
   const int dbg_oa = (int)knob("NRGK_DEBUG_OA", 0);
   std::vector<EigBlock> act = blks;
   oa_steps = 0;
+  bool asked = false;
   for (int it = 0; it < oa_max && !act.empty(); it++) {
     const int na = (int)act.size();
     // 32 x 32 tiles of the active blocks: all of them, and the (i <= j) half for the symmetrisation
@@ -763,15 +757,6 @@ void Chain::eigensolve_mixed() {
           if (ti <= tj) tiles_sym.push_back(int4{a, ti, tj, 0});
         }
     }
-    Staging::Region rg = stg.open(Staging::span<EigBlock>(act.size()) + Staging::span<int4>(tiles_all.size()) +
-                                  Staging::span<int4>(tiles_sym.size()) + Staging::span<double>(4 * na) +
-                                  Staging::span<double>(na));
-    const EigBlock* m_blk = stg.place(rg, act);
-    const int4* m_all = stg.place(rg, tiles_all);
-    const int4* m_sym = stg.place(rg, tiles_sym);
-    double* m_conv = stg.place_zero<double>(rg, 4 * na);
-    double* m_offmax = stg.place_zero<double>(rg, na);
-    stg.commit(rg, st);
     std::vector<GemmProb> g1, g2, g3;
     for (auto& b : act) {
       const int n = b.n;
@@ -787,8 +772,23 @@ void Chain::eigensolve_mixed() {
       g2.push_back(GemmProb{X, P, nullptr, Sm, n, n, n, n, n, n, n, 1, 0, 1.0, 0.0, 0, 0, 1});
       g3.push_back(GemmProb{X, E, X, X2, n, n, n, n, n, n, n, 0, 0, 1.0, 1.0, 0, 0});
     }
-    run_gemms(g1);
-    run_gemms(g2);
+    const int t1 = prepare_gemm(g1), t2 = prepare_gemm(g2), t3 = prepare_gemm(g3);
+    // everything the step's launches read from the host in one copy (a copy is a launch of its own, 4 us)
+    Staging::Region rg = stg.open(Staging::span<EigBlock>(act.size()) + Staging::span<int4>(tiles_all.size()) +
+                                  Staging::span<int4>(tiles_sym.size()) + Staging::span<double>(4 * na) +
+                                  Staging::span<double>(na) + Staging::span<GemmProb>(g1.size()) +
+                                  Staging::span<GemmProb>(g2.size()) + Staging::span<GemmProb>(g3.size()));
+    const EigBlock* m_blk = stg.place(rg, act);
+    const int4* m_all = stg.place(rg, tiles_all);
+    const int4* m_sym = stg.place(rg, tiles_sym);
+    double* m_conv = stg.place_zero<double>(rg, 4 * na);
+    double* m_offmax = stg.place_zero<double>(rg, na);
+    const GemmProb* m_g1 = stg.place(rg, g1);
+    const GemmProb* m_g2 = stg.place(rg, g2);
+    const GemmProb* m_g3 = stg.place(rg, g3);
+    stg.commit(rg, st);
+    launch_products(g1, m_g1, t1);
+    launch_products(g2, m_g2, t2);
     check("P=HX", dP, false);
     check("S=X^T P", dS, false);
     check("R=X^T X", dR, false);
@@ -805,14 +805,19 @@ void Chain::eigensolve_mixed() {
     prof_end("oa_update", 5, 0.0, oa_bytes);
     check("oa_update (E)", dE, false);
     check("oa_update (lam)", dlam_tmp.as<double>(), true);
-    const double* h_conv = stg.get(m_conv, 4 * na, st);
-    run_gemms(g3);
-    sync();
-    if (it == 0) small_done();
-    const std::vector<double> conv(h_conv, h_conv + 4 * na);
+    // The FP32 start vectors are never at the first step's stopping point (blocks that need no step, diagonal ones say,
+    // are, and take a second that leaves them where they are), so its result is not waited for.
+    const bool ask = it > 0 || oa_max == 1 || dbg_oa > 0;
+    const double* h_conv = ask ? stg.get(m_conv, 4 * na, st) : nullptr;
+    launch_products(g3, m_g3, t3);
+    if (ask) sync();
     std::swap(dX, dX2);
     check("X+XE", dX.as<double>(), false);
     oa_steps = it + 1;
+    if (!ask) continue;
+    if (!asked) small_done();
+    asked = true;
+    const std::vector<double> conv(h_conv, h_conv + 4 * na);
     std::vector<EigBlock> next;
     for (int a = 0; a < na; a++) {
       // NRGK_DEBUG_OA=n: per step, the residual (in noise units) and orthogonality defect of every
@@ -829,12 +834,24 @@ void Chain::eigensolve_mixed() {
                         (double)act[a].n * rot * rot <= d_tol;
       if (!last && !pred) next.push_back(act[a]);
     }
-    // the finished blocks' vectors into both iterate buffers (the device applies the same test)
-    if (next.size() < act.size())
+    // the finished blocks' vectors into both iterate buffers, if there is another step (the device applies the
+    // same test)
+    if (!next.empty() && next.size() < act.size())
       launch_copy_converged(m_blk, na, m_conv, e_tol, d_tol, e_pred, d_pred, dX.as<double>(), dX2.as<double>(), st);
     act.swap(next);
   }
-  launch_final_sort(dblk, nb, d_tiles_blk, (int)n_tiles_blk, dX.as<double>(), dlam_tmp.as<double>(),
+  // 32 x 32 tiles of every block, for the gather into U
+  std::vector<int4> tiles_blk;
+  for (int bi = 0; bi < nb; bi++) {
+    const int T = (blks[bi].n + 31) / 32;
+    for (int ti = 0; ti < T; ti++)
+      for (int tj = 0; tj < T; tj++) tiles_blk.push_back(int4{bi, ti, tj, 0});
+  }
+  Staging::Region rg = stg.open(Staging::span<EigBlock>(blks.size()) + Staging::span<int4>(tiles_blk.size()));
+  const EigBlock* dblk = stg.place(rg, blks);
+  const int4* d_tiles_blk = stg.place(rg, tiles_blk);
+  stg.commit(rg, st);
+  launch_final_sort(dblk, nb, d_tiles_blk, (int)tiles_blk.size(), dX.as<double>(), dlam_tmp.as<double>(),
                     dU.as<double>(), dlam_raw.as<double>(), d_sidx.as<int>(), final_sort_lds(nmax_m), st);
   const int* hs = stg.get(d_stats.as<int>(), 4, st);
   large_blocks_join(*this);

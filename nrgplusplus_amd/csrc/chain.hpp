@@ -140,7 +140,7 @@ struct Chain {
   DevBuf dH, dX, dX2, d_oa, dU, dY, dC, d_rrv;
   DevBuf dlam_tmp, dlam_raw, dlam_shift[2];
   int lcur = 0;
-  DevBuf d_eig, d_stats, d_kept, d_trunc, d_eig_act, d_cid, d_sidx;
+  DevBuf d_stats, d_kept, d_trunc, d_cid, d_sidx;
   // FP32 stage (k_mid.hip): working matrices, tau, T's workspaces, cluster list
   DevBuf d_mid_A, d_mid_tau, d_mid_ws, d_mid_q;
   int oa_steps = 0, oa_unconverged = 0;
@@ -265,6 +265,8 @@ struct Chain {
   void set_state(const nrgk_site_desc* st, int cnt);
   void ensure_all_eig();
   void run_gemms(std::vector<GemmProb>& probs);
+  // one launch of the batched kernel over prepared problems, d their copy on the device
+  void launch_products(const std::vector<GemmProb>& probs, const GemmProb* d, int tiles);
 
  private:
   void init_device();
