@@ -697,7 +697,8 @@ __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __res
 
 // The WY factor of panel p of each block: T_p upper triangular with H_{j0} .. H_{j0+nb-1} =
 // I - V_p T_p V_p^T (forward, columnwise); V_p T_p goes to VT beside V (columns of zeros past the last
-// reflector).
+// reflector).  The Gram matrix on the matrix cores, T a row to a thread, V T a row to a thread: a chain of two barriers
+// (16 chains of blocks of up to 190 rows: 25 -> 12.5 us).
 __global__ void __launch_bounds__(256) k_mid_larft(const MidBlock* __restrict__ bl, int nblk,
                                                    const float* __restrict__ Va, const float* __restrict__ taua,
                                                    float* __restrict__ VTa) {
@@ -708,37 +709,44 @@ __global__ void __launch_bounds__(256) k_mid_larft(const MidBlock* __restrict__ 
   const int n = B.n, ldv = 16 * md_strips(n), j0 = g * MD_NB, nb = min(MD_NB, n - 1 - j0);
   const float* V = Va + B.v_off + (long long)j0 * ldv;
   float* VT = VTa + B.v_off + (long long)j0 * ldv;
-  __shared__ float St[MD_NB][65], G[MD_NB][MD_NB + 1], T[MD_NB][MD_NB + 1];
-  const int tid = threadIdx.x, a = tid >> 4, c = tid & 15;
-  float acc = 0.0f;
-  for (int r0 = j0; r0 < ldv; r0 += 64) {
-    for (int e = tid; e < MD_NB * 64; e += 256) {
-      const int j = e >> 6, r = r0 + (e & 63);
-      St[j][e & 63] = j < nb && r < ldv ? V[(long long)j * ldv + r] : 0.0f;
-    }
-    __syncthreads();
-    for (int q = 0; q < 64; q++) acc += St[a][q] * St[c][q];
-    __syncthreads();
+  __shared__ float G[4][MD_NB][MD_NB], T[MD_NB][MD_NB + 1], tau[MD_NB];
+  const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
+  if (tid < nb) tau[tid] = taua[B.e_off + j0 + tid];
+  // G = V^T V: a wave takes every fourth piece of 16 rows, lane (lk, li) rows 4 lk .. + 3 of it, column li
+  flt4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int r0 = j0 + 16 * wv; r0 < ldv; r0 += 64) {
+    flt4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (li < nb) v = *reinterpret_cast<const flt4*>(V + (long long)li * ldv + r0 + 4 * lk);
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], v[i], acc, 0, 0, 0);
   }
-  G[a][c] = acc;
-  T[a][c] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; i++) G[wv][4 * lk + i][li] = acc[i];
   __syncthreads();
-  for (int i = 0; i < nb; i++) {
-    const float ti = taua[B.e_off + j0 + i];
-    float x = 0.0f;
-    if (tid < i)
-      for (int q = tid; q < i; q++) x += T[tid][q] * G[q][i];
-    __syncthreads();
-    if (tid < i) T[tid][i] = -ti * x;
-    if (tid == i) T[i][i] = ti;
-    __syncthreads();
+  if (tid < MD_NB) {  // a thread per row of T, which needs no other row
+    float t[MD_NB];
+#pragma unroll
+    for (int i = 0; i < MD_NB; i++) {
+      float x = 0.0f;
+#pragma unroll
+      for (int q = 0; q < MD_NB; q++)
+        if (q < i) x += t[q] * ((G[0][q][i] + G[1][q][i]) + (G[2][q][i] + G[3][q][i]));
+      t[i] = i >= nb || tid > i ? 0.0f : tid == i ? tau[i] : -tau[i] * x;
+      T[tid][i] = t[i];
+    }
   }
-  for (int e = tid; e < MD_NB * ldv; e += 256) {
-    const int j = e / ldv, r = e - j * ldv;
-    float x = 0.0f;
-    if (r > j0)
-      for (int i = 0; i <= min(j, nb - 1); i++) x += V[(long long)i * ldv + r] * T[i][j];
-    if (j0 + j < ldv) VT[(long long)j * ldv + r] = x;
+  __syncthreads();
+  for (int r = tid; r < ldv; r += 256) {
+    float v[MD_NB];
+#pragma unroll
+    for (int q = 0; q < MD_NB; q++) v[q] = q < nb && r > j0 ? V[(long long)q * ldv + r] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < MD_NB; q++) {
+      float x = 0.0f;
+#pragma unroll
+      for (int a = 0; a <= q; a++) x += v[a] * T[a][q];
+      if (j0 + q < ldv) VT[(long long)q * ldv + r] = x;
+    }
   }
 }
 
