@@ -745,10 +745,12 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
 
 // deterministic start vector entries in [-1, 1)
 __device__ __forceinline__ double ht_start(unsigned p, unsigned i) {
-  unsigned x = p * 0x9E3779B9u ^ (i + 1u) * 0x85EBCA6Bu;
+  unsigned x = p << 16 ^ i;  // (both below 2^16)
   x ^= x >> 16;
   x *= 0x7FEB352Du;
   x ^= x >> 15;
+  x *= 0x846CA68Bu;
+  x ^= x >> 16;
   return (double)(int)x * (1.0 / 2147483648.0);
 }
 
