@@ -743,15 +743,15 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
   if (mine && ln == 0) lam[B.e_off + j] = ldexp(0.5 * (a + c), ex);
 }
 
-// deterministic start vector entries in [-1, 1)
+// deterministic start vector entries in [-1, 1), none of them zero (a block of one row has but one)
 __device__ __forceinline__ double ht_start(unsigned p, unsigned i) {
-  unsigned x = p << 16 ^ i;  // (both below 2^16)
+  unsigned x = (p << 16 ^ i) + 0x9E3779B9u;  // (both below 2^16)
   x ^= x >> 16;
   x *= 0x7FEB352Du;
   x ^= x >> 15;
   x *= 0x846CA68Bu;
   x ^= x >> 16;
-  return (double)(int)x * (1.0 / 2147483648.0);
+  return (double)(int)(x | 1u) * (1.0 / 2147483648.0);
 }
 
 // Rows per register tile of the column loops below: each tile's loads are issued together, so a
