@@ -67,8 +67,8 @@ struct Ctx;
 // it (one request of the server, one eigh call, one of the chains of a z-average), and hipMalloc, hipFree and
 // hipHostMalloc each wait for the whole device: 16 chains at K = 512 spent 25 ms growing their buffers in the
 // first sites and 54 ms giving them back, of 187 ms.  Memory is given here only when no stream uses it any
-// more.  Bounded: beyond `limit` bytes memory is freed; what is held is freed when an allocation
-// fails or would take the context past its capacity, when the capacity is set, and with the context.
+// more.  Bounded: beyond `limit` bytes what has lain idle longest is freed; all that is held is freed when an
+// allocation fails or would take the context past its capacity, when the capacity is set, and with the context.
 class MemPool {
  public:
   size_t limit = 0;         // device bytes held at most
@@ -88,21 +88,31 @@ class MemPool {
     std::lock_guard<std::mutex> lk(m_);
     auto it = dev_.find(size);
     if (it == dev_.end()) return nullptr;
-    void* p = it->second;
+    void* p = it->second.p;
     dev_.erase(it);
     held_ -= size;
     return p;
   }
   void give(void* p, size_t size) {
+    std::vector<void*> out;  // freed outside of the lock
     {
       std::lock_guard<std::mutex> lk(m_);
+      while (size <= limit && held_ + size > limit && !dev_.empty()) {
+        auto old = dev_.begin();
+        for (auto it = dev_.begin(); it != dev_.end(); ++it)
+          if (it->second.since < old->second.since) old = it;
+        out.push_back(old->second.p);
+        held_ -= old->first;
+        dev_.erase(old);
+      }
       if (held_ + size <= limit) {
-        dev_.emplace(size, p);
+        dev_.emplace(size, Idle{p, clock_++});
         held_ += size;
-        return;
+      } else {
+        out.push_back(p);
       }
     }
-    (void)hipFree(p);
+    for (void* q : out) (void)hipFree(q);
   }
   std::pair<char*, char*> take_staging(size_t size) {
     std::lock_guard<std::mutex> lk(m_);
@@ -129,7 +139,7 @@ class MemPool {
   }
   size_t held() const { return held_; }
   void trim() {
-    std::multimap<size_t, void*> d;
+    std::multimap<size_t, Idle> d;
     std::multimap<size_t, std::pair<char*, char*>> s;
     {
       std::lock_guard<std::mutex> lk(m_);
@@ -138,7 +148,7 @@ class MemPool {
       held_ = 0;
       host_held_ = 0;
     }
-    for (auto& e : d) (void)hipFree(e.second);
+    for (auto& e : d) (void)hipFree(e.second.p);
     for (auto& e : s) {
       (void)hipHostFree(e.second.first);
       (void)hipFree(e.second.second);
@@ -146,8 +156,13 @@ class MemPool {
   }
 
  private:
+  struct Idle {
+    void* p;
+    unsigned long long since;
+  };
   std::mutex m_;
-  std::multimap<size_t, void*> dev_;
+  std::multimap<size_t, Idle> dev_;
+  unsigned long long clock_ = 0;
   std::multimap<size_t, std::pair<char*, char*>> staging_;
   std::atomic<size_t> held_{0}, host_held_{0};
 };
