@@ -704,7 +704,7 @@ void Chain::eigensolve_mixed() {
     launch_ht_sturm(dht, mht, W, dlam_tmp.as<double>(), 1e-11, st);
     launch_ht_stein(dht, mht, W, dlam_tmp.as<double>(), dX.as<double>(), scr, 1e-6, 1,
                     d_mid_q.as<int>() + 64, d_mid_q.as<int>(), st);
-    prof_end("mid_tridiag", 7, 0.0, 0.0);
+    prof_end("mid_tridiag", 5, 0.0, 0.0);
     prof_begin("mid_back");
     launch_mid_back(dm, mid, V, d_mid_tau.as<float>(), V + vo, dX.as<double>(), st);
     prof_end("mid_back", 2, 1.5 * fl, 0.0);
