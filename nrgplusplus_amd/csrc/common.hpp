@@ -535,7 +535,7 @@ struct MidBlock {
   int e_off;        // offset of the block's tau (prefix of n)
 };
 
-// Wide-block eigensolver (k_tridiag.hip): blocked Householder tridiagonalisation in FP64, bisection
+// Wide-block eigensolver (k_tridiag.hip): blocked Householder tridiagonalisation in FP64, multisection
 // for the eigenvalues, inverse iteration for the eigenvectors, WY back-transformation.  All n x n
 // arenas of a block share the block's element offset a_off (row-major, leading dimension n):
 //   A    working copy of H; the lower triangle is reduced in place; later the V T products

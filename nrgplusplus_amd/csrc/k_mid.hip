@@ -6,7 +6,7 @@
 //   k_ht_sturm    eigenvalues of T (FP64, multisection)
 //   k_ht_stein_*  eigenvectors of T (FP64 inverse iteration, clusters orthonormalised; k_tridiag.hip)
 //   k_mid_larft   the WY factors V_p T_p, a workgroup per panel
-//   k_mid_back    X = Q Z, a workgroup per 64 columns, every panel in one launch
+//   k_mid_back    X = Q Z, a workgroup per 32 columns, every panel in one launch
 //
 // The whole sequence takes a dozen launches whatever the block widths; the one-sided block Jacobi it
 // replaces took n/16 dependent launches per sweep and nine sweeps for the widest blocks.
@@ -750,21 +750,22 @@ __global__ void __launch_bounds__(256) k_mid_larft(const MidBlock* __restrict__ 
   }
 }
 
-// X = Q Z for 64 columns of one block: Z (FP64, the eigenvectors of T) in the matrix-core layout in
-// registers (wave w: row tiles w, w + 16, w + 32), the panels applied last first, Z -= (V_p T_p) (V_p^T Z).
+// X = Q Z for 32 columns of one block: Z (FP64, the eigenvectors of T) in the matrix-core layout in
+// registers (wave w: row tiles w, w + MB_WAVES, ..), the panels applied last first, Z -= (V_p T_p) (V_p^T Z).
 // Register r of a 16 x 16 piece holds rows 4 (l/16) + r of it, which is the right-hand operand of a
 // 4-row step over those rows as it stands, so Z never leaves the registers; each wave's share of
-// V_p^T Z meets the others' in LDS.
-constexpr int MB_THREADS = 1024;
-constexpr int MB_WAVES = MB_THREADS / 64;
-constexpr int MB_RT = MD_MAX / 16 / MB_WAVES;
-__global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restrict__ bl, int nblk,
-                                                         const float* __restrict__ Va, const float* __restrict__ VTa,
-                                                         double* __restrict__ Xa) {
-  __shared__ float Yp[MB_WAVES][MD_NB][64];
-  __shared__ float Ys[MD_NB][80];
+// V_p^T Z meets the others' in LDS.  Two barriers a panel and, before they were asked for ahead, two waits for
+// memory: blocks of up to 360 rows (8 waves) 98 -> 47 us, of up to 620 (16 waves) 234 -> 129 us.  32 columns to a
+// workgroup leave registers for that; 64 would spill.
+constexpr int MB_CT = 2;
+template <int MB_WAVES, int MB_RT>
+__global__ void __launch_bounds__(64 * MB_WAVES) k_mid_back(const MidBlock* __restrict__ bl, int nblk,
+                                                            const float* __restrict__ Va, const float* __restrict__ VTa,
+                                                            double* __restrict__ Xa) {
+  __shared__ float Yp[MB_WAVES][MD_NB][16 * MB_CT];
+  __shared__ float Ys[MD_NB][16 * MB_CT + 16];
   int g = blockIdx.x;
-  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n + 63) / 64; });
+  const int b = find_task(nblk, g, [&](int i) { return (bl[i].n + 16 * MB_CT - 1) / (16 * MB_CT); });
   if (b < 0) return;
   const MidBlock B = bl[b];
   const int n = B.n, ldv = 16 * md_strips(n), NT = ldv / 16;
@@ -772,42 +773,61 @@ __global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restr
   const float* VT = VTa + B.v_off;
   double* X = Xa + B.h_off;
   const int tid = threadIdx.x, wv = tid >> 6, l = tid & 63, li = l & 15, lk = l >> 4;
-  flt4 z[MB_RT][4];
+  flt4 z[MB_RT][MB_CT];
 #pragma unroll
   for (int q = 0; q < MB_RT; q++)
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++)
+    for (int ct = 0; ct < MB_CT; ct++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 64 * g + 16 * ct + li;
+        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 16 * MB_CT * g + 16 * ct + li;
         z[q][ct][r] = row < n && col < n ? (float)X[(long long)row * n + col] : 0.0f;
       }
-  for (int p = n > 1 ? (n - 2) / MD_NB : -1; p >= 0; p--) {
-    const int j0 = p * MD_NB;  // panel column j0 + j beyond n - 2 has no reflector: V T is zero there
-    flt4 y[4];
+  // panel p's V and V T for this wave's row tiles: V a panel ahead, V T ahead of the panel's barriers, without
+  // conditions (a tile or column that is not there repeats another and is left out where it would be used)
+  flt4 av[MB_RT];
+  auto load_v = [&](int p) {
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++) y[ct] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int q = 0; q < MB_RT; q++)
+      av[q] = *reinterpret_cast<const flt4*>(V + (long long)min(p * MD_NB + li, n - 1) * ldv +
+                                             16 * min(wv + MB_WAVES * q, NT - 1) + 4 * lk);
+  };
+  const int p0 = n > 1 ? (n - 2) / MD_NB : -1;
+  if (p0 >= 0) load_v(p0);
+  for (int p = p0; p >= 0; p--) {
+    const int j0 = p * MD_NB;  // panel column j0 + j beyond n - 2 has no reflector: V T is zero there
+    float at[MB_RT][4];
+#pragma unroll
+    for (int q = 0; q < MB_RT; q++)
+#pragma unroll
+      for (int ks = 0; ks < 4; ks++)
+        at[q][ks] = VT[(long long)min(j0 + 4 * ks + lk, ldv - 1) * ldv + 16 * min(wv + MB_WAVES * q, NT - 1) + li];
+    flt4 y[MB_CT];
+#pragma unroll
+    for (int ct = 0; ct < MB_CT; ct++) y[ct] = flt4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int q = 0; q < MB_RT; q++) {
       const int rt = wv + MB_WAVES * q;
       if (rt < p || rt >= NT) continue;
-      flt4 a = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (j0 + li < n - 1) a = *reinterpret_cast<const flt4*>(V + (long long)(j0 + li) * ldv + 16 * rt + 4 * lk);
+#pragma unroll
+      for (int r = 0; r < 4; r++) av[q][r] = j0 + li < n - 1 ? av[q][r] : 0.0f;
 #pragma unroll
       for (int r = 0; r < 4; r++)
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++) y[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[r], z[q][ct][r], y[ct], 0, 0, 0);
+        for (int ct = 0; ct < MB_CT; ct++) y[ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[q][r], z[q][ct][r], y[ct], 0, 0, 0);
     }
+    load_v(max(p - 1, 0));
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++)
+    for (int ct = 0; ct < MB_CT; ct++)
 #pragma unroll
       for (int r = 0; r < 4; r++) Yp[wv][4 * lk + r][16 * ct + li] = y[ct][r];
     __syncthreads();
-    {
+    for (int e = tid; e < MD_NB * 16 * MB_CT; e += 64 * MB_WAVES) {
+      const int j = e / (16 * MB_CT), q = e % (16 * MB_CT);
       float acc = 0.0f;
 #pragma unroll
-      for (int w = 0; w < MB_WAVES; w++) acc += Yp[w][tid >> 6][l];
-      Ys[tid >> 6][l] = acc;
+      for (int w = 0; w < MB_WAVES; w++) acc += Yp[w][j][q];
+      Ys[j][q] = acc;
     }
     __syncthreads();
 #pragma unroll
@@ -817,9 +837,9 @@ __global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restr
 #pragma unroll
       for (int ks = 0; ks < 4; ks++) {
         const int j = 4 * ks + lk;
-        const float a = j0 + j < ldv ? -VT[(long long)(j0 + j) * ldv + 16 * rt + li] : 0.0f;
+        const float a = j0 + j < ldv ? -at[q][ks] : 0.0f;
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++)
+        for (int ct = 0; ct < MB_CT; ct++)
           z[q][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Ys[j][16 * ct + li], z[q][ct], 0, 0, 0);
       }
     }
@@ -827,10 +847,10 @@ __global__ void __launch_bounds__(MB_THREADS) k_mid_back(const MidBlock* __restr
 #pragma unroll
   for (int q = 0; q < MB_RT; q++)
 #pragma unroll
-    for (int ct = 0; ct < 4; ct++)
+    for (int ct = 0; ct < MB_CT; ct++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 64 * g + 16 * ct + li;
+        const int row = 16 * (wv + MB_WAVES * q) + 4 * lk + r, col = 16 * MB_CT * g + 16 * ct + li;
         if (row < n && col < n) X[(long long)row * n + col] = (double)z[q][ct][r];
       }
 }
@@ -850,14 +870,19 @@ void launch_mid_reduce(const MidBlock* d_bl, const std::vector<MidBlock>& bl, co
 }
 void launch_mid_back(const MidBlock* d_bl, const std::vector<MidBlock>& bl, const float* V, const float* tau, float* VT,
                      double* X, hipStream_t s) {
+  int nmax = 1;
+  for (const auto& b : bl) nmax = std::max(nmax, b.n);
+  const bool narrow = nmax <= 384;  // what eight waves' row tiles hold: half the waves to a barrier (360 rows: 98 -> 93 us)
+  const int cols = 16 * MB_CT;
   int gp = 0, gc = 0;
   for (const auto& b : bl) {
     gp += (b.n + MD_NB - 2) / MD_NB;
-    gc += (b.n + 63) / 64;
+    gc += (b.n + cols - 1) / cols;
   }
   NRGK_LAUNCH(k_mid_larft, dim3(gp), dim3(256), 0, s, d_bl, (int)bl.size(), V, tau, VT);
   NRGK_HIP(hipGetLastError());
-  NRGK_LAUNCH(k_mid_back, dim3(gc), dim3(MB_THREADS), 0, s, d_bl, (int)bl.size(), V, (const float*)VT, X);
+  if (narrow) NRGK_LAUNCH((k_mid_back<8, 3>), dim3(gc), dim3(512), 0, s, d_bl, (int)bl.size(), V, (const float*)VT, X);
+  else NRGK_LAUNCH((k_mid_back<16, 3>), dim3(gc), dim3(1024), 0, s, d_bl, (int)bl.size(), V, (const float*)VT, X);
   NRGK_HIP(hipGetLastError());
 }
 void set_mid_lds_limit() {

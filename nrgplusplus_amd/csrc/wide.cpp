@@ -1,5 +1,5 @@
 // The wide sector blocks of an iteration (wider than the batched solver's crossover): their
-// eigenvalues from a blocked FP64 Householder tridiagonalisation and bisection, on a side stream of
+// eigenvalues from a blocked FP64 Householder tridiagonalisation and multisection, on a side stream of
 // the chain beside the batched solve of the other blocks; their eigenvectors by inverse iteration and
 // WY back-transformation, only for the columns that are read (k_tridiag.hip).
 //
