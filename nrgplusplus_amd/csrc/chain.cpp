@@ -563,9 +563,9 @@ void Chain::eigensolve_mixed() {
   }
   // Batches whose blocks all have up to SM_MAX rows: one launch for their whole solve, a workgroup each.
   // Measured at K = 64 (blocks of up to 25 rows, ~50 launches per step before): 0.80 -> 0.36 ms per step;
-  // 40 blocks of 2 .. 64 rows: 1.34 -> 0.79 ms.  Beside wider blocks, whose rounds take the narrow ones
+  // 40 blocks of 2 .. 64 rows: 1.34 -> 0.79 ms.  Beside wider blocks, whose launches take the narrow ones
   // along at no cost, that launch would come on top (0.33 ms at 64 rows: 60.7 -> 66.2 ms for 25 steps at
-  // K = 500).
+  // K = 500 when it was measured).
   int small_max = 0;
   for (int n : cur_n)
     if (n <= mixed_max) small_max = std::max(small_max, n);
