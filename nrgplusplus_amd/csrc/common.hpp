@@ -266,9 +266,11 @@ struct Ctx {
 // Page-locked staging for one stream's small transfers.  put() copies host data into pinned memory
 // and enqueues one asynchronous copy to its device twin, returning the device address; get()
 // enqueues a device-to-host copy into pinned memory and returns the host address, readable once the
-// stream is synchronised.  Regions are handed out front to back and stay valid until reset(), which
-// the owner calls after synchronising the stream.  Running out of room opens a further chunk (no
-// region moves while in use); reset() merges the chunks into one.
+// stream is synchronised.  Regions are handed out front to back.  The owner calls reset() after
+// synchronising the stream; the next take() then starts from the front again, in stream order behind
+// whatever was launched since, so until then every region may still be read, on the host and by
+// launches.  Running out of room opens a further chunk, kept like the others until the owner goes: a
+// chunk that left earlier would be another chain's (MemPool) while this one still reads it.
 struct Staging {
   struct Chunk {
     char* host = nullptr;
@@ -276,6 +278,7 @@ struct Staging {
     size_t cap = 0, used = 0;
   };
   std::vector<Chunk> chunks;
+  size_t cur = 0;  // the chunk that regions come from
   Ctx* ctx = nullptr;
   Staging() = default;
   Staging(const Staging&) = delete;
@@ -293,6 +296,7 @@ struct Staging {
       }
     }
     chunks.clear();
+    cur = 0;
   }
   void add_chunk(size_t bytes) {
     Chunk c;
@@ -326,9 +330,10 @@ struct Staging {
   // an aligned region of `bytes`: (host, device) addresses
   std::pair<char*, char*> take(size_t bytes) {
     const size_t need = (bytes + 255) & ~size_t(255);
-    if (chunks.empty() || chunks.back().used + need > chunks.back().cap)
+    while (cur < chunks.size() && chunks[cur].used + need > chunks[cur].cap) cur++;
+    if (cur == chunks.size())
       add_chunk(std::max<size_t>({need, chunks.empty() ? 0 : 2 * chunks.back().cap, size_t(1) << 20}));
-    Chunk& c = chunks.back();
+    Chunk& c = chunks[cur];
     const size_t o = c.used;
     c.used += need;
     return {c.host + o, c.dev + o};
@@ -402,13 +407,8 @@ struct Staging {
     return reinterpret_cast<const T*>(h);
   }
   void reset() {
-    if (chunks.size() > 1) {
-      size_t total = 0;
-      for (auto& c : chunks) total += c.cap;
-      release();
-      add_chunk(total);
-    }
-    if (!chunks.empty()) chunks.back().used = 0;
+    for (auto& c : chunks) c.used = 0;
+    cur = 0;
   }
 };
 

@@ -1,0 +1,88 @@
+// Host-side checks of the library's memory layer (csrc/common.hpp), compiled with the host compiler and
+// stand-ins for the HIP calls it makes: "device" memory is malloc'ed, so nothing here needs a GPU.
+// Usage: host_memory <check>; prints one line and exits with 0 if the check holds.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "../nrgplusplus_amd/csrc/common.hpp"
+
+static int failures = 0;
+#define CHECK(c)                                                \
+  do {                                                          \
+    if (!(c)) {                                                 \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #c);       \
+      failures++;                                               \
+    }                                                           \
+  } while (0)
+
+extern "C" {
+// (freed memory is overwritten and kept, so that a later read of it shows)
+static std::map<void*, size_t> live;
+hipError_t hipMalloc(void** p, size_t n) {
+  live[*p = std::malloc(n)] = n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  CHECK(!p || live.count(p));
+  if (p) std::memset(p, 0xA5, live[p]);
+  live.erase(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+const char* hipGetErrorString(hipError_t) { return "stand-in"; }
+}
+
+using namespace nrgk;
+
+// What get() read back stays readable after reset() until the staging's owner takes new regions, and a chunk
+// that a launch made after reset() may still read goes to nobody else before the owner's next synchronisation,
+// also where the interval needed several chunks and another owner's staging takes some at once.
+static void staging_readback() {
+  Ctx ctx;
+  ctx.set_capacity(size_t(1) << 30);
+  Staging a, b;
+  a.ctx = b.ctx = &ctx;
+  std::vector<double> dev(1000), big(200000, 1.0);
+  for (size_t i = 0; i < dev.size(); i++) dev[i] = (double)i;
+  for (int round = 0; round < 3; round++) {
+    double* first = a.put(big, nullptr);
+    a.put(big, nullptr);  // a second chunk, and a third
+    a.put(big, nullptr);
+    const double* r = a.get(dev.data(), dev.size(), nullptr);
+    if (round == 0) CHECK(a.chunks.size() > 1);
+    a.reset();
+    std::vector<double> other(200000, -1.0);
+    for (int k = 0; k < 3; k++) b.put(other, nullptr);  // (chunks of the same sizes)
+    b.get(other.data(), dev.size(), nullptr);
+    CHECK(std::memcmp(r, dev.data(), dev.size() * sizeof(double)) == 0);
+    CHECK(first[0] == 1.0 && first[199999] == 1.0);
+    b.reset();
+  }
+  // the regions are filled again from the front: an owner's memory settles
+  const size_t used = ctx.used;
+  for (int round = 0; round < 5; round++) {
+    for (int k = 0; k < 3; k++) a.put(big, nullptr);
+    a.reset();
+  }
+  CHECK(ctx.used == used);
+  b.release();
+  a.release();
+  CHECK(ctx.used == 0);
+}
+
+int main(int argc, char** argv) {
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "staging_readback") staging_readback();
+  else return 2;
+  std::printf("%s: %s\n", what.c_str(), failures ? "failed" : "ok");
+  return failures != 0;
+}
