@@ -160,7 +160,9 @@ int nrgk_chain_step(nrgk_chain* chain, const double* t_hopping, int n_hopping, d
  * Ascending eigenvalues go to w (sum dims[b]), the eigenvectors as the columns of each block to U
  * (packed like H).  Host arrays; mode NRGK_MODE_MIXED or NRGK_MODE_PLAIN64.  Allocates its
  * device buffers per call.  NRGK_ERR_NOCONV when a block does not converge (the small blocks' Jacobi, the
- * FP64 refinement within its step limit, or dsyevd); the reference only prints dsyevd's info. */
+ * FP64 refinement within its step limit, or dsyevd); the reference only prints dsyevd's info.  In
+ * NRGK_MODE_MIXED a block with a NaN or an infinity (or, wider than the crossover, with entries above 1e154, whose
+ * squares overflow) comes back as NaN, the others' results stand, and the status is NRGK_OK. */
 int nrgk_eigh_batched(nrgk_ctx* ctx, int n_blocks, const int* dims, const double* H, double* w, double* U,
                       int mode);
 /* Several independent chains (z-shifted discretisations, parameter points, requests) advanced by one

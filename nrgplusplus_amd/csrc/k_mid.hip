@@ -669,7 +669,8 @@ __global__ void __launch_bounds__(MD_THREADS) k_mid_reduce(const MidBlock* __res
   if (l == 0) s_max[wv] = mx;
   __syncthreads();
   for (int w = 0; w < MD_WAVES; w++) mx = s_max[w] > mx || s_max[w] != s_max[w] ? s_max[w] : mx;
-  // (a NaN or an infinity goes on into X and the refinement, which leaves such a block unconverged)
+  // (a NaN or an infinity goes on into X and through the refinement, whose maxima pass over NaN and so count
+  // the block as converged: it comes out as NaN, which a chain's truncation reports)
   const int ex = mx > 0.0 && mx <= 1.7976931348623157e308 ? ilogb(mx) + 1 : 0;
   MdReg& m = *reinterpret_cast<MdReg*>(lds);
   if (n <= MD_REG) {

@@ -655,8 +655,10 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
   __shared__ double rlo[4], rhi[4];
   __shared__ unsigned short grid[256];
   double lo = 1e300, hi = -1e300;
+  bool fin = true;
   for (int i = tid; i < n; i += 256) {
     const double di = w.d[i], rad = (i < n - 1 ? fabs(w.e[i]) : 0.0) + (i > 0 ? fabs(w.e[i - 1]) : 0.0);
+    fin = fin && fabs(di) + rad <= 1.7976931348623157e308;  // (fmin and fmax pass over NaN)
     lo = fmin(lo, di - rad);
     hi = fmax(hi, di + rad);
   }
@@ -669,13 +671,15 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
     rlo[wv] = lo;
     rhi[wv] = hi;
   }
-  __syncthreads();
+  fin = __syncthreads_and(fin);
   lo = fmin(fmin(rlo[0], rlo[1]), fmin(rlo[2], rlo[3]));
   hi = fmax(fmax(rhi[0], rhi[1]), fmax(rhi[2], rhi[3]));
   const double tn = fmax(fabs(lo), fabs(hi));
   const int j = g * ST_PER + tid / ST_LANES, ln = tid & (ST_LANES - 1);
-  if (!(tn > 0.0 && tn <= 1.7976931348623157e308)) {  // T = 0: every eigenvalue is exactly zero
-    if (j < n && ln == 0) lam[B.e_off + j] = 0.0;
+  // T = 0: every eigenvalue is exactly zero.  A NaN or an infinity in T (of the block, or of a wide block's
+  // entries above 1e154, whose squares overflow): every one is NaN, which a chain's truncation reports
+  if (!fin || tn == 0.0) {
+    if (j < n && ln == 0) lam[B.e_off + j] = fin ? 0.0 : __longlong_as_double(0x7ff8000000000000ll);
     return;
   }
   const int ex = ilogb(tn) + 1;  // ||T|| in [1/2, 1) after scaling
