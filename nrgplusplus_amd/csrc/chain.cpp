@@ -19,53 +19,6 @@ ThreadCounts& thread_counts() {
   return tc;
 }
 
-// ------------------------------------------------------------------ DevBuf
-void DevBuf::ensure(size_t bytes) {
-  if (bytes <= cap) return;
-  release();
-  const size_t want = bytes + bytes / 4 + 256;
-  size = retired ? MemPool::size_class(want) : want;
-  if (ctx) ctx->charge(want);
-  if (ctx && retired) p = ctx->pool.take(size);
-  if (!p) {
-    if (ctx && ctx->capacity && ctx->used + ctx->pool.held() > ctx->capacity) ctx->pool.trim();
-    hipError_t e = hipMalloc(&p, size);
-    if (e != hipSuccess && ctx) {
-      // the device waits, as hipFree made it, and everything idle is freed
-      if (retired && hipDeviceSynchronize() == hipSuccess) retired->give_all();
-      ctx->pool.trim();
-      size = want;
-      e = hipMalloc(&p, size);
-    }
-    if (e != hipSuccess) {
-      if (ctx) ctx->refund(want);
-      p = nullptr;
-      throw Error(NRGK_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(want) + "): " + hipGetErrorString(e));
-    }
-  }
-  cap = want;
-}
-void DevBuf::release() {
-  if (p) {
-    if (retired) retired->add(p, size);
-    else (void)hipFree(p);
-    if (ctx) ctx->refund(cap);
-  }
-  p = nullptr;
-  cap = 0;
-}
-void Retired::give_all() {
-  std::vector<std::pair<void*, size_t>> b;
-  {
-    std::lock_guard<std::mutex> lk(m);
-    b.swap(bufs);
-  }
-  for (auto& [p, size] : b) {
-    if (ctx) ctx->pool.give(p, size);
-    else (void)hipFree(p);
-  }
-}
-
 template <class T>
 static T* upload(DevBuf& buf, const std::vector<T>& v, hipStream_t s) {
   buf.ensure(std::max<size_t>(1, v.size()) * sizeof(T));

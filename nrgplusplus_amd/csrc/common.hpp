@@ -63,6 +63,13 @@ inline hipError_t stream_sync(hipStream_t s) {
 // ------------------------------------------------------------------ device buffers
 struct Ctx;
 
+// The result of an allocation whose failure the caller deals with.  The runtime keeps a failure until somebody
+// asks for it: left there, it would come out of the next launch's check, for a launch that went well.
+inline hipError_t handled(hipError_t e) {
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 // Idle device and page-locked memory of a context, for its next chains.  A chain's buffers come and go with
 // it (one request of the server, one eigh call, one of the chains of a z-average), and hipMalloc, hipFree and
 // hipHostMalloc each wait for the whole device: 16 chains at K = 512 spent 25 ms growing their buffers in the
@@ -319,9 +326,9 @@ struct Staging {
     chunks.push_back(c);
   }
   static hipError_t allocate(Chunk& c) {
-    hipError_t e = hipHostMalloc((void**)&c.host, c.cap, hipHostMallocDefault);
+    hipError_t e = handled(hipHostMalloc((void**)&c.host, c.cap, hipHostMallocDefault));
     if (e == hipSuccess) {
-      e = hipMalloc((void**)&c.dev, c.cap);
+      e = handled(hipMalloc((void**)&c.dev, c.cap));
       if (e != hipSuccess) (void)hipHostFree(c.host);
     }
     if (e != hipSuccess) c.host = c.dev = nullptr;

@@ -1,5 +1,5 @@
-// Host-side checks of the library's memory layer (csrc/common.hpp), compiled with the host compiler and
-// stand-ins for the HIP calls it makes: "device" memory is malloc'ed, so nothing here needs a GPU.
+// Host-side checks of the library's memory layer (csrc/common.hpp, csrc/memory.cpp), compiled with the host
+// compiler and stand-ins for the HIP calls it makes: "device" memory is malloc'ed, so nothing here needs a GPU.
 // Usage: host_memory <check>; prints one line and exits with 0 if the check holds.
 #include <cstdio>
 #include <cstdlib>
@@ -8,7 +8,7 @@
 #include <string>
 #include <vector>
 
-#include "../nrgplusplus_amd/csrc/common.hpp"
+#include "../nrgplusplus_amd/csrc/memory.cpp"
 
 static int failures = 0;
 #define CHECK(c)                                                \
@@ -22,10 +22,23 @@ static int failures = 0;
 extern "C" {
 // (freed memory is overwritten and kept, so that a later read of it shows)
 static std::map<void*, size_t> live;
+static int fail_next = 0;  // allocations to refuse
+static hipError_t last_error = hipSuccess;
 hipError_t hipMalloc(void** p, size_t n) {
+  if (fail_next > 0) {
+    fail_next--;
+    return last_error = hipErrorOutOfMemory;
+  }
   live[*p = std::malloc(n)] = n;
   return hipSuccess;
 }
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipFree(void* p) {
   CHECK(!p || live.count(p));
   if (p) std::memset(p, 0xA5, live[p]);
@@ -79,9 +92,52 @@ static void staging_readback() {
   CHECK(ctx.used == 0);
 }
 
+// An allocation that fails, is retried after idle memory was freed and succeeds leaves no error behind (the next
+// launch's check would report it), nor does one that fails for good with NRGK_ERR_NOMEM; the account stands.
+static void failed_allocation() {
+  Ctx ctx;
+  ctx.set_capacity(size_t(1) << 30);
+  Retired ret;
+  ret.ctx = &ctx;
+  {
+    DevBuf old(&ctx, &ret);
+    old.ensure(1 << 20);
+  }
+  ret.give_all();
+  CHECK(ctx.pool.held() > 0);
+  DevBuf b(&ctx, &ret);
+  fail_next = 1;
+  b.ensure(3 << 20);
+  CHECK(b.p && last_error == hipSuccess);
+  CHECK(ctx.pool.held() == 0);
+  Staging st;
+  st.ctx = &ctx;
+  fail_next = 1;
+  st.take(100);
+  CHECK(st.chunks.size() == 1 && last_error == hipSuccess);
+  const size_t used = ctx.used;
+  DevBuf c(&ctx, &ret);
+  for (int k = 0; k < 2; k++) {
+    fail_next = 4;
+    int status = 0;
+    try {
+      if (k == 0) c.ensure(1 << 20);
+      else st.take(4 << 20);
+    } catch (const Error& e) {
+      status = e.status;
+    }
+    CHECK(status == NRGK_ERR_NOMEM && last_error == hipSuccess);
+    CHECK(ctx.used == used && !c.p);
+  }
+  fail_next = 0;
+  c.ensure(1 << 20);
+  CHECK(c.p);
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "staging_readback") staging_readback();
+  else if (what == "failed_allocation") failed_allocation();
   else return 2;
   std::printf("%s: %s\n", what.c_str(), failures ? "failed" : "ok");
   return failures != 0;

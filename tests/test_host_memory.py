@@ -1,4 +1,4 @@
-"""The library's memory layer on the CPU: csrc/common.hpp compiled with the host compiler against
+"""The library's memory layer on the CPU: csrc/common.hpp and csrc/memory.cpp compiled with the host compiler against
 stand-ins for the HIP calls (tests/host_memory.cpp)."""
 import os
 import subprocess
@@ -16,7 +16,7 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["staging_readback"])
+@pytest.mark.parametrize("what", ["staging_readback", "failed_allocation"])
 def test_memory_layer(checks, what):
     r = subprocess.run([checks, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
