@@ -86,8 +86,7 @@ void Chain::init_device() {
   hold = std::make_shared<StreamHold>();
   NRGK_HIP(hipStreamCreateWithFlags(&hold->st, hipStreamNonBlocking));
   st = hold->st;
-  retired.ctx = ctx;
-  retired.st = st;
+  retired.attach(ctx, st);
   for (auto& e : ev) NRGK_HIP(hipEventCreate(&e));
 }
 

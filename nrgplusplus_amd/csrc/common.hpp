@@ -84,13 +84,10 @@ class MemPool {
   MemPool(const MemPool&) = delete;
   MemPool& operator=(const MemPool&) = delete;
   ~MemPool() { trim(); }
-  // Size of the allocation behind a request: eight classes to the octave, so that chains whose sectors differ
-  // a little fit each other's buffers; at most an eighth more than was asked for.
-  static size_t size_class(size_t bytes) {
-    size_t step = 4096;
-    while (step * 16 < bytes) step *= 2;
-    return (bytes + step - 1) / step * step;
-  }
+  // Allocations come in eight sizes to the octave (multiples of 256 bytes up to 4 KB), so that chains whose sectors
+  // differ a little fit each other's buffers: the one at or above `bytes`, and the one at or below.
+  static size_t size_above(size_t bytes) { return (bytes + step(bytes) - 1) / step(bytes) * step(bytes); }
+  static size_t size_below(size_t bytes) { return bytes / step(bytes) * step(bytes); }
   void* take(size_t size) {
     std::lock_guard<std::mutex> lk(m_);
     auto it = dev_.find(size);
@@ -101,25 +98,30 @@ class MemPool {
     return p;
   }
   void give(void* p, size_t size) {
-    std::vector<void*> out;  // freed outside of the lock
+    std::lock_guard<std::mutex> fl(free_m_);
+    std::vector<std::pair<void*, size_t>> out;
     {
       std::lock_guard<std::mutex> lk(m_);
-      while (size <= limit && held_ + size > limit && !dev_.empty()) {
+      size_t idle = held_;
+      while (size <= limit && idle + size > limit && !dev_.empty()) {
         auto old = dev_.begin();
         for (auto it = dev_.begin(); it != dev_.end(); ++it)
           if (it->second.since < old->second.since) old = it;
-        out.push_back(old->second.p);
-        held_ -= old->first;
+        out.emplace_back(old->second.p, old->first);
+        idle -= old->first;
         dev_.erase(old);
       }
-      if (held_ + size <= limit) {
+      if (idle + size <= limit) {
         dev_.emplace(size, Idle{p, clock_++});
         held_ += size;
-      } else {
-        out.push_back(p);
+        p = nullptr;
       }
     }
-    for (void* q : out) (void)hipFree(q);
+    for (auto& e : out) {
+      (void)hipFree(e.first);
+      held_ -= e.second;
+    }
+    if (p) (void)hipFree(p);
   }
   std::pair<char*, char*> take_staging(size_t size) {
     std::lock_guard<std::mutex> lk(m_);
@@ -146,48 +148,54 @@ class MemPool {
   }
   size_t held() const { return held_; }
   void trim() {
+    std::lock_guard<std::mutex> fl(free_m_);
     std::multimap<size_t, Idle> d;
     std::multimap<size_t, std::pair<char*, char*>> s;
     {
       std::lock_guard<std::mutex> lk(m_);
       d.swap(dev_);
       s.swap(staging_);
-      held_ = 0;
-      host_held_ = 0;
     }
-    for (auto& e : d) (void)hipFree(e.second.p);
+    for (auto& e : d) {
+      (void)hipFree(e.second.p);
+      held_ -= e.first;
+    }
     for (auto& e : s) {
       (void)hipHostFree(e.second.first);
       (void)hipFree(e.second.second);
+      held_ -= e.first;
+      host_held_ -= e.first;
     }
   }
 
  private:
+  static size_t step(size_t bytes) {
+    size_t s = 256;
+    while (s * 16 < bytes) s *= 2;
+    return s;
+  }
   struct Idle {
     void* p;
     unsigned long long since;
   };
   std::mutex m_;
+  std::mutex free_m_;  // taken before m_: who waits for it finds freed what was on its way out (held_ counts it till then)
   std::multimap<size_t, Idle> dev_;
   unsigned long long clock_ = 0;
   std::multimap<size_t, std::pair<char*, char*>> staging_;
   std::atomic<size_t> held_{0}, host_held_{0};
 };
 
-// Buffers that their owner has let go of while its stream may still use them: given to the context's pool
-// when the owner, having drained its streams, says so, or with the owner.
+// Buffers that their owner has let go of while its stream may still use them (nothing launched later does):
+// given to the context's pool when the owner, having drained its streams, says so, or with the owner, or when the
+// context needs the room (Ctx::drain).  Until then they count as used.
 struct Retired {
-  Ctx* ctx = nullptr;
-  hipStream_t st = nullptr;
-  std::mutex m;
-  std::vector<std::pair<void*, size_t>> bufs;
+  typedef std::vector<std::pair<void*, size_t>> List;
   Retired() = default;
   Retired(const Retired&) = delete;
   Retired& operator=(const Retired&) = delete;
-  ~Retired() {
-    if (!bufs.empty() && st) (void)hipStreamSynchronize(st);
-    give_all();
-  }
+  ~Retired();
+  void attach(Ctx* c, hipStream_t s);
   void add(void* p, size_t size) {
     std::lock_guard<std::mutex> lk(m);
     bufs.emplace_back(p, size);
@@ -196,7 +204,18 @@ struct Retired {
     std::lock_guard<std::mutex> lk(m);
     return bufs.empty();
   }
+  void take(List& out) {
+    std::lock_guard<std::mutex> lk(m);
+    out.insert(out.end(), bufs.begin(), bufs.end());
+    bufs.clear();
+  }
   void give_all();
+
+ private:
+  Ctx* ctx = nullptr;
+  hipStream_t st = nullptr;
+  std::mutex m;
+  List bufs;
 };
 
 // A device allocation that only grows; per-iteration scratch reuses it without hipMalloc in the
@@ -205,15 +224,14 @@ struct Retired {
 // allocated and freed directly.
 struct DevBuf {
   void* p = nullptr;
-  size_t cap = 0;
-  size_t size = 0;  // of the allocation (cap, rounded up to the pool's size class)
+  size_t cap = 0;  // bytes, as allocated and charged
   Ctx* ctx = nullptr;
   Retired* retired = nullptr;
   DevBuf() = default;
   explicit DevBuf(Ctx* c, Retired* r = nullptr) : ctx(c), retired(r) {}
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), cap(o.cap), size(o.size), ctx(o.ctx), retired(o.retired) {
+  DevBuf(DevBuf&& o) noexcept : p(o.p), cap(o.cap), ctx(o.ctx), retired(o.retired) {
     o.p = nullptr;
     o.cap = 0;
   }
@@ -222,7 +240,6 @@ struct DevBuf {
       release();
       p = o.p;
       cap = o.cap;
-      size = o.size;
       ctx = o.ctx;
       retired = o.retired;
       o.p = nullptr;
@@ -255,19 +272,38 @@ struct Ctx {
     capacity = bytes;
     pool.limit = bytes / 32;  // 8 GiB of a whole device
   }
+  // Admission: `used` counts every byte that chains hold on the device, retired buffers too, so that with the
+  // pool (emptied where both would exceed it, make_room) the capacity is never passed.
   void charge(size_t bytes) {
     size_t u = used.load();
-    do {
-      if (capacity && u + bytes > capacity)
+    for (bool drained = false;;) {
+      if (!capacity || u + bytes <= capacity) {
+        if (used.compare_exchange_weak(u, u + bytes)) return;
+      } else if (!drained) {
+        drain();
+        drained = true;
+        u = used.load();
+      } else {
         throw Error(NRGK_ERR_NOMEM, "nrgk: device capacity exceeded (" + std::to_string(u + bytes) + " > " +
                                         std::to_string(capacity) + " bytes)");
-    } while (!used.compare_exchange_weak(u, u + bytes));
+      }
+    }
   }
+  void make_room() {  // before an allocation that has been charged
+    if (capacity && used + pool.held() > capacity) pool.trim();
+  }
+  // every owner's retired buffers to the pool, once the device has drained
+  void drain();
   void refund(size_t bytes) {
     size_t u = used.load();
     while (!used.compare_exchange_weak(u, bytes < u ? u - bytes : 0)) {
     }
   }
+
+ private:
+  friend struct Retired;
+  std::mutex lists_m;
+  std::vector<Retired*> lists;
 };
 
 // Page-locked staging for one stream's small transfers.  put() copies host data into pinned memory
@@ -307,13 +343,14 @@ struct Staging {
   }
   void add_chunk(size_t bytes) {
     Chunk c;
-    c.cap = MemPool::size_class(bytes);
+    c.cap = MemPool::size_above(bytes);
     if (ctx) ctx->charge(c.cap);
     if (ctx) std::tie(c.host, c.dev) = ctx->pool.take_staging(c.cap);
     if (!c.host) {
-      if (ctx && ctx->capacity && ctx->used + ctx->pool.held() > ctx->capacity) ctx->pool.trim();
+      if (ctx) ctx->make_room();
       hipError_t e = allocate(c);
       if (e != hipSuccess && ctx) {
+        ctx->drain();
         ctx->pool.trim();
         e = allocate(c);
       }

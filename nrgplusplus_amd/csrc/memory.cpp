@@ -5,49 +5,77 @@
 
 namespace nrgk {
 
+// A quarter of headroom; from a pool, as much of it as its size at or below that leaves (9 to 25 %).
 void DevBuf::ensure(size_t bytes) {
   if (bytes <= cap) return;
   release();
-  const size_t want = bytes + bytes / 4 + 256;
-  size = retired ? MemPool::size_class(want) : want;
-  if (ctx) ctx->charge(want);
+  const size_t want = bytes + bytes / 4 + 256, size = retired ? MemPool::size_below(want) : want;
+  if (ctx) ctx->charge(size);
   if (ctx && retired) p = ctx->pool.take(size);
   if (!p) {
-    if (ctx && ctx->capacity && ctx->used + ctx->pool.held() > ctx->capacity) ctx->pool.trim();
+    if (ctx) ctx->make_room();
     hipError_t e = handled(hipMalloc(&p, size));
-    if (e != hipSuccess && ctx) {
-      // the device waits, as hipFree made it, and everything idle is freed
-      if (retired && hipDeviceSynchronize() == hipSuccess) retired->give_all();
+    if (e != hipSuccess && ctx) {  // everything idle is freed
+      ctx->drain();
       ctx->pool.trim();
-      size = want;
       e = handled(hipMalloc(&p, size));
     }
     if (e != hipSuccess) {
-      if (ctx) ctx->refund(want);
+      if (ctx) ctx->refund(size);
       p = nullptr;
-      throw Error(NRGK_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(want) + "): " + hipGetErrorString(e));
+      throw Error(NRGK_ERR_NOMEM, std::string("hipMalloc(") + std::to_string(size) + "): " + hipGetErrorString(e));
     }
   }
-  cap = want;
+  cap = size;
 }
 void DevBuf::release() {
   if (p) {
-    if (retired) retired->add(p, size);
-    else (void)hipFree(p);
-    if (ctx) ctx->refund(cap);
+    if (retired) {
+      retired->add(p, cap);
+    } else {
+      (void)hipFree(p);
+      if (ctx) ctx->refund(cap);
+    }
   }
   p = nullptr;
   cap = 0;
 }
-void Retired::give_all() {
-  std::vector<std::pair<void*, size_t>> b;
+
+void Retired::attach(Ctx* c, hipStream_t s) {
+  ctx = c;
+  st = s;
+  std::lock_guard<std::mutex> lk(c->lists_m);
+  c->lists.push_back(this);
+}
+Retired::~Retired() {
+  if (!ctx) return;
   {
-    std::lock_guard<std::mutex> lk(m);
-    b.swap(bufs);
+    std::lock_guard<std::mutex> lk(ctx->lists_m);
+    ctx->lists.erase(std::find(ctx->lists.begin(), ctx->lists.end(), this));
   }
+  if (!bufs.empty() && st) (void)hipStreamSynchronize(st);
+  give_all();
+}
+void Retired::give_all() {
+  List b;
+  take(b);
   for (auto& [p, size] : b) {
-    if (ctx) ctx->pool.give(p, size);
+    ctx->pool.give(p, size);
+    ctx->refund(size);
+  }
+}
+void Ctx::drain() {
+  Retired::List b;
+  {
+    std::lock_guard<std::mutex> lk(lists_m);
+    for (Retired* r : lists) r->take(b);
+  }
+  if (b.empty()) return;
+  const bool idle = hipDeviceSynchronize() == hipSuccess;
+  for (auto& [p, size] : b) {
+    if (idle) pool.give(p, size);
     else (void)hipFree(p);
+    refund(size);
   }
 }
 

@@ -20,8 +20,7 @@ namespace nrgk {
 
 Obs::Obs(Chain* c, int n_ops, const int* nblocks, const int* bi, const int* bj, const double* data) : ch(c), nops(n_ops) {
   hold = ch->hold;
-  retired.ctx = ch->ctx;
-  retired.st = ch->st;
+  retired.attach(ch->ctx, ch->st);
   for (DevBuf* b : {&buf[0], &buf[1], &dseg, &dC, &dY}) b->ctx = ch->ctx, b->retired = &retired;
   NRGK_REQUIRE(ch->phase == Chain::FRESH, NRGK_ERR_STATE, "nrgk: observables are created before the first site");
   ch->need_full_u = true;  // the rotation reads every column of U
@@ -135,8 +134,7 @@ Fdm::Fdm(Chain* c, Obs* o, int nb, double emin, double emax) : ch(c), obs(o), nb
   NRGK_REQUIRE(nb > 0 && emin > 0 && emax > emin, NRGK_ERR_INVALID, "nrgk: bad FDM binning");
   delE = (nbins - 1.0) / std::log(e_max / e_min);  // fdmSpectrum.hpp:351-354
   hold = ch->hold;
-  retired.ctx = ch->ctx;
-  retired.st = ch->st;
+  retired.attach(ch->ctx, ch->st);
   for (DevBuf* b : {&dpos, &dneg, &dsum, &dbf, &dred[0], &dred[1], &dRA, &dAR, &dT1, &drho, &ditems, &dpt, &dE, &dth, &dQ})
     b->ctx = ch->ctx, b->retired = &retired;
 }
@@ -202,6 +200,7 @@ void Fdm::record() {
     sh->q_ops = sysop->nops;
   }
   c.sync();
+  retired.give_all();
   sh->E.assign(h_e, h_e + c.N_tot);
   if (h_q) sh->Q.assign(h_q, h_q + (size_t)sh->q_ops * c.N_tot);
   shells.push_back(std::move(sh));

@@ -5,7 +5,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <mutex>
+#include <random>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../nrgplusplus_amd/csrc/memory.cpp"
@@ -22,6 +26,8 @@ static int failures = 0;
 extern "C" {
 // (freed memory is overwritten and kept, so that a later read of it shows)
 static std::map<void*, size_t> live;
+static size_t live_bytes = 0, live_peak = 0;  // of device memory
+static std::mutex hip_m;
 static int fail_next = 0;  // allocations to refuse
 static hipError_t last_error = hipSuccess;
 hipError_t hipMalloc(void** p, size_t n) {
@@ -29,7 +35,10 @@ hipError_t hipMalloc(void** p, size_t n) {
     fail_next--;
     return last_error = hipErrorOutOfMemory;
   }
+  std::lock_guard<std::mutex> lk(hip_m);
   live[*p = std::malloc(n)] = n;
+  live_bytes += n;
+  live_peak = std::max(live_peak, live_bytes);
   return hipSuccess;
 }
 hipError_t hipGetLastError() {
@@ -40,13 +49,22 @@ hipError_t hipGetLastError() {
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipFree(void* p) {
+  std::lock_guard<std::mutex> lk(hip_m);
   CHECK(!p || live.count(p));
-  if (p) std::memset(p, 0xA5, live[p]);
+  if (!p) return hipSuccess;
+  std::memset(p, 0xA5, live[p]);
+  live_bytes -= live[p];
   live.erase(p);
   return hipSuccess;
 }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { return hipFree(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) {
+  std::free(p);
+  return hipSuccess;
+}
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
   std::memcpy(d, s, n);
   return hipSuccess;
@@ -98,7 +116,7 @@ static void failed_allocation() {
   Ctx ctx;
   ctx.set_capacity(size_t(1) << 30);
   Retired ret;
-  ret.ctx = &ctx;
+  ret.attach(&ctx, nullptr);
   {
     DevBuf old(&ctx, &ret);
     old.ensure(1 << 20);
@@ -134,10 +152,81 @@ static void failed_allocation() {
   CHECK(c.p);
 }
 
+// Owners that grow, drop and replace buffers: what lies on the device never passes the capacity, whether used,
+// retired or idle, what fits beside the buffers in use is not refused, and the account is what the buffers hold.
+static void capacity_bounds(unsigned seed, Ctx& ctx, bool alone) {
+  std::mt19937 rng(seed);
+  auto owner = [&] {
+    auto r = std::make_unique<Retired>();
+    r->attach(&ctx, nullptr);
+    return r;
+  };
+  struct Own {
+    std::unique_ptr<Retired> r;
+    std::vector<DevBuf> b;
+  };
+  std::vector<Own> own(3);
+  size_t refused = 0;
+  for (auto& o : own) o.r = owner();
+  auto held = [&] {
+    size_t n = 0;
+    for (auto& o : own)
+      for (auto& b : o.b) n += b.cap;
+    return n;
+  };
+  for (int k = 0; k < 4000; k++) {
+    Own& o = own[rng() % own.size()];
+    const int what = rng() % 40;
+    if (what == 0) {
+      o.b.clear();
+    } else if (what == 1) {
+      o.r->give_all();  // (a synchronisation)
+    } else if (what == 2) {
+      o.b.clear();
+      o.r = owner();
+    } else {
+      if (o.b.size() < 6) o.b.emplace_back(&ctx, o.r.get());
+      DevBuf& b = o.b[rng() % o.b.size()];
+      const size_t bytes = size_t(1) << (8 + rng() % 15), n = bytes + rng() % bytes;
+      const size_t others = held() - (n > b.cap ? b.cap : 0), old = b.cap;
+      try {
+        b.ensure(n);
+        CHECK(b.cap >= n && b.cap <= std::max(old, n + n / 4 + 256));
+        static_cast<char*>(b.p)[0] = static_cast<char*>(b.p)[n - 1] = 1;
+      } catch (const Error& e) {
+        refused++;
+        CHECK(e.status == NRGK_ERR_NOMEM && !b.p);
+        if (alone) CHECK(others + MemPool::size_below(n + n / 4 + 256) > ctx.capacity);
+      }
+    }
+  }
+  if (alone) {
+    for (auto& o : own) o.r->give_all();
+    CHECK(ctx.used == held());
+    CHECK(refused > 0);
+  }
+}
+static void capacity() {
+  Ctx ctx;
+  ctx.set_capacity(size_t(20) << 20);
+  for (unsigned s = 0; s < 5; s++) {
+    live_peak = 0;
+    capacity_bounds(s, ctx, true);
+    CHECK(live_peak <= ctx.capacity && live_peak > ctx.capacity / 2);
+    CHECK(ctx.used == 0 && live_bytes == ctx.pool.held());
+  }
+  std::vector<std::thread> ts;
+  for (unsigned s = 0; s < 4; s++) ts.emplace_back([&, s] { capacity_bounds(100 + s, ctx, false); });
+  for (auto& t : ts) t.join();
+  CHECK(live_peak <= ctx.capacity);
+  CHECK(ctx.used == 0 && live_bytes == ctx.pool.held());
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   if (what == "staging_readback") staging_readback();
   else if (what == "failed_allocation") failed_allocation();
+  else if (what == "capacity") capacity();
   else return 2;
   std::printf("%s: %s\n", what.c_str(), failures ? "failed" : "ok");
   return failures != 0;

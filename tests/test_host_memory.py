@@ -16,7 +16,7 @@ def checks(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["staging_readback", "failed_allocation"])
+@pytest.mark.parametrize("what", ["staging_readback", "failed_allocation", "capacity"])
 def test_memory_layer(checks, what):
     r = subprocess.run([checks, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
