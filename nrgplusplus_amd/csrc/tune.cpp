@@ -4,7 +4,8 @@
 // the device -- the batched path forming every eigenvector (the refinement needs them), the Householder
 // path the eigenvalues and the first n/4 eigenvectors (the kept columns an RG step reads) -- and the
 // crossover is the widest candidate at which the batched path is not slower.  The result is cached in a
-// text file per GPU model and CU count, which every context reads when it is created.
+// text file per GPU model and CU count, which every context reads when it is created; the file names the
+// solver it was measured with (TUNE_SOLVER), and one measured with another is not used.
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -18,26 +19,31 @@
 
 namespace nrgk {
 
+// Counts up with every change to either path that can move the crossover (files before 2 name none: their
+// crossover was measured against block Jacobi rounds that the batched path no longer takes).
+constexpr int TUNE_SOLVER = 2;
+
 std::string tune_cache_path(const Ctx& c) {
   if (const char* p = std::getenv("NRGK_TUNE_CACHE")) return p;
   const char* home = std::getenv("HOME");
   return std::string(home ? home : "/tmp") + "/.cache/nrgk/tune-" + c.arch + "-" + std::to_string(c.n_cu) + "cu.txt";
 }
 
-// "crossover <n>" from the cache file, if it exists and was written for this GPU
+// "crossover <n>" from the cache file, if it exists and was written for this GPU and this solver
 void tune_load(Ctx& c) {
   std::ifstream f(tune_cache_path(c));
   if (!f) return;
   std::string line, key;
   std::string arch;
-  int cu = -1, cross = -1;
+  int cu = -1, cross = -1, solver = -1;
   while (std::getline(f, line)) {
     std::istringstream is(line);
     is >> key;
     if (key == "gpu") is >> arch >> cu;
+    else if (key == "solver") is >> solver;
     else if (key == "crossover") is >> cross;
   }
-  if (arch == c.arch && cu == c.n_cu && cross >= 32 && cross <= 768) {
+  if (arch == c.arch && cu == c.n_cu && solver == TUNE_SOLVER && cross >= 32 && cross <= 768) {
     c.mixed_max = cross;
     c.tuned = true;
   }
@@ -107,6 +113,7 @@ int tune_crossover(Ctx* ctx, const std::string& path, std::vector<std::vector<do
     std::ofstream f(path);
     if (f) {
       f << "gpu " << ctx->arch << " " << ctx->n_cu << "\n";
+      f << "solver " << TUNE_SOLVER << "\n";
       f << "crossover " << cross << "\n";
       for (auto& r : table)
         f << "# n " << (int)r[0] << " blocks " << (int)r[1] << " batched_ms " << r[2] << " householder_ms " << r[3] << "\n";
