@@ -219,7 +219,7 @@ int nrgk_chain_fdag_blocks(nrgk_chain* chain, int op, int* n_blocks, int* bi, in
  * dims = kept counts. */
 int nrgk_chain_set_state(nrgk_chain* chain, const nrgk_site_desc* state, int cnt);
 /* per-step device timings (ms): assemble, eigensolve, truncate, rotate; and eigensolver stats (the most sweeps of
- * a small block's Jacobi, the widest cluster) */
+ * a small block's Jacobi, 0 in a step without it; the widest cluster) */
 int nrgk_chain_step_stats(nrgk_chain* chain, double* ms4, int* jacobi_sweeps, int* max_cluster);
 /* the last truncation: E_cut = sorted[K] (discard_higher_energies, nrgcore.hpp:285) and the number of
  * eigenvalues within 2e-10 of E_cut + 1e-8 (either side), whose keep/discard decision an eigenvalue

@@ -487,6 +487,7 @@ static double knob(const char* name, double dflt) {
 // K2 + K6: start vectors by an FP32 Householder solve, then Ogita-Aishima refinement in FP64.
 void Chain::eigensolve_mixed() {
   const int S = (int)cur_qn.size();
+  sweeps = 0;
   // blocks wider than the crossover (the context's, tuned or 768; NRGK_MIXED_MAX overrides it) go to
   // the wide-block path on the side stream
   const int mixed_max = mixed_max_override >= 0 ? mixed_max_override : (int)knob("NRGK_MIXED_MAX", ctx->mixed_max);
@@ -579,7 +580,7 @@ void Chain::eigensolve_mixed() {
     large_blocks_join(*this);
     wide_join();
     sync();
-    sweeps = maxcluster = unresolved = oa_steps = 0;
+    maxcluster = unresolved = oa_steps = 0;
     small_done();
     large_blocks_check(*this);
     if (need_full_u || fail_on_unconverged) {
