@@ -128,7 +128,8 @@ int nrgk_ctx_used_bytes(nrgk_ctx* ctx, size_t* used, size_t* capacity);
  * the batched path is not slower.  The result and the measured times go to a cache file (cache_path, or
  * NULL: $NRGK_TUNE_CACHE, else $HOME/.cache/nrgk/tune-<arch>-<CUs>cu.txt) that every context created
  * later on the same GPU model reads (a file measured with another version of the solver is ignored).  table[n_rows][4]: width, blocks, batched ms, wide-path ms (may
- * be NULL).  NRGK_MIXED_MAX, when set, overrides the crossover per call. */
+ * be NULL).  NRGK_MIXED_MAX, when set, overrides the crossover per call (values above 768
+ * count as 768, the widest block that the batched path takes). */
 int nrgk_tune(nrgk_ctx* ctx, const char* cache_path, int* crossover, double* table, int cap_rows, int* n_rows);
 /* the context's crossover and whether it came from the autotuner (its cache or nrgk_tune) */
 int nrgk_ctx_crossover(nrgk_ctx* ctx, int* crossover, int* tuned);

@@ -488,9 +488,11 @@ static double knob(const char* name, double dflt) {
 void Chain::eigensolve_mixed() {
   const int S = (int)cur_qn.size();
   sweeps = 0;
-  // blocks wider than the crossover (the context's, tuned or 768; NRGK_MIXED_MAX overrides it) go to
-  // the wide-block path on the side stream
-  const int mixed_max = mixed_max_override >= 0 ? mixed_max_override : (int)knob("NRGK_MIXED_MAX", ctx->mixed_max);
+  // blocks wider than the crossover (the context's, tuned or 768; NRGK_MIXED_MAX overrides it, up to what the
+  // batched solver takes) go to the wide-block path on the side stream
+  const int mixed_max = mixed_max_override >= 0
+                            ? mixed_max_override
+                            : (int)std::min(knob("NRGK_MIXED_MAX", ctx->mixed_max), (double)MD_MAX);
   std::vector<int> big;
   for (int s = 0; s < S; s++)
     if (cur_n[s] > mixed_max) big.push_back(s);
