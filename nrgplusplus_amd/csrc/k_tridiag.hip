@@ -797,7 +797,12 @@ __device__ __forceinline__ void ht_bwd_load(const double* __restrict__ U, int n,
 // elimination of the iterate share one pass (the L factor is not kept), the upper factor's three
 // diagonals go to the scratch f0 (as the pivot's reciprocal), f1, f2 at entry i * mp + slot, then one
 // backward pass.  A pivot smaller than piv0 in magnitude is moved out to +-piv0 (dlagtf/dlagts'
-// perturbation), which bounds the growth of one step by about 1 / piv0.
+// perturbation), which bounds the growth of one step by about 1 / piv0, before it
+// is compared with the entry below it: where the shift equals entries of T's diagonal (weakly coupled levels, whose
+// eigenvalues the multisection finds to the last bit), a zero pivot that went through an exchange made the step
+// tell the copies of an eigenvalue apart far below eps ||T||, one copy took over every iterate of the cluster, and
+// orthogonalising them left rounding, amplified (defects of 1e-6 to 1 for chains of levels 0 and 1 coupled by 1e-14
+// to 1e-4; at most 2e-12 so).
 // Each pass requests the next HT_RT rows before it stores the current ones: a wait on vector memory
 // also waits for every store issued before the awaited load, so the loads are not held behind them.
 // 1 / x to an ulp or so: the pivots' reciprocals stand in the elimination's dependent chain, where the IEEE
@@ -812,9 +817,9 @@ __device__ __forceinline__ double ht_rcp(double x) {
 // branches: lanes that exchange rows i and i + 1 stand beside lanes that do not.
 __device__ __forceinline__ void ht_fwd_row(double sub, double nd, double nu, double x, double piv0, double* f0, double* f1,
                                            double* f2, double* ur, int p, int slot, double& cd, double& cu, double& xi) {
-  const bool sw = fabs(cd) < fabs(sub);
   const double pc = fabs(cd) < piv0 ? (cd < 0.0 ? -piv0 : piv0) : cd;
-  const double r = ht_rcp(sw ? sub : pc), ml = (sw ? cd : sub) * r;
+  const bool sw = fabs(pc) < fabs(sub);
+  const double r = ht_rcp(sw ? sub : pc), ml = (sw ? pc : sub) * r;
   f0[slot] = r;
   f1[slot] = sw ? nd : cu;
   f2[slot] = sw ? nu : 0.0;
