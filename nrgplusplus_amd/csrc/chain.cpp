@@ -496,10 +496,10 @@ void Chain::eigensolve_mixed() {
   std::vector<int> big;
   for (int s = 0; s < S; s++)
     if (cur_n[s] > mixed_max) big.push_back(s);
-  const size_t bytes64_all = std::max<long long>(1, tot_elems) * sizeof(double);
-  dX.ensure(bytes64_all);  // every buffer the side stream touches is sized before it starts
-  dX2.ensure(bytes64_all);
-  dU.ensure(bytes64_all);
+  const size_t bytes64 = std::max<long long>(1, tot_elems) * sizeof(double);
+  dX.ensure(bytes64);  // every buffer the side stream touches is sized before it starts
+  dX2.ensure(bytes64);
+  dU.ensure(bytes64);
   dlam_raw.ensure(std::max<long long>(1, N_tot) * sizeof(double));
   // the wide blocks: the FP64 Householder path (default) or, with NRGK_WIDE_SOLVER=rocsolver,
   // rocSOLVER dsyevd per block on the side streams
@@ -539,13 +539,12 @@ void Chain::eigensolve_mixed() {
     small_sec.push_back(s);
     nmax_s = std::max(nmax_s, n);
   }
-  int* d_small = nullptr;  // status per block, then the largest sweep count
-  const int* h_small = nullptr;
-  std::vector<int> redo;  // sectors whose block the batched solve left unconverged
+  const int* h_small = nullptr;  // status per block, then the largest sweep count
+  std::vector<int> redo;         // sectors whose block the batched solve left unconverged
   if (!small.empty()) {
     Staging::Region rg = stg.open(Staging::span<EigBlock>(small.size()) + Staging::span<int>(small.size() + 1));
     const EigBlock* db = stg.place(rg, small);
-    d_small = stg.place_zero<int>(rg, small.size() + 1);
+    int* d_small = stg.place_zero<int>(rg, small.size() + 1);
     stg.commit(rg, st);
     prof_begin("eig_small");
     launch_eig_small(db, (int)small.size(), nmax_s, dH.as<double>(), dU.as<double>(), dlam_raw.as<double>(), d_small,
@@ -553,12 +552,6 @@ void Chain::eigensolve_mixed() {
     prof_end("eig_small", 1, 0.0, 0.0);
     h_small = stg.get(d_small, small.size() + 1, st);
   }
-  auto small_done = [&] {  // after a synchronisation
-    if (small.empty()) return;
-    for (size_t i = 0; i < small.size(); i++)
-      if (h_small[i]) redo.push_back(small_sec[i]);
-    sweeps = h_small[small.size()];
-  };
   // A block the batched solve left short of its stopping point is solved again in FP64 by the direct
   // solver (the next Hamiltonian is built from these vectors, so they must meet the same bar as every
   // other block's); nrgk_chain_refine_stats reports how many were.  The stand-alone nrgk_eigh_batched
@@ -578,12 +571,16 @@ void Chain::eigensolve_mixed() {
     blks.push_back(b);
   }
   const int nb = (int)blks.size();
-  if (nb == 0) {  // every block went to the side streams: no batched launch (empty grids)
+  if (nb == 0) {  // every block is small or wide: no batched launch (empty grids)
     large_blocks_join(*this);
     wide_join();
     sync();
     maxcluster = unresolved = oa_steps = 0;
-    small_done();
+    if (!small.empty()) {
+      for (size_t i = 0; i < small.size(); i++)
+        if (h_small[i]) redo.push_back(small_sec[i]);
+      sweeps = h_small[small.size()];
+    }
     large_blocks_check(*this);
     if (need_full_u || fail_on_unconverged) {
       wide_vectors(true);
@@ -596,7 +593,6 @@ void Chain::eigensolve_mixed() {
   for (auto& b : blks) nmax_m = std::max(nmax_m, b.n);
   // ---- FP32 stage (k_mid.hip): every block's start vectors in a dozen launches, widest blocks first
   // (each is one workgroup's work in the reduction)
-  const size_t bytes64 = std::max<long long>(1, tot_elems) * sizeof(double);
   std::vector<int> order(nb);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blks[x].n > blks[y].n; });
@@ -622,9 +618,6 @@ void Chain::eigensolve_mixed() {
     so += 3LL * e.n * t.mpad;
     no += e.n;
   }
-  dX.ensure(bytes64);
-  dX2.ensure(bytes64);
-  dU.ensure(bytes64);
   // five n x n arenas for the refinement: P = H X, S, R, E and the Rayleigh-Ritz scratch Q; before it, the
   // same memory holds the Householder vectors, V T, and the inverse iteration's factors
   const long long na = std::max<long long>(1, tot_elems);
@@ -633,7 +626,6 @@ void Chain::eigensolve_mixed() {
   double *dS = dP + na, *dR = dS + na, *dE = dR + na, *dQ = dE + na;
   d_rrv.ensure(std::max<long long>(1, N_tot) * 3 * sizeof(double));
   dlam_tmp.ensure(std::max<long long>(1, N_tot) * sizeof(double));
-  dlam_raw.ensure(std::max<long long>(1, N_tot) * sizeof(double));
   d_cid.ensure(std::max<long long>(1, N_tot) * sizeof(int));
   d_sidx.ensure(std::max<long long>(1, N_tot) * sizeof(int));
   d_mid_A.ensure((size_t)po * sizeof(float));
@@ -699,7 +691,6 @@ void Chain::eigensolve_mixed() {
   const int dbg_oa = (int)knob("NRGK_DEBUG_OA", 0);
   std::vector<EigBlock> act = blks;
   oa_steps = 0;
-  bool asked = false;
   for (int it = 0; it < oa_max && !act.empty(); it++) {
     const int na = (int)act.size();
     // 32 x 32 tiles of the active blocks: all of them, and the (i <= j) half for the symmetrisation
@@ -770,8 +761,6 @@ void Chain::eigensolve_mixed() {
     check("X+XE", dX.as<double>(), false);
     oa_steps = it + 1;
     if (!ask) continue;
-    if (!asked) small_done();
-    asked = true;
     const std::vector<double> conv(h_conv, h_conv + 4 * na);
     std::vector<EigBlock> next;
     for (int a = 0; a < na; a++) {
