@@ -516,11 +516,12 @@ void Chain::eigensolve_mixed() {
     large_blocks_begin(*this, {});
     wide_begin(big);
   }
-  // Batches whose blocks all have up to SM_MAX rows: one launch for their whole solve, a workgroup each.
-  // Measured at K = 64 (blocks of up to 25 rows, ~50 launches per step before): 0.80 -> 0.36 ms per step;
-  // 40 blocks of 2 .. 64 rows: 1.34 -> 0.79 ms.  Beside wider blocks, whose launches take the narrow ones
-  // along at no cost, that launch would come on top (0.33 ms at 64 rows: 60.7 -> 66.2 ms for 25 steps at
-  // K = 500 when it was measured).
+  // Batches whose blocks (but for the wide ones) all have up to SM_MAX rows: one launch for their whole solve, a
+  // workgroup each.  Measured at K = 64 (blocks of up to 25 rows, ~50 launches per step before): 0.80 -> 0.36 ms per
+  // step; 40 blocks of 2 .. 64 rows: 1.34 -> 0.79 ms.  Beside wider batched blocks, whose launches take the narrow
+  // ones along at no cost, that launch comes on top (0.33 ms at 64 rows): with the small blocks sent to it there too,
+  // 25 steps at K = 500 take 31.9 ms against 25.6, 21 at K = 1024 41.2 against 37.3, sixteen chains at K = 512 104
+  // against 89.
   int small_max = 0;
   for (int n : cur_n)
     if (n <= mixed_max) small_max = std::max(small_max, n);

@@ -638,8 +638,9 @@ __global__ void __launch_bounds__(256) k_ht_syr2k(const HtBlock* __restrict__ bl
 // p_i / p_{i-1} of the usual form take a reciprocal and three more.  T is scaled to about unit norm, so
 // the polynomials stay in range over eight steps, after which they are rescaled by a power of two.
 // A pass costs a wavefront about nine operations a row whatever LANES is, so more lanes pay while the
-// wavefronts still find free SIMDs: sixteen for 4 100 eigenvalues in blocks of up to 360 rows take 85 us where
-// eight take 117 and one takes 600; where the eigenvalues alone fill the chip, one lane each does the least work.
+// wavefronts still find free SIMDs: sixteen for 4 100 eigenvalues in blocks of up to 330 rows take 91 us where
+// eight take 104 and one takes 300; where the eigenvalues alone fill the chip, one lane each does the least work
+// (54 800 in blocks of 769 to 4 230 rows: 5.9 ms against 7.1 and 10.6).
 constexpr int ST_UNROLL = 8;
 template <int ST_LANES>
 __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl, int nblk, const double* __restrict__ Wa,
@@ -747,7 +748,9 @@ __global__ void __launch_bounds__(256) k_ht_sturm(const HtBlock* __restrict__ bl
   if (mine && ln == 0) lam[B.e_off + j] = ldexp(0.5 * (a + c), ex);
 }
 
-// deterministic start vector entries in [-1, 1), none of them zero (a block of one row has but one)
+// deterministic start vector entries in [-1, 1), none of them zero (a block of one row has but one): the published
+// 32-bit integer hash lowbias32 (C. Wellons, hash-prospector, public domain), whose shifts and multipliers are found
+// by search, of the entry's indices
 __device__ __forceinline__ double ht_start(unsigned p, unsigned i) {
   unsigned x = (p << 16 ^ i) + 0x9E3779B9u;  // (both below 2^16)
   x ^= x >> 16;
@@ -1443,7 +1446,13 @@ void launch_ht_sturm(const HtBlock* d_bl, const std::vector<HtBlock>& bl, const 
     for (const auto& b : bl) g += (b.n + 256 / lanes - 1) / (256 / lanes);
     return g;
   };
-  // (1 024 SIMDs; a wavefront holds 64 / lanes eigenvalues)
+  // A wavefront holds 64 / lanes eigenvalues, and the chip has 1 024 SIMDs.  Sixteen against eight lanes: blocks of
+  // one width cross at one wave a SIMD, 4 096 eigenvalues (360 rows: 113 against 119 us at 3 960, 168 against 122 at
+  // 5 040), a chain's sectors, whose narrow blocks end early, between 6 000 and 8 000 (122 against 148 us, 189 against
+  // 182); the line at 5 120 lies between the two.  Eight against one: one width crosses at about 24 000 (360 rows:
+  // 284 against 359 us at 15 800, 373 against 366 at 24 000), a chain's wide sectors between 28 600 and 54 800 (2.8
+  // against 3.9 ms, 7.1 against 5.9); the line at two waves a SIMD, 16 384, lies below both, so that between them one
+  // lane is taken where eight would be faster.
   if (total * 16 <= 80 * 1024)
     NRGK_LAUNCH(k_ht_sturm<16>, dim3(grid(16)), dim3(256), lds, s, d_bl, (int)bl.size(), W, lam, rtol);
   else if (total * 8 <= 2 * 64 * 1024)
